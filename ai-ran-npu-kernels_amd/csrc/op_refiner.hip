@@ -16,8 +16,9 @@
 // its taps along the subcarrier axis (taps at subcarrier offsets -dil, 0,
 // +dil; symbol offsets stay -1, 0, +1), which widens the network's view of
 // the band: dilations 1, 2, 4, 8, 16, 1 see 65 subcarriers.  Weight
-// gradients are fp32 VALU outer products over LDS
-// tiles, reduced across workgroups in a fixed order.
+// gradients contract over the pixels on the same MFMA, both operands through
+// transposing LDS reads; the workgroups' partial sums are added in a fixed
+// order.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -654,81 +655,257 @@ __global__ void __launch_bounds__(256, 2) ConvKernel(ConvArgs a)
 }
 
 // ---------------------------------------------------------- weight gradient
-// Partial sums of one workgroup over its tiles (64 pixels of one symbol
-// row): part[tap][co][ci] = sum_p dz[p][co] a[p + off(tap)][ci] and
-// part[9 COUT CIN + co] = sum_p dz[p][co].  Thread: co = t % COUT and the
-// channel group g = t / COUT of CIN / (256 / COUT) input channels.
-template <int CIN, int COUT, int HALO>
-__global__ void __launch_bounds__(256) WgradKernel(const bf16 *__restrict__ act, const bf16 *__restrict__ dz,
-                                                   float *__restrict__ part, uint32_t S, uint32_t W, int dil_arg)
+// Workgroups (and partial sums) of one layer's weight gradient: a row step
+// costs about 0.5 us of a CU, a workgroup's partial (up to 148 KB written and
+// read again) about 0.06 us of the chip, so their sum is least near
+// sqrt(8 steps) workgroups, at most one per CU.
+inline uint32_t WgradGroups(uint32_t steps, uint32_t cus)
 {
-    constexpr int TILE = 64;
-    constexpr int G = 256 / COUT;
-    constexpr int CG = CIN / G;
-    __shared__ float sa[3][TILE + 2 * HALO][CIN];
-    const int dil = HALO == 1 ? 1 : dil_arg;
-    const int tw = TILE + 2 * dil;
-    __shared__ float sd[TILE][COUT];
-    const int t = threadIdx.x;
-    const int co = t % COUT, g = t / COUT;
-    float acc[9][CG];
-#pragma unroll
-    for (int k = 0; k < 9; ++k)
-#pragma unroll
-        for (int c = 0; c < CG; ++c) acc[k][c] = 0.0f;
-    float db = 0.0f;
-    const uint32_t wtiles = (W + TILE - 1) / TILE;
-    const uint32_t ntiles = S * kSym * wtiles;
-    for (uint32_t ti = blockIdx.x; ti < ntiles; ti += gridDim.x) {
-        const uint32_t wt_i = ti % wtiles, sh = ti / wtiles;
-        const uint32_t h = sh % kSym;
-        const size_t s = sh / kSym;
-        const int w0 = static_cast<int>(wt_i) * TILE;
-        for (int e = t; e < 3 * tw * CIN; e += 256) {
-            const int c = e % CIN, rp = e / CIN, p = rp % tw, r = rp / tw;
-            const int hh = static_cast<int>(h) + r - 1, ww = w0 + p - dil;
-            float v = 0.0f;
-            if (hh >= 0 && hh < kSym && ww >= 0 && ww < static_cast<int>(W))
-                v = static_cast<float>(act[((s * kSym + hh) * W + ww) * CIN + c]);
-            sa[r][p][c] = v;
-        }
-        for (int e = t; e < TILE * COUT; e += 256) {
-            const int c = e % COUT, p = e / COUT;
-            const int ww = w0 + p;
-            sd[p][c] = ww < static_cast<int>(W) ? static_cast<float>(dz[((s * kSym + h) * W + ww) * COUT + c]) : 0.0f;
-        }
-        __syncthreads();
-        for (int p = 0; p < TILE; ++p) {
-            const float d = sd[p][co];
-            db += d;
-#pragma unroll
-            for (int kh = 0; kh < 3; ++kh)
-#pragma unroll
-                for (int kw = 0; kw < 3; ++kw) {
-                    const float *ar = &sa[kh][p + kw * dil][g * CG];
-#pragma unroll
-                    for (int c = 0; c < CG; ++c) acc[kh * 3 + kw][c] += d * ar[c];
-                }
-        }
-        __syncthreads();
-    }
-    float *o = part + static_cast<size_t>(blockIdx.x) * (9 * COUT * CIN + COUT);
-#pragma unroll
-    for (int k = 0; k < 9; ++k)
-#pragma unroll
-        for (int c = 0; c < CG; ++c) o[(static_cast<size_t>(k) * COUT + co) * CIN + g * CG + c] = acc[k][c];
-    if (g == 0) o[9 * COUT * CIN + co] = db;
+    uint32_t nb = 1;
+    while (nb * nb < 8u * steps && nb < cus) ++nb;
+    return std::min(nb, steps);
 }
 
-// grad[i] = sum_b part[b][i] in block order.
+// Four 16-bit values of one channel: a group of 16 lanes reads 4 pixels x 16
+// channels (lane i: channels 4 (i % 4) .. + 3 of pixel i / 4) and lane i gets
+// channel i of the 4 pixels (the transposing LDS read of gfx950).
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ inline bf16x8 TransposedFrag(const char *lds, uint32_t byte, uint32_t step)
+{
+    using P = __attribute__((address_space(3))) s16x4 *;
+    const bf16x4 lo = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((P)(lds + byte)));
+    const bf16x4 hi = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((P)(lds + byte + step)));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// Partial weight gradient of one workgroup: part[tap][co][ci] = sum dz[p][co]
+// a[p + off(tap)][ci] and part[9 COUT CIN + co] = sum dz[p][co] over the
+// workgroup's share of the row steps (slot, 64-pixel column, activation row
+// r; consecutive rows of a column are consecutive steps).  The step of row r
+// pairs it with the dz rows r + 1, r, r - 1 (taps kh = 0, 1, 2), so each row
+// of either tensor is read from memory about once.
+//
+// The contraction runs over pixels, on MFMA v_mfma_f32_32x32x16_bf16 (exact
+// bf16 products, fp32 sums): A = dz^T (32 output channels x 16 pixels), B =
+// the activations (16 pixels x 32 input channels).  Memory and LDS hold the
+// channels of a pixel together, so both operands come through transposing
+// LDS reads, where a tap's pixel offset is an address.  A wave holds the 9
+// taps of one 32 x 32 channel block (144 accumulators) and takes its share of
+// each step's four 16-pixel products: 3 + 3 operands for 9 MFMAs, below the
+// LDS bandwidth.  The rows go memory -> registers two steps ahead, -> LDS one
+// step ahead (two activation rows, a ring of four dz rows); the 64-byte
+// halves of a 128-byte pixel swap on every other pixel pair, which makes the
+// transposing reads of 4 pixels free of bank conflicts.  Outside the grid the
+// loads' range check returns zero.
+//
+// 8 slots of 14 x 3276, 64 -> 64 channels: 49 us (27 GFLOP, 550 TFLOP/s; the
+// two tensors are 94 MB, 19 us of memory) against 1086-2203 us of the fp32
+// vector kernel before it; bound by the two waves per SIMD that 144
+// accumulators leave, the LDS reads of one hiding behind the other's MFMAs.
+template <int CIN, int COUT, int HALO>
+__global__ void __launch_bounds__(512, 2) WgradKernel(const bf16 *__restrict__ act, const bf16 *__restrict__ dz,
+                                                      float *__restrict__ part, uint32_t S, uint32_t W, int dil_arg)
+{
+    constexpr int TILE = 64, THREADS = 512;
+    constexpr int CHI = CIN / 8, CHO = COUT / 8;        // 16-byte chunks per pixel
+    constexpr int APX = TILE + 2 * HALO;                // pixels of an activation row
+    constexpr int NKA = (APX * CHI + THREADS - 1) / THREADS;
+    constexpr int CB_I = CIN / 32, NB = (COUT / 32) * CB_I;  // channel blocks
+    constexpr int KG = 8 / NB, KS = 4 / KG;             // waves per block, 16-pixel products of each
+    constexpr int A_BYTES = APX * CIN * 2, D_BYTES = TILE * COUT * 2;
+    constexpr int N_PART = 9 * COUT * CIN + COUT;
+    static_assert(NB * KG == 8 && KG * KS == 4 && TILE * CHO <= THREADS, "work split");
+    __shared__ __align__(16) char smem[2 * A_BYTES + 4 * D_BYTES];
+    static_assert(sizeof(smem) >= (KG - 1) * NB * 4096 && sizeof(smem) >= THREADS * 32, "reductions reuse the rows");
+    char *const sa = smem, *const sd = smem + 2 * A_BYTES;
+    const int dil = HALO == 1 ? 1 : dil_arg;
+    const int tid = static_cast<int>(threadIdx.x), lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int blk = wave % NB, kg = wave / NB;
+    const int bo = blk / CB_I, bi = blk % CB_I;
+    // Byte of pixel p's 64-byte half `half` in a row of C channels.
+    auto half_at = [](int p, int half, int c) { return c == 64 ? p * 128 + 64 * (half ^ ((p >> 1) & 1)) : p * 64; };
+    const int lpx = 8 * (lane >> 5) + ((lane & 15) >> 2);            // the lane's pixel of a product
+    const int lch = 32 * ((lane >> 4) & 1) + 8 * (lane & 3);         // and channel byte of the half
+    uint32_t aoff[3];
+#pragma unroll
+    for (int kw = 0; kw < 3; ++kw) aoff[kw] = half_at(lpx + kw * dil, bi, CIN) + lch + kg * KS * 16 * CIN * 2;
+    const uint32_t doff = half_at(lpx, bo, COUT) + lch + kg * KS * 16 * COUT * 2;
+
+    f32x16 acc[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[k][i] = 0.0f;
+    float db[8] = {};
+
+    const uint32_t wtiles = (W + TILE - 1) / TILE;
+    const uint64_t steps = static_cast<uint64_t>(S) * wtiles * kSym;
+    const uint32_t t0 = static_cast<uint32_t>(steps * blockIdx.x / gridDim.x);
+    const uint32_t t1 = static_cast<uint32_t>(steps * (blockIdx.x + 1) / gridDim.x);
+    // Position in the sequence of row steps: within a column's share r0 .. r1
+    // the first steps only bring in dz rows (r0 - 1 and r0).
+    struct Pos {
+        uint32_t item;
+        int r0, r1, u;
+    };
+    auto start = [&](uint32_t t) {
+        Pos p;
+        p.item = t / kSym;
+        p.r0 = static_cast<int>(t % kSym);
+        p.r1 = static_cast<int>(min(t1 - 1u, p.item * kSym + kSym - 1u) - p.item * kSym);
+        p.u = max(p.r0 - 2, -1);
+        return p;
+    };
+    auto done = [&](const Pos &p) { return p.item * kSym + static_cast<uint32_t>(p.r1 + 1) >= t1 && p.u > p.r1; };
+    auto next = [&](Pos &p) {
+        ++p.u;
+        if (p.u > p.r1 && (p.item * kSym + p.r1 + 1) < t1) p = start(p.item * kSym + p.r1 + 1);
+    };
+    const uint32_t a_bytes = kSym * W * CIN * 2, d_bytes = kSym * W * COUT * 2;
+    struct Stage {
+        uint4 a[NKA], d;
+    };
+    // The rows of step p: activation row u (a product step), dz row u + 1.
+    auto load = [&](const Pos &p, Stage &st) {
+        if (done(p)) return;
+        const uint32_t s = p.item / wtiles;
+        const int w0 = static_cast<int>(p.item % wtiles) * TILE;
+        const bf16 *as = act + static_cast<size_t>(s) * kSym * W * CIN;
+        const bf16 *ds = dz + static_cast<size_t>(s) * kSym * W * COUT;
+        if (p.u >= p.r0) {
+#pragma unroll
+            for (int k = 0; k < NKA; ++k) {
+                const int e = k * THREADS + tid, px = e / CHI;
+                const int ww = w0 - dil + px;
+                const bool in = px < TILE + 2 * dil && ww >= 0 && ww < static_cast<int>(W);
+                st.a[k] = BufferLoad16(as, a_bytes, in ? 16u * ((p.u * W + ww) * CHI + e % CHI) : kOutside);
+            }
+        }
+        const int px = tid / CHO, ww = w0 + px;
+        const bool in = px < TILE && ww < static_cast<int>(W) && p.u + 1 < kSym;
+        st.d = BufferLoad16(ds, d_bytes, in ? 16u * (((p.u + 1) * W + ww) * CHO + tid % CHO) : kOutside);
+    };
+    auto store = [&](const Pos &p, const Stage &st, uint32_t n) {
+        if (done(p)) return;
+        if (p.u >= p.r0) {
+            char *row = sa + (n & 1u) * A_BYTES;
+#pragma unroll
+            for (int k = 0; k < NKA; ++k) {
+                const int e = k * THREADS + tid, px = e / CHI, c = e % CHI;
+                if (px < APX) *reinterpret_cast<uint4 *>(row + half_at(px, c >> 2, CIN) + 16 * (c & 3)) = st.a[k];
+            }
+        }
+        const int px = tid / CHO, c = tid % CHO;
+        if (px < TILE) {
+            *reinterpret_cast<uint4 *>(sd + (n & 3u) * D_BYTES + half_at(px, c >> 2, COUT) + 16 * (c & 3)) = st.d;
+            if (p.u + 1 >= p.r0 && p.u + 1 <= p.r1) {
+                const uint32_t v[4] = {st.d.x, st.d.y, st.d.z, st.d.w};
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    db[j] += __builtin_bit_cast(float, j & 1 ? v[j >> 1] & 0xffff0000u : v[j >> 1] << 16);
+            }
+        }
+    };
+    if (t0 < t1) {
+        Pos cur = start(t0), ahead = cur;
+        Stage s1{}, s2{};
+        load(ahead, s1);
+        store(ahead, s1, 0);
+        next(ahead);
+        load(ahead, s1);
+        Pos mid = ahead;
+        next(ahead);
+        // Step n: its rows are in LDS, those of step n + 1 in s1, and those of
+        // n + 2 are loaded.  The barrier makes every wave's part of step n's
+        // rows visible and frees the rows last read at step n - 1, which the
+        // stores after the products overwrite.
+        for (uint32_t n = 0; !done(cur); ++n) {
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+            asm volatile("" : : : "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" : : : "memory");
+            load(ahead, s2);
+            if (cur.u >= cur.r0) {
+                const char *ar = sa + (n & 1u) * A_BYTES;
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) {
+                    bf16x8 fa[3];
+#pragma unroll
+                    for (int kw = 0; kw < 3; ++kw)
+                        fa[kw] = TransposedFrag(ar, aoff[kw] + ks * 16 * CIN * 2, 4 * CIN * 2);
+#pragma unroll
+                    for (int kh = 0; kh < 3; ++kh) {
+                        // dz row u + 1 - kh, brought in at step n - kh.
+                        const int h = cur.u + 1 - kh;
+                        if (h < 0 || h >= kSym) continue;
+                        const bf16x8 fd = TransposedFrag(sd + ((n - kh) & 3u) * D_BYTES,
+                                                         doff + ks * 16 * COUT * 2, 4 * COUT * 2);
+#pragma unroll
+                        for (int kw = 0; kw < 3; ++kw)
+                            acc[kh * 3 + kw] =
+                                __builtin_amdgcn_mfma_f32_32x32x16_bf16(fd, fa[kw], acc[kh * 3 + kw], 0, 0, 0);
+                    }
+                }
+            }
+            store(mid, s1, n + 1);
+            s1 = s2;
+            cur = mid;
+            mid = ahead;
+            next(ahead);
+        }
+    }
+    // The waves of a channel block are summed in wave order, tap by tap.
+    float *o = part + static_cast<size_t>(blockIdx.x) * N_PART;
+    float *red = reinterpret_cast<float *>(smem);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        __syncthreads();
+        if (kg > 0) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) red[((kg - 1) * NB + blk) * 1024 + i * 64 + lane] = acc[k][i];
+        }
+        __syncthreads();
+        if (kg == 0) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                float v = acc[k][i];
+#pragma unroll
+                for (int g = 1; g < KG; ++g) v += red[((g - 1) * NB + blk) * 1024 + i * 64 + lane];
+                const int co = bo * 32 + 8 * (i / 4) + 4 * (lane >> 5) + (i & 3);
+                o[(static_cast<size_t>(k) * COUT + co) * CIN + bi * 32 + (lane & 31)] = v;
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 8; ++j) red[tid * 8 + j] = db[j];
+    __syncthreads();
+    if (tid < COUT) {
+        float v = 0.0f;
+        for (int px = 0; px < TILE; ++px) v += red[(px * CHO + tid / 8) * 8 + tid % 8];
+        o[9 * COUT * CIN + tid] = v;
+    }
+}
+
+// grad[i] = sum_b part[b][i], fixed order: four quarters of the partials,
+// each in order (64 elements x 4 quarters per workgroup: a layer's 36,928
+// elements give 577 workgroups reading whole 256-byte rows).
 __global__ void __launch_bounds__(256) ReduceKernel(const float *__restrict__ part, uint32_t nb, uint32_t n,
                                                     float *__restrict__ grad)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    __shared__ float red[4][64];
+    const uint32_t q = threadIdx.x >> 6, i = blockIdx.x * 64u + (threadIdx.x & 63u);
+    const uint32_t b0 = nb * q / 4u, b1 = nb * (q + 1u) / 4u;
     float s = 0.0f;
-    for (uint32_t b = 0; b < nb; ++b) s += part[static_cast<size_t>(b) * n + i];
-    grad[i] = s;
+    if (i < n) {
+#pragma unroll 8
+        for (uint32_t b = b0; b < b1; ++b) s += part[static_cast<size_t>(b) * n + i];
+    }
+    red[q][threadIdx.x & 63u] = s;
+    __syncthreads();
+    if (q == 0 && i < n) grad[i] = (s + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
 }
 
 // ------------------------------------------------------------------ loss
@@ -931,22 +1108,21 @@ template <int CIN, int COUT>
 void LaunchWgrad(const AiranCeRefiner *r, const bf16 *act, const bf16 *dz, uint32_t S, uint32_t W, int layer,
                  hipStream_t s)
 {
-    const uint32_t ntiles = S * kSym * ((W + 63) / 64);
-    const uint32_t nb = std::min<uint32_t>(ntiles, static_cast<uint32_t>(r->cus) * 2);
+    const uint32_t nb = WgradGroups(S * kSym * ((W + 63) / 64), static_cast<uint32_t>(r->cus));
     const int dil = r->dil[layer];
     if (dil == 1)
-        hipLaunchKernelGGL((WgradKernel<CIN, COUT, 1>), dim3(nb), dim3(256), 0, s, act, dz, r->part, S, W, 1);
+        hipLaunchKernelGGL((WgradKernel<CIN, COUT, 1>), dim3(nb), dim3(512), 0, s, act, dz, r->part, S, W, 1);
     else if (dil <= 2)
-        hipLaunchKernelGGL((WgradKernel<CIN, COUT, 2>), dim3(nb), dim3(256), 0, s, act, dz, r->part, S, W, dil);
+        hipLaunchKernelGGL((WgradKernel<CIN, COUT, 2>), dim3(nb), dim3(512), 0, s, act, dz, r->part, S, W, dil);
     else if (dil <= 4)
-        hipLaunchKernelGGL((WgradKernel<CIN, COUT, 4>), dim3(nb), dim3(256), 0, s, act, dz, r->part, S, W, dil);
+        hipLaunchKernelGGL((WgradKernel<CIN, COUT, 4>), dim3(nb), dim3(512), 0, s, act, dz, r->part, S, W, dil);
     else if (dil <= 8)
-        hipLaunchKernelGGL((WgradKernel<CIN, COUT, 8>), dim3(nb), dim3(256), 0, s, act, dz, r->part, S, W, dil);
+        hipLaunchKernelGGL((WgradKernel<CIN, COUT, 8>), dim3(nb), dim3(512), 0, s, act, dz, r->part, S, W, dil);
     else
-        hipLaunchKernelGGL((WgradKernel<CIN, COUT, kMaxDil>), dim3(nb), dim3(256), 0, s, act, dz, r->part, S, W,
+        hipLaunchKernelGGL((WgradKernel<CIN, COUT, kMaxDil>), dim3(nb), dim3(512), 0, s, act, dz, r->part, S, W,
                            dil);
     const uint32_t n = static_cast<uint32_t>(WeightCount(layer) + kCout[layer]);
-    hipLaunchKernelGGL(ReduceKernel, dim3(airan::CeilDiv(n, 256)), dim3(256), 0, s, r->part, nb, n,
+    hipLaunchKernelGGL(ReduceKernel, dim3(airan::CeilDiv(n, 64)), dim3(256), 0, s, r->part, nb, n,
                        r->grad + ParamOffset(layer));
 }
 
@@ -1057,7 +1233,7 @@ int32_t airan_ce_refiner_Create(const PuschMimoConfig *config, uint32_t max_slot
         return fail(AIRAN_LAUNCH_FAILED);
     r->cus = prop.multiProcessorCount;
     const size_t px = static_cast<size_t>(max_slots) * kSym * g.used;
-    const size_t nwg = static_cast<size_t>(r->cus) * 2;
+    const size_t nwg = static_cast<size_t>(r->cus);  // WgradGroups at most
     r->part_floats = nwg * (9 * 64 * 64 + 64);
     auto alloc = [](auto **p, size_t bytes) { return hipMalloc(reinterpret_cast<void **>(p), bytes) == hipSuccess; };
     bool ok = alloc(&r->params, kParams * 4) && alloc(&r->adam_m, kParams * 4) && alloc(&r->adam_v, kParams * 4) &&

@@ -64,6 +64,15 @@ def test_refiner_gradients_match_oracle(oracle, gpu_stream, S, W, dil, scale):
     ref.close()
 
 
+# The weight gradient's work split: one pixel, a whole 64-pixel column, one
+# past it, and shares of row steps that begin and end inside a column (also
+# with every halo).  The bounds are the ones derived above.
+@pytest.mark.parametrize("S,W,dil", [(1, 1, None), (1, 64, None), (2, 65, [2, 4, 8, 16, 1, 1]),
+                                     (3, 129, [1, 2, 4, 8, 16, 1])], ids=["w1", "w64", "w65", "w129_3slots"])
+def test_refiner_gradients_work_split(oracle, gpu_stream, S, W, dil):
+    test_refiner_gradients_match_oracle(oracle, gpu_stream, S, W, dil, None)
+
+
 def test_refiner_training_beats_ls_interpolation(gpu_stream):
     """Training on slots of one channel (300 ns, 100 Hz, Rx correlation 0.5,
     34 dB) teaches the network something its linear-interpolation input
