@@ -298,14 +298,6 @@ __global__ void __launch_bounds__(256) EstimateInputKernel(__half *__restrict__ 
     }
 }
 
-// x32 = float(x) for an input given in bf16 (airan_ce_refiner_Gradients).
-__global__ void __launch_bounds__(256) WidenKernel(const bf16 *__restrict__ x, float *__restrict__ x32, size_t n)
-{
-    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-         i += static_cast<size_t>(gridDim.x) * blockDim.x)
-        x32[i] = static_cast<float>(x[i]);
-}
-
 // Residual scale per slot: sqrt of the mean over Rx of the slot's noise
 // variance (fp16 [slots][NR]), or 1 without a noise input.
 __global__ void __launch_bounds__(64) NoiseScaleKernel(const __half *__restrict__ noise, uint32_t nr, uint32_t slots,
@@ -329,8 +321,8 @@ struct ConvArgs {
     const bf16 *in;      // [S][14][W][CIN]
     const bf16 *wt;      // [9][COUT][CIN]
     const float *bias;   // [COUT] (kEpiRelu, kEpiResid, kEpiGrid)
-    const bf16 *aux;     // kEpiMask: activation [S][14][W][COUT]
-    const float *aux32;  // kEpiResid: X in fp32 [S][14][W][COUT]
+    const bf16 *aux;     // kEpiMask: activation [S][14][W][COUT]; kEpiResid without aux32: X in bf16
+    const float *aux32;  // kEpiResid: X in fp32 [S][14][W][COUT], or null
     const float *scale;  // kEpiResid, kEpiGrid: residual scale per slot [S]
     bf16 *out;           // kEpiRelu, kEpiMask: [S][14][W][COUT]
     float *out_f32;      // kEpiResid: [S][14][W][COUT]
@@ -379,7 +371,7 @@ __device__ inline uint4 BufferLoad16(const void *base, uint32_t bytes, uint32_t 
 // out[p][co] = epilogue(acc), acc = bias[co] + sum_{tap, ci} in[p + off(tap)][ci]
 // wt[tap][co][ci] (the bias is the accumulator's initial value; none for kEpiMask):
 //   kEpiRelu   bf16(max(acc, 0))
-//   kEpiResid  scale[slot] acc + aux32   (fp32)
+//   kEpiResid  scale[slot] acc + aux32   (fp32; + float(aux) without aux32)
 //   kEpiMask   bf16(aux > 0 ? acc : 0)   (gradient through the ReLU)
 //   kEpiGrid   the residual output straight into the channel grid:
 //              g[co / 2] = fp16(scale[slot] acc + float(g[co / 2]))
@@ -537,9 +529,19 @@ __global__ void __launch_bounds__(256, 2) ConvKernel(ConvArgs a)
             }
             if constexpr (EPI == kEpiResid) {
 #pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    res32[g] = w < W ? *reinterpret_cast<const float4 *>(a.aux32 + px_out * COUT + co0 + 8 * g)
-                                     : make_float4(0, 0, 0, 0);
+                for (int g = 0; g < 4; ++g) {
+                    res32[g] = make_float4(0, 0, 0, 0);
+                    if (w >= W) continue;
+                    const size_t o = px_out * COUT + co0 + 8 * g;
+                    if (a.aux32 != nullptr) {
+                        res32[g] = *reinterpret_cast<const float4 *>(a.aux32 + o);
+                    } else {
+                        // bf16 is the upper half of the fp32 of its value.
+                        const uint2 b = *reinterpret_cast<const uint2 *>(a.aux + o);
+                        res32[g] = make_float4(__uint_as_float(b.x << 16), __uint_as_float(b.x & 0xffff0000u),
+                                               __uint_as_float(b.y << 16), __uint_as_float(b.y & 0xffff0000u));
+                    }
+                }
             }
             // Grid element of accumulator i = 4 g + e: channel co0 + 8 g + e,
             // i.e. link co0 / 2 + 4 g + e / 2 (re for even e, im for odd).
@@ -911,36 +913,57 @@ __global__ void __launch_bounds__(256) ReduceKernel(const float *__restrict__ pa
 // ------------------------------------------------------------------ loss
 // dz = bf16(2 w_s (out - target) / N); per-block sums of w_s (out - target)^2,
 // w_s the weight of the element's slot (1 without weights; the training
-// weights have mean 1 over the batch).
+// weights have mean 1 over the batch).  Grid (blocks per slot, slots); a
+// thread takes 8 elements at a time (the slots hold a multiple of 8; global
+// loads of several words need dword alignment only, which floats have).  Bound
+// by memory: 10 bytes an element, 117 MB for 8 slots of 14 x 3276 x 32 in
+// 20 us; one element at a time in 256 workgroups, with a 64-bit division
+// for its slot, it took 107 us.
 __global__ void __launch_bounds__(256) LossKernel(const float *__restrict__ out, const float *__restrict__ tgt,
                                                   const float *__restrict__ slot_w,
-                                                  const float *__restrict__ res_scale, size_t per_slot,
+                                                  const float *__restrict__ res_scale, uint32_t per_slot,
                                                   bf16 *__restrict__ dz, double *__restrict__ part, size_t n)
 {
     __shared__ double red[4];
     double acc = 0.0;
     const float scale = static_cast<float>(2.0 / static_cast<double>(n));
-    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-         i += static_cast<size_t>(gridDim.x) * blockDim.x) {
-        const float w = slot_w != nullptr ? slot_w[i / per_slot] : 1.0f;
-        const float e = out[i] - tgt[i];
-        acc += static_cast<double>(w) * e * e;
-        // out = aux + scale_s z: the gradient of the last pre-activation z.
-        dz[i] = static_cast<bf16>(w * e * scale * res_scale[i / per_slot]);
+    const uint32_t s = blockIdx.y;
+    const float w = slot_w != nullptr ? slot_w[s] : 1.0f, rs = res_scale[s];
+    const size_t base = static_cast<size_t>(s) * per_slot;
+    for (uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) * 8u; i < per_slot; i += gridDim.x * blockDim.x * 8u) {
+        const float4 o0 = *reinterpret_cast<const float4 *>(out + base + i);
+        const float4 o1 = *reinterpret_cast<const float4 *>(out + base + i + 4);
+        const float4 t0 = *reinterpret_cast<const float4 *>(tgt + base + i);
+        const float4 t1 = *reinterpret_cast<const float4 *>(tgt + base + i + 4);
+        const float e[8] = {o0.x - t0.x, o0.y - t0.y, o0.z - t0.z, o0.w - t0.w,
+                            o1.x - t1.x, o1.y - t1.y, o1.z - t1.z, o1.w - t1.w};
+        bf16x8 d;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            acc += static_cast<double>(w) * e[j] * e[j];
+            // out = aux + scale_s z: the gradient of the last pre-activation z.
+            d[j] = static_cast<bf16>(w * e[j] * scale * rs);
+        }
+        *reinterpret_cast<bf16x8 *>(dz + base + i) = d;
     }
     for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+    if (threadIdx.x == 0)
+        part[blockIdx.y * gridDim.x + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-__global__ void __launch_bounds__(64) LossFinishKernel(const double *__restrict__ part, uint32_t nb, size_t n,
-                                                       float *__restrict__ loss)
+__global__ void __launch_bounds__(256) LossFinishKernel(const double *__restrict__ part, uint32_t nb, size_t n,
+                                                        float *__restrict__ loss)
 {
-    if (threadIdx.x != 0) return;
+    __shared__ double red[4];
     double s = 0.0;
-    for (uint32_t b = 0; b < nb; ++b) s += part[b];
-    *loss = static_cast<float>(s / static_cast<double>(n));
+    for (uint32_t b = threadIdx.x; b < nb; b += blockDim.x) s += part[b];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        *loss = static_cast<float>(((red[0] + red[1]) + (red[2] + red[3])) / static_cast<double>(n));
 }
 
 // ------------------------------------------------------------- optimiser
@@ -1042,7 +1065,7 @@ struct AiranCeRefiner {
 
 namespace {
 
-constexpr uint32_t kLossBlocks = 256;
+constexpr uint32_t kLossBlocks = 2048;  // 8 per CU; at least one per slot (max_slots <= 1024)
 
 template <int CIN, int COUT, int EPI>
 void LaunchConv(const AiranCeRefiner *r, const ConvArgs &a, hipStream_t s)
@@ -1066,10 +1089,11 @@ void LaunchConv(const AiranCeRefiner *r, const ConvArgs &a, hipStream_t s)
 }
 
 // Forward of the network on x [S][14][W][32] -> out [S][14][W][32] fp32,
-// keeping the hidden activations; with grid_re / grid_im the last layer
+// keeping the hidden activations; x32 is the residual's base (null: x
+// itself); with grid_re / grid_im the last layer
 // instead adds its output to the fp16 channel grid [S][16][14][pad] in place
 // (the residual base is the grid itself; slots with keep[s] == 0 untouched).
-void Forward(const AiranCeRefiner *r, const bf16 *x, uint32_t S, uint32_t W, hipStream_t s,
+void Forward(const AiranCeRefiner *r, const bf16 *x, const float *x32, uint32_t S, uint32_t W, hipStream_t s,
              __half *grid_re = nullptr, __half *grid_im = nullptr, const uint8_t *keep = nullptr)
 {
     ConvArgs a{};
@@ -1096,7 +1120,8 @@ void Forward(const AiranCeRefiner *r, const bf16 *x, uint32_t S, uint32_t W, hip
             a.pad = r->g.pad;
             LaunchConv<64, 32, kEpiGrid>(r, a, s);
         } else {
-            a.aux32 = r->x32;
+            a.aux32 = x32;
+            a.aux = x;
             a.scale = r->res_scale;
             a.out_f32 = r->out;
             LaunchConv<64, 32, kEpiResid>(r, a, s);
@@ -1130,10 +1155,12 @@ void LaunchWgrad(const AiranCeRefiner *r, const bf16 *act, const bf16 *dz, uint3
 void Backward(const AiranCeRefiner *r, const bf16 *x, const float *target, const float *slot_w, uint32_t S,
               uint32_t W, float *loss, hipStream_t s)
 {
-    const size_t n = static_cast<size_t>(S) * kSym * W * kCh;
-    hipLaunchKernelGGL(LossKernel, dim3(kLossBlocks), dim3(256), 0, s, r->out, target, slot_w, r->res_scale,
-                       static_cast<size_t>(kSym) * W * kCh, r->dz[0], r->loss_part, n);
-    hipLaunchKernelGGL(LossFinishKernel, dim3(1), dim3(64), 0, s, r->loss_part, kLossBlocks, n,
+    const uint32_t per_slot = kSym * W * kCh;
+    const size_t n = static_cast<size_t>(S) * per_slot;
+    const uint32_t bps = std::min(kLossBlocks / S, airan::CeilDiv(per_slot, 256 * 8));
+    hipLaunchKernelGGL(LossKernel, dim3(bps, S), dim3(256), 0, s, r->out, target, slot_w, r->res_scale, per_slot,
+                       r->dz[0], r->loss_part, n);
+    hipLaunchKernelGGL(LossFinishKernel, dim3(1), dim3(256), 0, s, r->loss_part, bps * S, n,
                        loss != nullptr ? loss : r->loss_dev);
     int cur = 0;
     for (int i = kLayers - 1; i >= 0; --i) {
@@ -1362,13 +1389,13 @@ int32_t airan_ce_refiner_EnqueueWithNoise(AiranCeRefiner *r, const void *h_ls_re
         hipLaunchKernelGGL(EstimateInputKernel<false>, dim3(airan::CeilDiv(g.pad, 64), kSym, slots), dim3(256), 0,
                            s, static_cast<__half *>(h_re), static_cast<__half *>(h_im), r->x, nullptr, g.used, g.pad,
                            true, keep);
-        Forward(r, r->x, slots, g.used, s, static_cast<__half *>(h_re), static_cast<__half *>(h_im), keep);
+        Forward(r, r->x, nullptr, slots, g.used, s, static_cast<__half *>(h_re), static_cast<__half *>(h_im), keep);
         return airan::LaunchStatus();
     }
     const InputArgs ia =
         MakeInput(r, static_cast<const __half *>(h_ls_re), static_cast<const __half *>(h_ls_im), r->x);
     hipLaunchKernelGGL(InputKernel, dim3(airan::CeilDiv(g.used, 256), slots), dim3(256), 0, s, ia);
-    Forward(r, r->x, slots, g.used, s);
+    Forward(r, r->x, r->x32, slots, g.used, s);
     hipLaunchKernelGGL(OutToGridKernel, dim3(airan::CeilDiv(g.pad, 256), kSym, slots), dim3(256), 0, s, r->out, keep,
                        static_cast<__half *>(h_re), static_cast<__half *>(h_im), g.used, g.pad, g.nr, g.nl);
     return airan::LaunchStatus();
@@ -1507,7 +1534,7 @@ int32_t airan_ce_refiner_TrainStep(AiranCeRefiner *r, uint32_t slots, float lr, 
         return AIRAN_INVALID_ARGUMENT;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const uint32_t W = r->g.used;
-    Forward(r, r->x, slots, W, s);
+    Forward(r, r->x, r->x32, slots, W, s);
     Backward(r, r->x, r->target, r->slot_w, slots, W, loss_out, s);
     ++r->step;
     const float bc1 = 1.0f - std::pow(0.9f, static_cast<float>(r->step));
@@ -1521,7 +1548,7 @@ int32_t airan_ce_refiner_TrainStep(AiranCeRefiner *r, uint32_t slots, float lr, 
 int32_t airan_ce_refiner_Forward(AiranCeRefiner *r, uint32_t slots, void *stream)
 {
     if (r == nullptr || stream == nullptr || slots == 0 || slots > r->max_slots) return AIRAN_INVALID_ARGUMENT;
-    Forward(r, r->x, slots, r->g.used, static_cast<hipStream_t>(stream));
+    Forward(r, r->x, r->x32, slots, r->g.used, static_cast<hipStream_t>(stream));
     return airan::LaunchStatus();
 }
 
@@ -1533,9 +1560,7 @@ int32_t airan_ce_refiner_Gradients(AiranCeRefiner *r, const void *x, const void 
         return AIRAN_INVALID_ARGUMENT;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bf16 *xb = static_cast<const bf16 *>(x);
-    hipLaunchKernelGGL(WidenKernel, dim3(256), dim3(256), 0, s, xb, r->x32,
-                       static_cast<size_t>(slots) * kSym * width * kCh);
-    Forward(r, xb, slots, width, s);
+    Forward(r, xb, nullptr, slots, width, s);
     Backward(r, xb, static_cast<const float *>(target), nullptr, slots, width, loss, s);
     if (hipMemcpyAsync(grad, r->grad, kParams * 4, hipMemcpyDeviceToDevice, s) != hipSuccess)
         return AIRAN_LAUNCH_FAILED;
