@@ -53,5 +53,5 @@ extern "C" int32_t airan_InitDevice(void)
 {
     int32_t st = airan::InitGoldTables();
     if (st == AIRAN_OK) st = airan::InitOfdmTables();
-    return st != AIRAN_OK ? st : airan::InitLdpcScratch();
+    return st != AIRAN_OK ? st : airan::InitLdpcTables();
 }

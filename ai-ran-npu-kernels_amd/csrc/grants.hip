@@ -184,8 +184,9 @@ struct AiranGrantBatch {
     uint32_t n_tiles = 0, tile = 256;
     std::vector<RaggedTile> host_tiles_src;  // (grant, ds, used) per row, for rebuilding tiles
     RaggedCb *cbs = nullptr;
-    uint32_t *reg_list = nullptr, *ws_list = nullptr, *tb_first = nullptr, *tb_count = nullptr;
-    uint32_t n_reg = 0, n_ws = 0;
+    uint32_t *many_list = nullptr, *few_list = nullptr, *other_list = nullptr;  // decoder launches
+    uint32_t *tb_first = nullptr, *tb_count = nullptr;
+    uint32_t n_many = 0, n_few = 0, n_other = 0;
     // CE groups: grants of one shape, adjacent in the channel buffers.
     struct CeGroup {
         ShapeKey key;
@@ -205,8 +206,7 @@ struct AiranGrantBatch {
     __half *h_re = nullptr, *h_im = nullptr;
     size_t ce_ws_bytes = 0;
     uint32_t *gold = nullptr;
-    int16_t *cw = nullptr, *lam = nullptr;
-    uint2 *ldpc_ws = nullptr;
+    int16_t *cw = nullptr;
     int8_t *bits = nullptr;
     uint8_t *iters = nullptr, *cb_ok = nullptr, *tb_ok = nullptr;
     uint32_t *tb_part = nullptr;
@@ -259,9 +259,9 @@ int32_t EnqueueStages(AiranGrantBatch *b, const void *iq, hipStream_t s)
                        b->h_im, b->noise_ce, b->gold, b->cw, b->grants, b->tiles);
     if ((st = airan::LaunchStatus()) != AIRAN_OK) return st;
     const uint32_t ncb = static_cast<uint32_t>(b->num_cb);
-    if ((st = airan::LaunchRateDematchRagged(b->grants, b->cbs, ncb, b->cw, b->lam, s)) != AIRAN_OK) return st;
-    if ((st = airan::LaunchLdpcRagged(b->cbs, b->reg_list, b->n_reg, b->ws_list, b->n_ws, b->opts.ldpc_iterations,
-                                      b->opts.early_stop != 0, b->lam, b->bits, b->iters, b->ldpc_ws, s)) != AIRAN_OK)
+    if ((st = airan::LaunchLdpcRagged(b->cbs, b->grants, {b->many_list, b->n_many}, {b->few_list, b->n_few},
+                                      {b->other_list, b->n_other}, b->opts.ldpc_iterations, b->opts.early_stop != 0,
+                                      b->cw, b->bits, b->iters, s)) != AIRAN_OK)
         return st;
     return airan::LaunchCrcRagged(b->cbs, ncb, b->bits, b->cb_ok, b->tb_part, b->tb_first, b->tb_count, b->tb_ok,
                                   b->n, s);
@@ -318,7 +318,7 @@ int32_t airan_pusch_grants_Create(const PuschMimoConfig *configs, const AiranTbP
     std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) { return keys[x] < keys[y]; });
     std::vector<RaggedGrant> rec(n);
     b->layout.resize(n);
-    uint64_t iq = 0, rx = 0, ref = 0, cwo = 0, gold = 0, bits = 0, lam = 0, ws = 0, cbi = 0;
+    uint64_t iq = 0, rx = 0, ref = 0, cwo = 0, gold = 0, bits = 0, cbi = 0;
     for (uint32_t i = 0; i < n; ++i) {
         const Geom &g = geom[i];
         const AiranTbPlanV1 &p = plans[i];
@@ -410,7 +410,7 @@ int32_t airan_pusch_grants_Create(const PuschMimoConfig *configs, const AiranTbP
     std::map<uint32_t, std::vector<RaggedStream>> streams;
     std::vector<RaggedItem> gen, ls, nz;
     std::vector<RaggedCb> cbs;
-    std::vector<uint32_t> reg, wsl, tb_first(n), tb_count(n);
+    std::vector<uint32_t> many, few, other, tb_first(n), tb_count(n);
     for (uint32_t i = 0; i < n; ++i) {
         const Geom &g = geom[i];
         const AiranTbPlanV1 &p = plans[i];
@@ -442,16 +442,12 @@ int32_t airan_pusch_grants_Create(const PuschMimoConfig *configs, const AiranTbP
             c.filler = p.filler;
             c.k = p.K;
             c.rows = rows;
-            c.lam_off = lam;
-            lam += 68ull * p.Z;
             c.bits_off = b->layout[i].bits_offset + static_cast<uint64_t>(r) * p.K;
-            c.ws_off = ws;
-            if (rows > 8) ws += static_cast<uint64_t>(rows) * p.Z;
             c.crc_cb = p.crc_cb;
             c.len_tb = p.crc_tb;
             c.poly_tb = airan::CrcTbPoly(p.crc_tb);
             c.xpow = airan::CrcXpowHost(p, r);
-            (rows > 8 ? wsl : reg).push_back(static_cast<uint32_t>(cbs.size()));
+            (p.Z != 384 ? other : rows > airan::LdpcFewRows() ? many : few).push_back(static_cast<uint32_t>(cbs.size()));
             cbs.push_back(c);
         }
     }
@@ -469,17 +465,22 @@ int32_t airan_pusch_grants_Create(const PuschMimoConfig *configs, const AiranTbP
     b->n_gen = static_cast<uint32_t>(gen.size());
     b->n_ls = static_cast<uint32_t>(ls.size());
     b->n_noise = static_cast<uint32_t>(nz.size());
-    b->n_reg = static_cast<uint32_t>(reg.size());
-    b->n_ws = static_cast<uint32_t>(wsl.size());
+    // The decoder's longest blocks (most rows) first, so that the launch ends
+    // with short ones.
+    for (std::vector<uint32_t> *l : {&many, &few, &other})
+        std::stable_sort(l->begin(), l->end(), [&](uint32_t x, uint32_t y) { return cbs[x].rows > cbs[y].rows; });
+    b->n_many = static_cast<uint32_t>(many.size());
+    b->n_few = static_cast<uint32_t>(few.size());
+    b->n_other = static_cast<uint32_t>(other.size());
     if (!Upload(&b->grants, rec, &by) || !Upload(&b->gen_items, gen, &by) || !Upload(&b->ls_items, ls, &by) ||
-        !Upload(&b->noise_items, nz, &by) || !Upload(&b->cbs, cbs, &by) || !Upload(&b->reg_list, reg, &by) ||
-        !Upload(&b->ws_list, wsl, &by) || !Upload(&b->tb_first, tb_first, &by) ||
+        !Upload(&b->noise_items, nz, &by) || !Upload(&b->cbs, cbs, &by) || !Upload(&b->many_list, many, &by) ||
+        !Upload(&b->few_list, few, &by) || !Upload(&b->other_list, other, &by) || !Upload(&b->tb_first, tb_first, &by) ||
         !Upload(&b->tb_count, tb_count, &by) || !DevAlloc(&b->rx_re, rx, &by) || !DevAlloc(&b->rx_im, rx, &by) ||
         !DevAlloc(&b->ref_re, ref, &by) || !DevAlloc(&b->ref_im, ref, &by) || !DevAlloc(&b->hls_re, hls, &by) ||
         !DevAlloc(&b->hls_im, hls, &by) || !DevAlloc(&b->noise_ls, noise, &by) ||
         !DevAlloc(&b->noise_ce, noise, &by) || !DevAlloc(&b->h_re, h, &by) || !DevAlloc(&b->h_im, h, &by) ||
         !DevAlloc(&b->gold, gold, &by) ||
-        !DevAlloc(&b->cw, cwo, &by) || !DevAlloc(&b->lam, lam, &by) || !DevAlloc(&b->ldpc_ws, ws, &by) ||
+        !DevAlloc(&b->cw, cwo, &by) ||
         !DevAlloc(&b->bits, bits, &by) || !DevAlloc(&b->iters, b->num_cb, &by) ||
         !DevAlloc(&b->cb_ok, b->num_cb, &by) || !DevAlloc(&b->tb_ok, n, &by) ||
         !DevAlloc(&b->tb_part, b->num_cb, &by))
@@ -544,9 +545,9 @@ void airan_pusch_grants_Destroy(AiranGrantBatch *b)
         if (f.streams) (void)hipFree(f.streams);
     airan::DestroyCeGrouped(b->ce_grouped);
     if (b->ce_ws_all) (void)hipFree(b->ce_ws_all);
-    void *bufs[] = {b->grants, b->gen_items, b->ls_items, b->noise_items, b->tiles, b->cbs, b->reg_list, b->ws_list,
+    void *bufs[] = {b->grants, b->gen_items, b->ls_items, b->noise_items, b->tiles, b->cbs, b->many_list, b->few_list, b->other_list,
                     b->tb_first, b->tb_count, b->rx_re, b->rx_im, b->ref_re, b->ref_im, b->hls_re, b->hls_im,
-                    b->noise_ls, b->noise_ce, b->h_re, b->h_im, b->gold, b->cw, b->lam, b->ldpc_ws,
+                    b->noise_ls, b->noise_ce, b->h_re, b->h_im, b->gold, b->cw,
                     b->bits, b->iters, b->cb_ok, b->tb_ok, b->tb_part};
     for (void *p : bufs)
         if (p) (void)hipFree(p);

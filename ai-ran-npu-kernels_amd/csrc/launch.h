@@ -130,14 +130,17 @@ int32_t LaunchDmrsRagged(const RaggedGrant *grants, const RaggedItem *gen_items,
                          __half *noise, hipStream_t s);
 // c_init of DMRS symbol `symbol` of cfg (mimo_dmrs_gen.cpp:38-45).
 uint32_t HostDmrsCinit(const PuschMimoConfig &cfg, uint32_t symbol);
-// Rate dematch of every code block into its decoder input (lam_off).
-int32_t LaunchRateDematchRagged(const RaggedGrant *grants, const RaggedCb *cbs, uint32_t num_cb, const int16_t *cw,
-                                int16_t *out, hipStream_t s);
-// LDPC (FP16 messages) of the listed code blocks: reg_list with <= 8 rows
-// (messages in registers), ws_list with more (messages in ws at ws_off).
-int32_t LaunchLdpcRagged(const RaggedCb *cbs, const uint32_t *reg_list, uint32_t n_reg, const uint32_t *ws_list,
-                         uint32_t n_ws, uint32_t iters, bool early_stop, const int16_t *lam, int8_t *bits,
-                         uint8_t *iters_out, uint2 *ws, hipStream_t s);
+// LDPC (FP16 messages) of the listed code blocks, from the grants' codeword
+// LLRs (rate dematch in the decoder's load): Z = 384 with more than
+// LdpcFewRows() rows, with at most as many, and blocks of other Z.
+struct RaggedLdpcList {
+    const uint32_t *list = nullptr;
+    uint32_t count = 0;
+};
+uint32_t LdpcFewRows();
+int32_t LaunchLdpcRagged(const RaggedCb *cbs, const RaggedGrant *grants, const RaggedLdpcList &many,
+                         const RaggedLdpcList &few, const RaggedLdpcList &other, uint32_t iters, bool early_stop,
+                         const int16_t *cw, int8_t *bits, uint8_t *iters_out, hipStream_t s);
 // CRC24B of every code block and the CRC of every TB (tb_first / tb_count
 // index the blocks of each TB).
 int32_t LaunchCrcRagged(const RaggedCb *cbs, uint32_t num_cb, const int8_t *bits, uint8_t *cb_ok, uint32_t *tb_part,

@@ -7,12 +7,13 @@
 // (int16 value < 0) (:719-780), i.e. a REF-mode posterior in [-0.5, 0)
 // decodes to 0.
 //
-// Mapping: one workgroup per code block; the posterior [68][Z] lives in LDS
-// as fp16 (52 KB at Z = 384); thread i owns check i of every row, so within a row the
-// Z threads touch a permutation of each column (no LDS write conflicts) and a
-// barrier separates rows.  A check's messages are stored compressed
-// (min1, min2, index of min1, sign bits): 8 bytes per (row, check) in
-// registers when the active rows fit REG_ROWS, otherwise in a global workspace.
+// Two kernels.  LdpcPairKernel (FP16 messages, at most 8 active rows): two
+// code blocks per workgroup, one in each fp16 half of every posterior word.
+// LdpcCheckPairKernel (the rest): one code block per workgroup, two checks
+// of it per lane.  In both the posterior lives in LDS, the message state in
+// registers, a thread owns the same checks of every row (within a row the
+// threads touch a permutation of each column, so nothing conflicts) and a
+// barrier separates rows.
 #include <algorithm>
 #include <mutex>
 
@@ -22,257 +23,26 @@
 #include "ragged.h"
 #include "ratematch.h"
 
-// Posterior of the code block owned by the workgroup ([68][Z] x 16 bit).
+// Posterior of the code blocks owned by a pair decoder workgroup whose
+// lifting size is not known at compile time.
 extern __shared__ uint16_t airan_ldpc_lam[];
-
-// Message state of airan_ldpc_decode_EnqueueNoAlloc: a fixed device array
-// instead of a caller workspace, for callers that cannot allocate.  Each GPU
-// the library runs on holds its own copy until the process ends.  32 MiB
-// covers the reference's 23-slot transport block (143 code blocks at all 46
-// rows, Z = 384: 20.2 MB).
-constexpr size_t kNoAllocScratchBytes = size_t{32} << 20;
-static __device__ __align__(256) uint2 scratch[kNoAllocScratchBytes / sizeof(uint2)];
 
 namespace {
 
-struct Bg1Dev {
-    uint16_t row_start[AIRAN_BG1_ROWS + 1];
-    uint8_t col[AIRAN_BG1_EDGES];
-    uint16_t shift[AIRAN_BG1_EDGES];
-};
-
-__constant__ Bg1Dev kBg1;
-
-// Per-device "constant tables loaded" flags of kBg1 and kLift, guarded by
+// Per-device "constant tables loaded" flags of kLift and kEdges, guarded by
 // one mutex (callers on several host threads may load them at once).
 std::mutex g_table_mutex;
-bool g_table_loaded[64] = {};
-
-int32_t LoadTable()
-{
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return AIRAN_LAUNCH_FAILED;
-    std::lock_guard<std::mutex> lock(g_table_mutex);
-    if (g_table_loaded[dev]) return AIRAN_OK;
-    Bg1Dev t{};
-    for (int i = 0; i <= AIRAN_BG1_ROWS; ++i) t.row_start[i] = AIRAN_BG1_ROW_START[i];
-    for (int e = 0; e < AIRAN_BG1_EDGES; ++e) {
-        t.col[e] = AIRAN_BG1_COL[e];
-        t.shift[e] = AIRAN_BG1_SHIFT[e];
-    }
-    if (hipMemcpyToSymbol(HIP_SYMBOL(kBg1), &t, sizeof(t)) != hipSuccess) return AIRAN_LAUNCH_FAILED;
-    g_table_loaded[dev] = true;
-    return AIRAN_OK;
-}
-
-// Device address of `scratch` per device (hipGetSymbolAddress with that
-// device current, at its first airan_InitDevice); the array's name is a host
-// stand-in and must not be passed to a kernel.
-void *g_scratch_ptr[64] = {};
-
-constexpr int kMaxDeg = AIRAN_BG1_MAX_DEG;
-
-__device__ inline float H16(float v) { return __half2float(__float2half_rn(v)); }
-
-// Message of edge k reconstructed from the compressed state
-// (w0 = fp16 min1 | fp16 min2 << 16, w1 = sign bits | index of min1 << 24):
-// alpha * sign * magnitude rounded to fp16, then (MODE_REF) stored as int8.
-template <int MODE>
-__device__ inline float EdgeMsg(uint32_t w0, uint32_t w1, int k)
-{
-    const uint32_t idx = w1 >> 24;
-    const uint32_t signs = w1 & 0x7ffffu;
-    const uint16_t mh = static_cast<uint16_t>(static_cast<uint32_t>(k) == idx ? (w0 >> 16) : (w0 & 0xffffu));
-    const float mag = __half2float(__ushort_as_half(mh));
-    const uint32_t neg = (__popc(signs) ^ (signs >> k)) & 1u;
-    const float nm = H16((neg ? -0.75f : 0.75f) * mag);
-    if (MODE == AIRAN_LDPC_MODE_REF) {
-        float q = rintf(nm);
-        return q > 127.0f ? 127.0f : (q < -127.0f ? -127.0f : q);
-    }
-    return nm;
-}
-
-// Check i of row r: gather, subtract old message, min1/min2/signs, scatter
-// the updated posterior (fp16 LDS).  Updates the compressed state in place.
-template <int MODE>
-__device__ inline void ProcessRow(uint16_t *lam, int r, uint32_t i, uint32_t Z, uint32_t &w0,
-                                  uint32_t &w1)
-{
-    const int e0 = kBg1.row_start[r];
-    const int deg = kBg1.row_start[r + 1] - e0;
-    uint32_t addr[kMaxDeg];
-    float ext[kMaxDeg];
-    float m1 = INFINITY, m2 = INFINITY;
-    uint32_t idx = 0, signs = 0;
-#pragma unroll
-    for (int k = 0; k < kMaxDeg; ++k) {
-        if (k < deg) {
-            const uint32_t z = static_cast<uint32_t>(kBg1.shift[e0 + k]) % Z;
-            uint32_t p = i + z;
-            p = p >= Z ? p - Z : p;
-            addr[k] = static_cast<uint32_t>(kBg1.col[e0 + k]) * Z + p;
-            const float v = __half2float(__ushort_as_half(lam[addr[k]]));
-            ext[k] = H16(v - EdgeMsg<MODE>(w0, w1, k));
-            const float a = fabsf(ext[k]);
-            signs |= static_cast<uint32_t>(!(ext[k] >= 0.0f)) << k;
-            if (a < m1) {
-                m2 = m1;
-                m1 = a;
-                idx = static_cast<uint32_t>(k);
-            } else if (a < m2) {
-                m2 = a;
-            }
-        }
-    }
-    w0 = static_cast<uint32_t>(__half_as_ushort(__float2half_rn(m1))) |
-         (static_cast<uint32_t>(__half_as_ushort(__float2half_rn(m2))) << 16);
-    w1 = signs | (idx << 24);
-#pragma unroll
-    for (int k = 0; k < kMaxDeg; ++k) {
-        if (k < deg) {
-            const uint32_t neg = (__popc(signs) ^ (signs >> k)) & 1u;
-            const float mag = (static_cast<uint32_t>(k) == idx) ? m2 : m1;
-            const float nm = H16((neg ? -0.75f : 0.75f) * mag);
-            lam[addr[k]] = __half_as_ushort(__float2half_rn(ext[k] + nm));
-        }
-    }
-}
-
-// MODE_REF: the reference's rint(clamp(v, +-5120)) < 0, which for an fp16
-// posterior is v < -0.5 (a NaN gives 0).  MODE_FP16 (no reference
-// counterpart): v < 0.
-template <int MODE>
-__device__ inline bool HardBit(const uint16_t *lam, uint32_t a)
-{
-    const float v = __half2float(__ushort_as_half(lam[a]));
-    return MODE == AIRAN_LDPC_MODE_REF ? v < -0.5f : v < 0.0f;
-}
-
-// True when check i of every active row is satisfied by the hard decisions.
-template <int MODE>
-__device__ inline bool ChecksOk(const uint16_t *lam, int rows, uint32_t i, uint32_t Z)
-{
-    bool ok = true;
-    for (int r = 0; r < rows; ++r) {
-        const int e0 = kBg1.row_start[r], e1 = kBg1.row_start[r + 1];
-        uint32_t par = 0;
-        for (int e = e0; e < e1; ++e) {
-            uint32_t p = i + static_cast<uint32_t>(kBg1.shift[e]) % Z;
-            p = p >= Z ? p - Z : p;
-            par ^= HardBit<MODE>(lam, static_cast<uint32_t>(kBg1.col[e]) * Z + p) ? 1u : 0u;
-        }
-        ok &= par == 0;
-    }
-    return ok;
-}
-
-struct LdpcDev {
-    uint32_t z, k, iters, rows, early_stop;
-};
-
-// RAGGED: block b decodes code block list[b] of a ragged batch, with that
-// block's Z, K, rows and buffer offsets (no lam_out).
-template <int MODE, int REG_ROWS, bool RAGGED = false>
-__global__ void __launch_bounds__(384) LdpcKernel(const int16_t *__restrict__ lam_in,
-                                                  int8_t *__restrict__ bits,
-                                                  int16_t *__restrict__ lam_out,
-                                                  uint8_t *__restrict__ iters_out,
-                                                  uint2 *__restrict__ msg_ws, LdpcDev d,
-                                                  const airan::RaggedCb *__restrict__ cbs = nullptr,
-                                                  const uint32_t *__restrict__ list = nullptr)
-{
-    uint16_t *lam = airan_ldpc_lam;
-    uint32_t cb = blockIdx.x;
-    size_t lam_off, bits_off, ws_off;
-    if constexpr (RAGGED) {
-        cb = list[blockIdx.x];
-        const airan::RaggedCb &c = cbs[cb];
-        d.z = c.z;
-        d.k = c.k;
-        d.rows = c.rows;
-        lam_off = c.lam_off;
-        bits_off = c.bits_off;
-        ws_off = c.ws_off;
-    } else {
-        lam_off = static_cast<size_t>(cb) * 68u * d.z;
-        bits_off = static_cast<size_t>(cb) * d.k;
-        ws_off = static_cast<size_t>(cb) * d.rows * d.z;
-    }
-    const uint32_t Z = d.z, N = 68u * Z;
-    const uint32_t i = threadIdx.x;
-    const int16_t *src = lam_in + lam_off;
-    for (uint32_t t = i; t < N; t += blockDim.x) {
-        const float scale = MODE == AIRAN_LDPC_MODE_REF ? 1.0f : 1.0f / 256.0f;
-        lam[t] = __half_as_ushort(__float2half_rn(static_cast<float>(src[t]) * scale));
-    }
-    uint32_t rw0[REG_ROWS > 0 ? REG_ROWS : 1], rw1[REG_ROWS > 0 ? REG_ROWS : 1];
-#pragma unroll
-    for (int r = 0; r < (REG_ROWS > 0 ? REG_ROWS : 1); ++r) {
-        rw0[r] = 0;
-        rw1[r] = 0;
-    }
-    uint2 *ws = msg_ws + ws_off;
-    if (REG_ROWS == 0 && i < Z)
-        for (uint32_t r = 0; r < d.rows; ++r) ws[r * Z + i] = make_uint2(0u, 0u);
-    __syncthreads();
-    const int rows = static_cast<int>(d.rows);
-    uint32_t it = 0;
-    for (; it < d.iters; ++it) {
-        if (REG_ROWS > 0) {
-#pragma unroll
-            for (int r = 0; r < REG_ROWS; ++r) {
-                if (r < rows) {
-                    if (i < Z) ProcessRow<MODE>(lam, r, i, Z, rw0[r], rw1[r]);
-                    __syncthreads();
-                }
-            }
-        } else {
-            for (int r = 0; r < rows; ++r) {
-                if (i < Z) {
-                    uint2 s = ws[r * Z + i];
-                    ProcessRow<MODE>(lam, r, i, Z, s.x, s.y);
-                    ws[r * Z + i] = s;
-                }
-                __syncthreads();
-            }
-        }
-        if (d.early_stop) {
-            const bool ok = i < Z ? ChecksOk<MODE>(lam, rows, i, Z) : true;
-            if (__syncthreads_and(ok ? 1 : 0)) {
-                ++it;
-                break;
-            }
-        }
-    }
-    if (iters_out != nullptr && i == 0) iters_out[cb] = static_cast<uint8_t>(it);
-    int8_t *bo = bits + bits_off;
-    for (uint32_t t = i; t < d.k; t += blockDim.x) bo[t] = HardBit<MODE>(lam, t) ? 1 : 0;
-    if (!RAGGED && lam_out != nullptr) {
-        int16_t *lo = lam_out + lam_off;
-        const float clip = MODE == AIRAN_LDPC_MODE_REF ? 5120.0f : 20.0f;
-        const float out_scale = MODE == AIRAN_LDPC_MODE_REF ? 1.0f : 256.0f;
-        for (uint32_t t = i; t < N; t += blockDim.x) {
-            float v = __half2float(__ushort_as_half(lam[t]));
-            v = v > clip ? clip : (v < -clip ? -clip : v);
-            lo[t] = static_cast<int16_t>(rintf(v * out_scale));
-        }
-    }
-}
-
-constexpr int kRegRows = 8;
 
 // ------------------------------------------------------------------ fast path
 // FP16 messages and at most kFastRows active rows (every code rate above
-// about 0.6), the same arithmetic as LdpcKernel<MODE_FP16> with:
+// about 0.75), with:
 //  * row degrees fixed at compile time and per-lifting-size edge words
 //    (col * Z | (shift mod Z) << 16) in constant memory, so an edge costs a
 //    scalar load and three VALU ops of addressing;
 //  * fp16 VALU arithmetic on the posterior: a single fp16 add/sub/mul of
 //    fp16 operands rounds exactly like the fp32 operation rounded to fp16
 //    (fp32 has 24 >= 2*11 + 2 significand bits, so rounding twice is
-//    innocuous), and the compressed state keeps the scaled magnitudes
-//    fp16(0.75 * min), which are the message magnitudes themselves;
+//    innocuous);
 //  * LDS holding only the (22 + rows) columns the active rows touch, so
 //    several code blocks share a CU; columns beyond never change.
 // With FUSED the decoder input is de-rate-matched on the fly from the
@@ -346,7 +116,7 @@ __device__ __forceinline__ uint32_t LiftAddr(uint32_t w, uint32_t i, uint32_t Z)
 //   above 0x7c00: negative, or a NaN), parity p;
 //   msg_k = (|x_k| == |min1| ? 0.75 min2 : 0.75 min1) with sign
 //   p ^ sign(x_k), and lam_k = x_k + msg_k.
-// This is the compressed-state decoder's arithmetic exactly: an edge whose
+// Selecting the second minimum by magnitude is selecting it by index: an edge whose
 // magnitude equals min1 without being min1's index implies min2 == min1, so
 // selecting by magnitude instead of index changes no value; and a message's
 // sign differs from the recorded sign bit only for a NaN extrinsic, whose
@@ -916,6 +686,615 @@ __global__ void __launch_bounds__(384)
     }
 }
 
+// ------------------------------------------------------------------ any rows
+// One code block per workgroup, two checks per lane: lane i of the first Z/2
+// owns checks i and i + Z/2 of every row.  Word j of a column in LDS holds
+// positions j (low half) and j + Z/2 (high half), so an edge with shift s
+// takes one word -- that of (i + s) mod Z/2 -- its halves exchanged where i + s
+// mod Z lands in the upper half (a rotate by 16 on the read and the write),
+// and every operation of the row is a packed one on both checks.  Unlike two
+// blocks per workgroup (LdpcPairKernel) this halves the LDS and the waves of a
+// block, so blocks of any rows, lifting size and iteration count share a CU.
+//
+// Message state, all in registers: the messages themselves for the four
+// degree-19 rows (76 words) and, up to kFewRows rows, for the others; beyond,
+// an extension row keeps its two scaled magnitudes and the signs and
+// minimum flags of its edges (one bit per edge and check), from which the old
+// message is rebuilt as it was computed.  Rows kStaticRows .. 45 (degrees 4 to
+// 8) run in one rolled loop over a table of edge words with their state in
+// register arrays indexed by the row (s_set_gpr_idx): unrolled, the code of
+// 316 edges would not fit the instruction cache.
+//
+// The arithmetic is that of PairRow (see there: values, parity, infinities and
+// NaN).  In MODE_REF the message that is kept (and subtracted in the next
+// iteration) is the reference's int8 one, its magnitude rounded half to even
+// and clamped to 127, while the posterior takes the fp16 one, so posteriors
+// grow from iteration to iteration and may become infinite.
+//
+// Bound by VALU issue (about 21 instructions per edge and two checks with
+// kept messages, 30 with rebuilt ones) and, with fewer blocks than CUs, by a
+// row's latency.  Against one check per lane with a compressed state that
+// went through memory every row, Z = 384: 200 blocks of 46 rows, 8
+// iterations at most 1029 -> 277 us; 143 blocks of 46 rows, 3 iterations, REF
+// 378 -> 135 us; 6 blocks of 9 rows 238 -> 49 us; 2282 ragged blocks, with the
+// rate dematch that was a pass of its own before, 1564 -> 438 us.
+constexpr int kRows = AIRAN_BG1_ROWS;
+constexpr int kFewRows = 10;     // rows of the kernel that keeps every message
+constexpr int kStaticRows = 10;  // rows unrolled; the rest have degrees 4 .. 8
+constexpr int kMinLoopDeg = 4, kMaxLoopDeg = 8;
+
+// Edge words per lifting size: LDS byte of the column's word (shift mod Z/2)
+// in bits 0 .. 15, 4 (Z/2 - shift mod Z/2) in bits 16 .. 25 (the lanes' 4 i
+// from which on the word index wraps), bit 31: shift >= Z/2.  A row's info:
+// first edge | degree << 16.  Padded for reads of kMaxLoopDeg words.
+struct Bg1EdgeDev {
+    uint32_t w[kNumLift][AIRAN_BG1_EDGES + kMaxLoopDeg];
+    uint32_t row[kRows + 2];
+};
+
+__constant__ Bg1EdgeDev kEdges;
+
+bool g_edges_loaded[64] = {};
+
+int32_t LoadEdgeTable()
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return AIRAN_LAUNCH_FAILED;
+    std::lock_guard<std::mutex> lock(g_table_mutex);
+    if (g_edges_loaded[dev]) return AIRAN_OK;
+    static Bg1EdgeDev t;  // under the lock
+    t = Bg1EdgeDev{};
+    for (int r = 0; r < kRows; ++r) {
+        const uint32_t e0 = AIRAN_BG1_ROW_START[r], deg = AIRAN_BG1_ROW_START[r + 1] - e0;
+        if (r >= kStaticRows && (deg < kMinLoopDeg || deg > kMaxLoopDeg)) return AIRAN_LAUNCH_FAILED;
+        t.row[r] = e0 | deg << 16;
+    }
+    for (int zi = 0; zi < kNumLift; ++zi) {
+        const uint32_t z = 24u << zi, zh = z / 2;
+        for (int e = 0; e < AIRAN_BG1_EDGES; ++e) {
+            const uint32_t s = AIRAN_BG1_SHIFT[e] % z, sh = s % zh;
+            t.w[zi][e] = 4u * (AIRAN_BG1_COL[e] * zh + sh) | 4u * (zh - sh) << 16 | (s >= zh ? 1u << 31 : 0u);
+        }
+    }
+    if (hipMemcpyToSymbol(HIP_SYMBOL(kEdges), &t, sizeof(t)) != hipSuccess) return AIRAN_LAUNCH_FAILED;
+    g_edges_loaded[dev] = true;
+    return AIRAN_OK;
+}
+
+// LDS byte of an edge's word for the lane (4 i = i4) and the rotation that
+// puts check i's position into the low half.
+struct EdgeAt {
+    uint32_t byte, rot;
+};
+
+// Edge e with Z = ZT: column and shift are compile-time constants, in the LDS
+// instruction's offset (the posterior starts at LDS address 0; the hardware
+// adds modulo 2^32, see EdgeByte).
+template <uint32_t ZT>
+__device__ __forceinline__ EdgeAt StaticEdge(int e, uint32_t i4)
+{
+    constexpr uint32_t zh = ZT / 2;
+    const uint32_t s = static_cast<uint32_t>(AIRAN_BG1_SHIFT[e]) % ZT, sh = s % zh;
+    const bool hi = s >= zh, wrap = sh != 0 && i4 >= 4u * (zh - sh);
+    return {(wrap ? i4 - 4u * zh : i4) + 4u * (AIRAN_BG1_COL[e] * zh + sh), wrap != hi ? 16u : 0u};
+}
+
+// The edge of table word w; zh4 = 2 Z.
+__device__ __forceinline__ EdgeAt TableEdge(uint32_t w, uint32_t i4, uint32_t zh4)
+{
+    const bool hi = (w >> 31) != 0, wrap = i4 >= ((w >> 16) & 0x3ffu);
+    return {i4 + (w & 0xffffu) - (wrap ? zh4 : 0u), wrap != hi ? 16u : 0u};
+}
+
+__device__ __forceinline__ uint32_t Rot16(uint32_t v, uint32_t rot) { return __builtin_amdgcn_alignbit(v, v, rot); }
+
+// The row's parity in the sign bits (PairRow's, with its exact count).
+template <int DEG>
+__device__ __forceinline__ uint32_t RowParity(const uint32_t (&x)[DEG], uint32_t sx, uint32_t mx, uint32_t *inf_flag)
+{
+    if (PkSubSatU16(mx, 0x7bff7bffu) != 0) {
+        *inf_flag = 1u;
+        uint32_t cnt = 0;
+#pragma unroll
+        for (int k = 0; k < DEG; ++k) cnt += AboveInf2(x[k]);
+        return (cnt & 1u) << 15 | ((cnt >> 16) & 1u) << 31;
+    }
+    return sx & 0x80008000u;
+}
+
+// int8 magnitude of an fp16 one: round half to even, at most 127 (0x57f0).
+__device__ __forceinline__ uint32_t Int8Magnitude2(uint32_t v)
+{
+    return PkMinU16(WH(__builtin_elementwise_rint(H2(v))), 0x57f057f0u);
+}
+
+// One row: edge(k, i4) places edge k, old(k) is its message (both checks),
+// put(k, x, e, m) takes the new one (e: 1 per half where the edge is at the
+// minimum); s1p and d12 return the kept messages' two magnitudes with the
+// row's parity in the sign bits, as s1p and s2p - s1p (mod 2^16 per half).  The addresses are computed anew for the second pass (three
+// instructions an edge, against two registers and a mask), and a long row is
+// taken kChunk edges at a time, both to stay within the registers.
+template <int MODE, int DEG, typename Edge, typename Old, typename Put>
+__device__ __forceinline__ void CheckRow(uint32_t *lam, uint32_t i4, uint32_t *inf_flag, uint32_t &s1p, uint32_t &d12,
+                                         Edge edge, Old old, Put put)
+{
+    constexpr int kChunk = 7;
+    uint32_t x[DEG];
+    uint32_t m1 = 0x7c007c00u, m2 = 0x7c007c00u, sx = 0, mx = 0;
+#pragma unroll
+    for (int k = 0; k < DEG; ++k) {
+        if (k > 0 && k % kChunk == 0) __builtin_amdgcn_sched_barrier(0);
+        const EdgeAt a = edge(k, i4);
+        x[k] = WH(H2(Rot16(LdsWord(lam, a.byte), a.rot)) - H2(old(k)));
+        const uint32_t mg = x[k] & 0x7fff7fffu;
+        m2 = PkMinU16(m2, PkMaxU16(m1, mg));
+        m1 = PkMinU16(m1, mg);
+        sx ^= x[k];
+        mx = PkMaxU16(mx, mg);
+    }
+    const uint32_t par = RowParity<DEG>(x, sx, mx, inf_flag);
+    const h2_t q = {static_cast<_Float16>(0.75f), static_cast<_Float16>(0.75f)};
+    const uint32_t f1 = WH(q * H2(m1)), f2 = WH(q * H2(m2)), f1p = f1 | par, fd = PkSubU16(f2 | par, f1p);
+    s1p = f1p;
+    d12 = fd;
+    if constexpr (MODE == AIRAN_LDPC_MODE_REF) {
+        s1p = Int8Magnitude2(f1) | par;
+        d12 = PkSubU16(Int8Magnitude2(f2) | par, s1p);
+    }
+    asm volatile("" : "+v"(i4));
+#pragma unroll
+    for (int k = 0; k < DEG; ++k) {
+        if (k > 0 && k % kChunk == 0) __builtin_amdgcn_sched_barrier(0);
+        const EdgeAt a = edge(k, i4);
+        const uint32_t e = PkSubSatU16(0x00010001u, (x[k] & 0x7fff7fffu) ^ m1);
+        const uint32_t sg = x[k] & 0x80008000u, m = PkMadU16(e, fd, f1p) ^ sg;
+        put(k, x[k], e, MODE == AIRAN_LDPC_MODE_REF ? PkMadU16(e, d12, s1p) ^ sg : m);
+        LdsWord(lam, a.byte) = Rot16(WH(H2(x[k]) + H2(m)), a.rot);
+    }
+}
+
+constexpr int StaticDeg(int r) { return AIRAN_BG1_ROW_START[r + 1] - AIRAN_BG1_ROW_START[r]; }
+
+// Unrolled row R with every message kept (msg: this row's words).
+template <int MODE, uint32_t ZT, int R>
+__device__ __forceinline__ void FullRow(uint32_t *lam, const uint32_t *tab, uint32_t i4, uint32_t zh4, uint32_t *msg,
+                                        uint32_t *inf_flag)
+{
+    constexpr int E0 = AIRAN_BG1_ROW_START[R], DEG = StaticDeg(R);
+    uint32_t s1p, d12;
+    auto edge = [&](int k, uint32_t i4) {
+        if constexpr (ZT != 0)
+            return StaticEdge<ZT>(E0 + k, i4);
+        else
+            return TableEdge(tab[E0 + k], i4, zh4);
+    };
+    CheckRow<MODE, DEG>(
+        lam, i4, inf_flag, s1p, d12, edge, [&](int k) { return msg[k]; },
+        [&](int k, uint32_t, uint32_t, uint32_t m) { msg[k] = m; });
+}
+
+// Unrolled row R (degree at most 10) with compressed state st: s1p, d12,
+// minimum flags (bit k / 16 + k of edge k), signs (the same).
+template <int MODE, uint32_t ZT, int R>
+__device__ __forceinline__ void PackedRow(uint32_t *lam, const uint32_t *tab, uint32_t i4, uint32_t zh4, uint32_t *st,
+                                          uint32_t *inf_flag)
+{
+    constexpr int E0 = AIRAN_BG1_ROW_START[R], DEG = StaticDeg(R);
+    static_assert(DEG <= 16, "one bit per edge and check");
+    const uint32_t o1 = st[0], od = st[1], oe = st[2], os = st[3];
+    uint32_t ne = 0, ns = 0;
+    auto edge = [&](int k, uint32_t i4) {
+        if constexpr (ZT != 0)
+            return StaticEdge<ZT>(E0 + k, i4);
+        else
+            return TableEdge(tab[E0 + k], i4, zh4);
+    };
+    CheckRow<MODE, DEG>(
+        lam, i4, inf_flag, st[0], st[1], edge,
+        [&](int k) { return PkMadU16((oe >> k) & 0x00010001u, od, o1) ^ ((os << (15 - k)) & 0x80008000u); },
+        [&](int k, uint32_t x, uint32_t e, uint32_t) {
+            ne |= e << k;
+            ns |= (x >> (15 - k)) & (0x00010001u << k);
+        });
+    st[2] = ne;
+    st[3] = ns;
+}
+
+// A row of the loop: state s1p, d12 and meta (edge k: sign bit k, minimum
+// flag bit 8 + k, and 16 above for the other check).  w: its edge words.
+template <int MODE, int DEG>
+__device__ __forceinline__ void LoopRow(uint32_t *lam, const uint32_t *w, uint32_t i4, uint32_t zh4, uint32_t &s1p,
+                                        uint32_t &d12, uint32_t &meta, uint32_t *inf_flag)
+{
+    const uint32_t o1 = s1p, od = d12, om = meta;
+    uint32_t nm = 0;
+    CheckRow<MODE, DEG>(
+        lam, i4, inf_flag, s1p, d12, [&](int k, uint32_t i4) { return TableEdge(w[k], i4, zh4); },
+        [&](int k) { return PkMadU16((om >> (8 + k)) & 0x00010001u, od, o1) ^ ((om << (15 - k)) & 0x80008000u); },
+        [&](int k, uint32_t x, uint32_t e, uint32_t) {
+            nm |= e << (8 + k);
+            nm |= (x >> (15 - k)) & (0x00010001u << k);
+        });
+    meta = nm;
+}
+
+// The unrolled rows from R on, a barrier after each.
+template <int MODE, uint32_t ZT, bool FULL, int R>
+__device__ __forceinline__ void StaticRows(uint32_t *lam, const uint32_t *tab, uint32_t i4, uint32_t zh4, bool mine,
+                                           int rows, uint32_t *core, uint32_t *ext, uint32_t *inf_flag)
+{
+    if constexpr (R < kStaticRows) {
+        // Opaque per row: the addresses depend on the lane alone and would
+        // otherwise be hoisted out of the iteration, every row's at once.
+        asm volatile("" : "+v"(i4));
+        if (R < 4 || R < rows) {
+            if (mine) {
+                if constexpr (R < 4)
+                    FullRow<MODE, ZT, R>(lam, tab, i4, zh4, core + AIRAN_BG1_ROW_START[R], inf_flag);
+                else if constexpr (FULL)
+                    FullRow<MODE, ZT, R>(lam, tab, i4, zh4, ext + (AIRAN_BG1_ROW_START[R] - AIRAN_BG1_ROW_START[4]),
+                                         inf_flag);
+                else
+                    PackedRow<MODE, ZT, R>(lam, tab, i4, zh4, ext + 4 * (R - 4), inf_flag);
+            }
+            __syncthreads();
+        }
+        StaticRows<MODE, ZT, FULL, R + 1>(lam, tab, i4, zh4, mine, rows, core, ext, inf_flag);
+    }
+}
+
+// Words of N rows' state, indexed by the (uniform) row.
+template <int N>
+struct RowState {
+    typedef uint32_t vec __attribute__((ext_vector_type(N)));
+    vec s1p, d12, meta;
+};
+
+// Rows r0 .. r0 + count - 1 of the loop.
+template <int MODE, int N>
+__device__ __forceinline__ void LoopRows(uint32_t *lam, const uint32_t *tab, int r0, int count, bool mine, uint32_t i4,
+                                         uint32_t zh4, RowState<N> &st, uint32_t *inf_flag)
+{
+    if (count <= 0) return;
+    uint32_t info = kEdges.row[r0];
+    uint32_t w[kMaxLoopDeg];
+#pragma unroll
+    for (int k = 0; k < kMaxLoopDeg; ++k) w[k] = tab[(info & 0xffffu) + k];
+#pragma nounroll
+    for (int j = 0; j < count; ++j) {
+        // The next row's words, on their way while this row is worked on.
+        const uint32_t ninfo = kEdges.row[r0 + j + 1];
+        uint32_t nw[kMaxLoopDeg];
+        const uint32_t ne0 = (info & 0xffffu) + (info >> 16);
+#pragma unroll
+        for (int k = 0; k < kMaxLoopDeg; ++k) nw[k] = tab[ne0 + k];
+        if (mine) {
+            uint32_t a = st.s1p[j], b = st.d12[j], c = st.meta[j];
+            switch (info >> 16) {
+            case 4: LoopRow<MODE, 4>(lam, w, i4, zh4, a, b, c, inf_flag); break;
+            case 5: LoopRow<MODE, 5>(lam, w, i4, zh4, a, b, c, inf_flag); break;
+            case 6: LoopRow<MODE, 6>(lam, w, i4, zh4, a, b, c, inf_flag); break;
+            case 7: LoopRow<MODE, 7>(lam, w, i4, zh4, a, b, c, inf_flag); break;
+            default: LoopRow<MODE, 8>(lam, w, i4, zh4, a, b, c, inf_flag); break;
+            }
+            st.s1p[j] = a;
+            st.d12[j] = b;
+            st.meta[j] = c;
+        }
+        __syncthreads();
+        info = ninfo;
+#pragma unroll
+        for (int k = 0; k < kMaxLoopDeg; ++k) w[k] = nw[k];
+    }
+}
+
+// Hard decisions per half as 0 / 1.  FP16: NegBit (negative, non-zero, not
+// NaN).  REF: the reference's rint(clamp(v, +-5120)) < 0, which for an fp16
+// posterior is v < -0.5 (a NaN gives 0), bits 0xb801 .. 0xfc00.
+template <int MODE>
+__device__ __forceinline__ uint32_t HardBits2(uint32_t v)
+{
+    if constexpr (MODE == AIRAN_LDPC_MODE_REF)
+        return PkMinU16(PkSubSatU16(0x44004400u, PkSubU16(v, 0xb801b801u)), 0x00010001u);
+    return NegBit2(v);
+}
+
+// Bit 0 / 16 set where check i / i + Z/2 of one of the rows [r0, r1) fails.
+// FP16 without EXACT: the sign-bit XOR (no posterior is -0, and without an
+// infinite or NaN extrinsic none is a NaN; see PairSyndrome).
+template <int MODE, bool EXACT>
+__device__ __forceinline__ uint32_t TableSyndrome(uint32_t *lam, const uint32_t *tab, int r0, int r1, uint32_t i4,
+                                                  uint32_t zh4)
+{
+    uint32_t bad = 0;
+#pragma nounroll
+    for (int r = r0; r < r1; ++r) {
+        const uint32_t info = kEdges.row[r];
+        const int deg = static_cast<int>(info >> 16);
+        uint32_t p = 0;
+#pragma unroll 4
+        for (int k = 0; k < deg; ++k) {
+            const EdgeAt a = TableEdge(tab[(info & 0xffffu) + k], i4, zh4);
+            const uint32_t v = Rot16(LdsWord(lam, a.byte), a.rot);
+            p ^= EXACT || MODE == AIRAN_LDPC_MODE_REF ? HardBits2<MODE>(v) : (v >> 15);
+        }
+        bad |= p & 0x00010001u;
+    }
+    return bad;
+}
+
+template <int MODE, uint32_t ZT, int R, int RE>
+__device__ __forceinline__ uint32_t StaticSyndrome(uint32_t *lam, uint32_t i4)
+{
+    uint32_t bad = 0;
+    if constexpr (R < RE) {
+        uint32_t p = 0;
+        asm volatile("" : "+v"(i4));  // as in StaticRows
+#pragma unroll
+        for (int k = 0; k < StaticDeg(R); ++k) {
+            if (k > 0 && k % 7 == 0) __builtin_amdgcn_sched_barrier(0);
+            const EdgeAt a = StaticEdge<ZT>(AIRAN_BG1_ROW_START[R] + k, i4);
+            const uint32_t v = Rot16(LdsWord(lam, a.byte), a.rot);
+            p ^= MODE == AIRAN_LDPC_MODE_REF ? HardBits2<MODE>(v) << 15 : v;
+        }
+        bad = (p >> 15) & 0x00010001u;
+        return bad | StaticSyndrome<MODE, ZT, R + 1, RE>(lam, i4);
+    }
+    return bad;
+}
+
+struct LdpcDev {
+    uint32_t z, zi, k, iters, rows, early_stop;
+};
+
+// Posterior start value (fp16) of a decoder input LLR.
+template <int MODE>
+__device__ __forceinline__ uint32_t StartH(int32_t v)
+{
+    return MODE == AIRAN_LDPC_MODE_REF ? BitsH(static_cast<h16>(static_cast<float>(v))) : InputH(v);
+}
+
+// Half-word index in LDS of posterior position t.
+__device__ __forceinline__ uint32_t HalfIndex(uint32_t t, uint32_t z, uint32_t zh)
+{
+    const uint32_t col = t / z, q = t - col * z;
+    return q < zh ? 2u * (col * zh + q) : 2u * (col * zh + q - zh) + 1u;
+}
+
+// Loads a ragged block's posterior start values from its grant's bit-plane
+// codeword LLRs: positions below nl, word j of a column = positions j and
+// j + Z/2 (the rate-dematch arithmetic of ratematch.h).  Where every
+// transmitted bit lands on its own position (RateSingle), the planes are read
+// in aligned 16-byte chunks of 8 symbols and scattered (see PairLoad);
+// otherwise each position gathers its LLRs.  Ends before the barrier that
+// makes the posterior visible.
+__device__ inline void CheckLoadCodeword(uint32_t *lam, uint32_t z, uint32_t nl, const int16_t *__restrict__ cw,
+                                         const airan::RaggedCb &c, const airan::RaggedGrant &gr)
+{
+    const uint32_t i = threadIdx.x, nt = blockDim.x, zh = z / 2;
+    uint16_t *lam16 = reinterpret_cast<uint16_t *>(lam);
+    const airan::RateDev r{gr.g.qm, gr.g.cw_symbols, gr.g.cw_stride, z, c.kprime, c.filler, c.ncb, 1};
+    const airan::RateCb rc = airan::RateCbSetup({c.e, c.k0, c.ncb, c.cw_symbol_offset}, r);
+    const int16_t *src = cw + gr.cw_off;
+    if (!airan::RateSingle(rc, r)) {
+        for (uint32_t t = i; t < nl; t += nt)
+            lam16[HalfIndex(t, z, zh)] = static_cast<uint16_t>(InputH(airan::RateDematchValue(t, rc, r, src)));
+        return;
+    }
+    const uint32_t two_z = 2u * z, fstart = r.kprime - two_z, nf = r.ncb - r.filler;
+    const int16_t *slot = src + static_cast<size_t>(rc.slot0) * r.qm * r.cw_stride;
+    for (uint32_t t = i; t < nl / 2u; t += nt) lam[t] = 0;
+    __syncthreads();
+    for (uint32_t t = two_z + fstart + i; t < min(nl, two_z + fstart + r.filler); t += nt)
+        lam16[HalfIndex(t, z, zh)] = static_cast<uint16_t>(InputH(5120));
+    // Symbol j of plane b: its position.
+    auto position = [&](uint32_t b, uint32_t j) {
+        uint32_t q = rc.q0 + b * rc.eq + j;
+        q = q >= nf ? q - nf : q;
+        return two_z + (q < fstart ? q : q + r.filler);
+    };
+    auto put = [&](uint32_t b, uint32_t j, int32_t v) {
+        const uint32_t t = position(b, j);
+        if (t >= nl) return;
+        v *= 8;
+        v = v > 5120 ? 5120 : (v < -5120 ? -5120 : v);
+        lam16[HalfIndex(t, z, zh)] = static_cast<uint16_t>(InputH(v));
+    };
+    // Chunks of 8 symbols at multiples of 8 of the slot's planes, the block's
+    // symbols [rem0, rem0 + eq) of each plane inside them.
+    const uint32_t c0 = rc.rem0 / 8u, nc = (rc.rem0 + rc.eq + 7u) / 8u - c0;
+    for (uint32_t b = 0; b < r.qm; ++b) {
+        const int16_t *plane = slot + static_cast<size_t>(b) * r.cw_stride;
+        for (uint32_t e = i; e < nc; e += nt) {
+            const uint32_t s0 = 8u * (c0 + e);
+            const uint4 raw = *reinterpret_cast<const uint4 *>(plane + s0);
+            const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+            const uint32_t j0 = s0 - rc.rem0;  // below zero (wrapped) in a first partial chunk
+            const bool whole = s0 >= rc.rem0 && s0 + 8u <= rc.rem0 + rc.eq;
+            const uint32_t q = whole ? rc.q0 + b * rc.eq + j0 : 0u, qn = q >= nf ? q - nf : q;
+            const uint32_t t0 = two_z + (qn < fstart ? qn : qn + r.filler);
+            const uint32_t half = t0 / zh, q0 = t0 - half * zh;  // runs of Z/2: even ones are low halves
+            if (whole && qn + 8u <= nf && (qn >= fstart || qn + 8u <= fstart) && t0 + 8u <= nl && q0 + 8u <= zh) {
+                const h2_t scale = {static_cast<_Float16>(1.0f / 32.0f), static_cast<_Float16>(1.0f / 32.0f)};
+                uint16_t *dst = lam16 + 2u * ((half >> 1) * zh + q0) + (half & 1u);
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) {
+                    const uint32_t cl = PkMinI16(PkMaxI16(w[k], 0xfd80fd80u), 0x02800280u);
+                    const uint32_t vb = WH(__builtin_convertvector(__builtin_bit_cast(s16x2, cl), h2_t) * scale);
+                    dst[4u * k] = static_cast<uint16_t>(vb);
+                    dst[4u * k + 2u] = static_cast<uint16_t>(vb >> 16);
+                }
+            } else {
+#pragma unroll
+                for (uint32_t x = 0; x < 8; ++x) {
+                    const uint32_t sym = s0 + x;
+                    if (sym >= rc.rem0 && sym < rc.rem0 + rc.eq)
+                        put(b, sym - rc.rem0, static_cast<int16_t>(w[x >> 1] >> (16u * (x & 1u))));
+                }
+            }
+        }
+    }
+}
+
+constexpr uint32_t kCheckThreads = 192;
+
+// MAXROWS: kFewRows or kRows.  RAGGED: block b decodes code block list[b] of a
+// ragged batch, reading the grant's bit-plane codeword LLRs (src) itself (the
+// standalone rate-dematch arithmetic), with that block's Z, K and rows (no
+// lam_out); otherwise src holds the decoder LLRs [cb][68 Z].
+template <int MODE, int MAXROWS, uint32_t ZT, bool RAGGED>
+__global__ void __launch_bounds__(kCheckThreads) __attribute__((amdgpu_waves_per_eu(MAXROWS <= kFewRows ? 3 : 2)))
+    LdpcCheckPairKernel(const int16_t *__restrict__ src, int8_t *__restrict__ bits, int16_t *__restrict__ lam_out,
+                        uint8_t *__restrict__ iters_out, LdpcDev d, const airan::RaggedCb *__restrict__ cbs,
+                        const airan::RaggedGrant *__restrict__ grants, const uint32_t *__restrict__ list)
+{
+    constexpr bool kFull = MAXROWS <= kFewRows;  // every message of rows 4 .. 9 kept
+    constexpr int kCoreEdges = AIRAN_BG1_ROW_START[4];
+    constexpr int kExtEdges = AIRAN_BG1_ROW_START[kStaticRows] - kCoreEdges;
+    // The posterior, then the waves' syndrome votes (two words) and the flag
+    // of an infinite or NaN extrinsic (sticky: it only selects the exact
+    // syndrome).  One array, so that the posterior is at LDS address 0.
+    __shared__ __align__(16) uint32_t lam[(22 + MAXROWS) * 192 + 4];
+    uint32_t *vote = lam + (22 + MAXROWS) * 192, *inf_flag = vote + 2;
+    const uint32_t i = threadIdx.x;
+    uint32_t cb = blockIdx.x;
+    size_t bits_off;
+    if constexpr (RAGGED) {
+        cb = list[blockIdx.x];
+        const airan::RaggedCb &c = cbs[cb];
+        d.z = c.z;
+        d.k = c.k;
+        d.rows = c.rows;
+        d.zi = 0;
+        while ((24u << d.zi) < d.z) ++d.zi;
+        bits_off = c.bits_off;
+    } else {
+        bits_off = static_cast<size_t>(cb) * d.k;
+    }
+    const uint32_t Z = ZT != 0 ? ZT : d.z, zh = Z / 2, zh4 = 2u * Z;
+    const int rows = static_cast<int>(d.rows);
+    const uint32_t nl = (22u + d.rows) * Z;  // positions the active rows touch
+    uint16_t *lam16 = reinterpret_cast<uint16_t *>(lam);
+    if (i < 3) vote[i] = 0;
+    if constexpr (RAGGED) {
+        CheckLoadCodeword(lam, Z, nl, src, cbs[cb], grants[cbs[cb].grant]);
+    } else {
+        const int16_t *s = src + static_cast<size_t>(cb) * 68u * Z;
+        if ((reinterpret_cast<uintptr_t>(src) & 7u) == 0) {
+            // Four words at a time: positions j .. j + 3 and their partners
+            // (Z is a multiple of 24: runs of 4 never cross a half).
+            const uint32_t per = zh / 4u, total = (22u + d.rows) * per;
+            for (uint32_t t = i; t < total; t += kCheckThreads) {
+                const uint32_t col = t / per, j = 4u * (t - col * per);
+                const uint2 a = *reinterpret_cast<const uint2 *>(s + col * Z + j);
+                const uint2 b = *reinterpret_cast<const uint2 *>(s + col * Z + zh + j);
+                auto word = [&](uint32_t x, uint32_t y, uint32_t sh) {
+                    return StartH<MODE>(static_cast<int16_t>(x >> sh)) | StartH<MODE>(static_cast<int16_t>(y >> sh)) << 16;
+                };
+                *reinterpret_cast<uint4 *>(lam + col * zh + j) =
+                    make_uint4(word(a.x, b.x, 0), word(a.x, b.x, 16), word(a.y, b.y, 0), word(a.y, b.y, 16));
+            }
+        } else {
+            for (uint32_t t = i; t < nl; t += kCheckThreads)
+                lam16[HalfIndex(t, Z, zh)] = static_cast<uint16_t>(StartH<MODE>(s[t]));
+        }
+    }
+    const uint32_t *tab = kEdges.w[d.zi];
+    uint32_t core[kCoreEdges];
+#pragma unroll
+    for (int e = 0; e < kCoreEdges; ++e) core[e] = 0;
+    uint32_t ext[kFull ? kExtEdges : 4 * (kStaticRows - 4)];
+#pragma unroll
+    for (uint32_t &v : ext) v = 0;
+    RowState<32> sa;  // rows kStaticRows .. + 31
+    RowState<4> sb;   // and the last four
+    static_assert(kStaticRows + 32 + 4 == kRows, "row states");
+    sa.s1p = sa.d12 = sa.meta = 0;
+    sb.s1p = sb.d12 = sb.meta = 0;
+    __syncthreads();
+    const bool mine = i < zh;
+    uint32_t it = 0;
+    while (it < d.iters) {
+        uint32_t i4 = 4u * i;
+        StaticRows<MODE, ZT, kFull, 0>(lam, tab, i4, zh4, mine, rows, core, ext, inf_flag);
+        if constexpr (MAXROWS > kStaticRows) {
+            LoopRows<MODE, 32>(lam, tab, kStaticRows, min(rows - kStaticRows, 32), mine, i4, zh4, sa, inf_flag);
+            LoopRows<MODE, 4>(lam, tab, kStaticRows + 32, rows - kStaticRows - 32, mine, i4, zh4, sb, inf_flag);
+        }
+        ++it;
+        if (d.early_stop) {
+            // The core rows first: a block that has not converged nearly
+            // always fails one of them.  Votes: a failing wave sets the word;
+            // it is cleared below, before the barriers of the next iteration.
+            const bool exact = MODE == AIRAN_LDPC_MODE_FP16 && *inf_flag != 0;
+            uint32_t bad = 0;
+            if (mine && !exact) {
+                if constexpr (ZT != 0)
+                    bad = StaticSyndrome<MODE, ZT, 0, 4>(lam, i4);
+                else
+                    bad = TableSyndrome<MODE, false>(lam, tab, 0, 4, i4, zh4);
+            } else if (mine) {
+                bad = TableSyndrome<MODE, true>(lam, tab, 0, 4, i4, zh4);
+            }
+            if (__ballot(bad != 0) != 0 && (i & 63u) == 0) vote[0] = 1u;
+            __syncthreads();
+            bool ok = vote[0] == 0;
+            if (ok) {
+                bad = 0;
+                if (mine && !exact) {
+                    if constexpr (ZT != 0 && MAXROWS <= kFewRows) {
+                        // Unrolled up to the few rows; a row beyond the
+                        // block's is not read (its column is not loaded).
+                        if (rows > 4) bad |= StaticSyndrome<MODE, ZT, 4, 5>(lam, i4);
+                        if (rows > 5) bad |= StaticSyndrome<MODE, ZT, 5, 6>(lam, i4);
+                        if (rows > 6) bad |= StaticSyndrome<MODE, ZT, 6, 7>(lam, i4);
+                        if (rows > 7) bad |= StaticSyndrome<MODE, ZT, 7, 8>(lam, i4);
+                        if (rows > 8) bad |= StaticSyndrome<MODE, ZT, 8, 9>(lam, i4);
+                        if (rows > 9) bad |= StaticSyndrome<MODE, ZT, 9, 10>(lam, i4);
+                    } else {
+                        bad = TableSyndrome<MODE, false>(lam, tab, 4, rows, i4, zh4);
+                    }
+                } else if (mine) {
+                    bad = TableSyndrome<MODE, true>(lam, tab, 4, rows, i4, zh4);
+                }
+                if (__ballot(bad != 0) != 0 && (i & 63u) == 0) vote[1] = 1u;
+                __syncthreads();
+                ok = vote[1] == 0;
+            }
+            if (ok) break;
+            __syncthreads();
+            if (i < 2) vote[i] = 0;
+        }
+    }
+    // (every posterior is final: the last row and the votes ended in barriers)
+    if (iters_out != nullptr && i == 0) iters_out[cb] = static_cast<uint8_t>(it);
+    int8_t *bo = bits + bits_off;
+    if ((d.k & 3u) == 0 && (reinterpret_cast<uintptr_t>(bo) & 3u) == 0) {
+        for (uint32_t t = 4u * i; t < d.k; t += 4u * kCheckThreads) {
+            const uint32_t h = HalfIndex(t, Z, zh), sh = h & 1u;
+            const uint4 v = *reinterpret_cast<const uint4 *>(lam + h / 2u);
+            auto bit = [&](uint32_t x) { return (HardBits2<MODE>(x) >> (16u * sh)) & 1u; };
+            *reinterpret_cast<uint32_t *>(bo + t) = bit(v.x) | bit(v.y) << 8 | bit(v.z) << 16 | bit(v.w) << 24;
+        }
+    } else {
+        for (uint32_t t = i; t < d.k; t += kCheckThreads)
+            bo[t] = static_cast<int8_t>(HardBits2<MODE>(lam16[HalfIndex(t, Z, zh)]) & 1u);
+    }
+    if (!RAGGED && lam_out != nullptr) {
+        const int16_t *s = src + static_cast<size_t>(cb) * 68u * Z;
+        int16_t *lo = lam_out + static_cast<size_t>(cb) * 68u * Z;
+        const float clip = MODE == AIRAN_LDPC_MODE_REF ? 5120.0f : 20.0f;
+        const float out_scale = MODE == AIRAN_LDPC_MODE_REF ? 1.0f : 256.0f;
+        for (uint32_t t = i; t < 68u * Z; t += kCheckThreads) {
+            // Columns beyond the active rows keep their input.
+            const uint32_t h = t < nl ? lam16[HalfIndex(t, Z, zh)] : StartH<MODE>(s[t]);
+            float v = static_cast<float>(HBits(h));
+            v = v > clip ? clip : (v < -clip ? -clip : v);
+            lo[t] = static_cast<int16_t>(rintf(v * out_scale));
+        }
+    }
+}
+
 // Workgroups resident on the device at once for a pair-decoder launch shape
 // (0 when the runtime cannot tell).
 uint32_t PairCapacity(const void *kernel, uint32_t threads, size_t lds)
@@ -965,6 +1344,49 @@ uint32_t LiftIndex(uint32_t z)
     return zi;
 }
 
+template <int MODE>
+void LaunchCheckPair(const LdpcDecodeOpArgsV1 *a, hipStream_t s)
+{
+    const LdpcDev d{a->z, LiftIndex(a->z), a->k, a->max_iterations, a->active_rows, a->early_stop ? 1u : 0u};
+    const bool few = a->active_rows <= static_cast<uint32_t>(kFewRows), z384 = a->z == 384;
+    using Kern = void (*)(const int16_t *, int8_t *, int16_t *, uint8_t *, LdpcDev, const airan::RaggedCb *,
+                          const airan::RaggedGrant *, const uint32_t *);
+    const Kern k = few ? (z384 ? LdpcCheckPairKernel<MODE, kFewRows, 384, false> : LdpcCheckPairKernel<MODE, kFewRows, 0, false>)
+                       : (z384 ? LdpcCheckPairKernel<MODE, kRows, 384, false> : LdpcCheckPairKernel<MODE, kRows, 0, false>);
+    hipLaunchKernelGGL(k, dim3(a->num_cb), dim3(kCheckThreads), 0, s, static_cast<const int16_t *>(a->lam_in),
+                       static_cast<int8_t *>(a->bits), static_cast<int16_t *>(a->lam_out),
+                       static_cast<uint8_t *>(a->iterations_out), d, nullptr, nullptr, nullptr);
+}
+
+// The decoder operator (validated arguments).
+int32_t LaunchDecode(const LdpcDecodeOpArgsV1 *a)
+{
+    int32_t st;
+    hipStream_t s = static_cast<hipStream_t>(a->stream);
+    const auto *in = static_cast<const int16_t *>(a->lam_in);
+    auto *bits = static_cast<int8_t *>(a->bits);
+    const bool aligned = (reinterpret_cast<uintptr_t>(in) & 7u) == 0 && (reinterpret_cast<uintptr_t>(bits) & 3u) == 0;
+    if (aligned && FastEligible(a->mode, a->z, a->active_rows)) {
+        if ((st = LoadLiftTable()) != AIRAN_OK) return st;
+        const uint32_t rows = a->active_rows;  // validated >= 4
+        LdpcFastDev fd{a->z, LiftIndex(a->z), a->k, a->max_iterations, rows, a->early_stop ? 1u : 0u, a->num_cb, {}};
+        const size_t fast_lds = static_cast<size_t>(22 + rows) * a->z * sizeof(uint32_t);
+        LaunchPair<false>(rows, airan::AlignUp(a->z, 64), fast_lds, s, in, nullptr, bits,
+                          static_cast<int16_t *>(a->lam_out), static_cast<uint8_t *>(a->iterations_out), fd, nullptr);
+        return airan::LaunchStatus();
+    }
+    if ((st = LoadEdgeTable()) != AIRAN_OK) return st;
+    if (a->mode == AIRAN_LDPC_MODE_FP16)
+        LaunchCheckPair<AIRAN_LDPC_MODE_FP16>(a, s);
+    else
+        LaunchCheckPair<AIRAN_LDPC_MODE_REF>(a, s);
+    return airan::LaunchStatus();
+}
+
+// Largest workspace that airan_ldpc_decode_EnqueueNoAlloc stands in for (the
+// reference's 143-block transport block at 46 rows, Z = 384: 20.2 MB).
+constexpr size_t kNoAllocMaxBytes = size_t{32} << 20;
+
 }  // namespace
 
 extern "C" {
@@ -986,109 +1408,66 @@ int32_t airan_ldpc_decode_ValidateOpArgs(const LdpcDecodeOpArgsV1 *a)
     return AIRAN_OK;
 }
 
+// The caller's part of the contract: a workspace of 8 bytes per (block, row,
+// check) above kFastRows rows.  The decoder keeps its message state in
+// registers and does not touch it.
 size_t airan_ldpc_decode_WorkspaceBytes(uint32_t num_cb, uint32_t z, uint32_t active_rows)
 {
-    if (active_rows <= static_cast<uint32_t>(kRegRows)) return 0;
+    if (active_rows <= static_cast<uint32_t>(kFastRows)) return 0;
     return static_cast<size_t>(num_cb) * active_rows * z * sizeof(uint2);
 }
 
-size_t airan_ldpc_decode_NoAllocMaxWorkspaceBytes(void) { return kNoAllocScratchBytes; }
+size_t airan_ldpc_decode_NoAllocMaxWorkspaceBytes(void) { return kNoAllocMaxBytes; }
 
 int32_t airan_ldpc_decode_EnqueueNoAlloc(const LdpcDecodeOpArgsV1 *a)
 {
-    int32_t st = airan_ldpc_decode_ValidateOpArgs(a);
+    const int32_t st = airan_ldpc_decode_ValidateOpArgs(a);
     if (st != AIRAN_OK) return st;
-    const size_t need = airan_ldpc_decode_WorkspaceBytes(a->num_cb, a->z, a->active_rows);
-    if (need > kNoAllocScratchBytes) return AIRAN_RESOURCE_TOO_SMALL;
-    if (need == 0) return airan_ldpc_decode_Enqueue(a, nullptr, 0);
-    if ((st = airan_InitDevice()) != AIRAN_OK) return st;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return AIRAN_LAUNCH_FAILED;
-    void *ws = nullptr;
-    {
-        std::lock_guard<std::mutex> lock(g_table_mutex);
-        ws = g_scratch_ptr[dev];
-    }
-    if (ws == nullptr) return AIRAN_LAUNCH_FAILED;
-    return airan_ldpc_decode_Enqueue(a, ws, need);
+    if (airan_ldpc_decode_WorkspaceBytes(a->num_cb, a->z, a->active_rows) > kNoAllocMaxBytes)
+        return AIRAN_RESOURCE_TOO_SMALL;
+    return LaunchDecode(a);
 }
 
 int32_t airan_ldpc_decode_Enqueue(const LdpcDecodeOpArgsV1 *a, void *workspace, size_t workspace_bytes)
 {
-    int32_t st = airan_ldpc_decode_ValidateOpArgs(a);
+    const int32_t st = airan_ldpc_decode_ValidateOpArgs(a);
     if (st != AIRAN_OK) return st;
-    if ((st = LoadTable()) != AIRAN_OK) return st;
     const size_t need = airan_ldpc_decode_WorkspaceBytes(a->num_cb, a->z, a->active_rows);
     if (need > 0 && (workspace == nullptr || workspace_bytes < need)) return AIRAN_RESOURCE_TOO_SMALL;
-    LdpcDev d{a->z, a->k, a->max_iterations, a->active_rows, a->early_stop ? 1u : 0u};
-    const uint32_t threads = airan::AlignUp(a->z, 64);
-    const size_t lds = static_cast<size_t>(68) * a->z * sizeof(uint16_t);
-    hipStream_t s = static_cast<hipStream_t>(a->stream);
-    const auto *in = static_cast<const int16_t *>(a->lam_in);
-    auto *bits = static_cast<int8_t *>(a->bits);
-    auto *lo = static_cast<int16_t *>(a->lam_out);
-    auto *io = static_cast<uint8_t *>(a->iterations_out);
-    auto *ws = static_cast<uint2 *>(workspace);
-    const bool aligned = (reinterpret_cast<uintptr_t>(in) & 7u) == 0 && (reinterpret_cast<uintptr_t>(bits) & 3u) == 0;
-    if (aligned && FastEligible(a->mode, a->z, a->active_rows)) {
-        if ((st = LoadLiftTable()) != AIRAN_OK) return st;
-        const uint32_t rows = a->active_rows;  // validated >= 4
-        LdpcFastDev fd{a->z, LiftIndex(a->z), a->k, a->max_iterations, rows, a->early_stop ? 1u : 0u, a->num_cb, {}};
-        const size_t fast_lds = static_cast<size_t>(22 + rows) * a->z * sizeof(uint32_t);
-        LaunchPair<false>(rows, threads, fast_lds, s, in, nullptr, bits, lo, io, fd, nullptr);
-        return airan::LaunchStatus();
-    }
-    const bool reg = a->active_rows <= static_cast<uint32_t>(kRegRows);
-    if (a->mode == AIRAN_LDPC_MODE_FP16) {
-        if (reg)
-            hipLaunchKernelGGL((LdpcKernel<AIRAN_LDPC_MODE_FP16, kRegRows>), dim3(a->num_cb), dim3(threads), lds, s, in, bits, lo, io, ws, d);
-        else
-            hipLaunchKernelGGL((LdpcKernel<AIRAN_LDPC_MODE_FP16, 0>), dim3(a->num_cb), dim3(threads), lds, s, in, bits, lo, io, ws, d);
-    } else {
-        if (reg)
-            hipLaunchKernelGGL((LdpcKernel<AIRAN_LDPC_MODE_REF, kRegRows>), dim3(a->num_cb), dim3(threads), lds, s, in, bits, lo, io, ws, d);
-        else
-            hipLaunchKernelGGL((LdpcKernel<AIRAN_LDPC_MODE_REF, 0>), dim3(a->num_cb), dim3(threads), lds, s, in, bits, lo, io, ws, d);
-    }
-    return airan::LaunchStatus();
+    return LaunchDecode(a);
 }
 
 }  // extern "C"
 
 namespace airan {
 
-int32_t LaunchLdpcRagged(const RaggedCb *cbs, const uint32_t *reg_list, uint32_t n_reg, const uint32_t *ws_list,
-                         uint32_t n_ws, uint32_t iters, bool early_stop, const int16_t *lam, int8_t *bits,
-                         uint8_t *iters_out, uint2 *ws, hipStream_t s)
+int32_t LaunchLdpcRagged(const RaggedCb *cbs, const RaggedGrant *grants, const RaggedLdpcList &many,
+                         const RaggedLdpcList &few, const RaggedLdpcList &other, uint32_t iters, bool early_stop,
+                         const int16_t *cw, int8_t *bits, uint8_t *iters_out, hipStream_t s)
 {
-    int32_t st = LoadTable();
+    const int32_t st = LoadEdgeTable();
     if (st != AIRAN_OK) return st;
-    const LdpcDev d{0, 0, iters, 0, early_stop ? 1u : 0u};
-    const size_t lds = static_cast<size_t>(68) * 384 * sizeof(uint16_t);
-    if (n_reg > 0)
-        hipLaunchKernelGGL((LdpcKernel<AIRAN_LDPC_MODE_FP16, kRegRows, true>), dim3(n_reg), dim3(384), lds, s, lam,
-                           bits, nullptr, iters_out, nullptr, d, cbs, reg_list);
-    if (n_ws > 0)
-        hipLaunchKernelGGL((LdpcKernel<AIRAN_LDPC_MODE_FP16, 0, true>), dim3(n_ws), dim3(384), lds, s, lam, bits,
-                           nullptr, iters_out, ws, d, cbs, ws_list);
+    const LdpcDev d{0, LiftIndex(384), 0, iters, 0, early_stop ? 1u : 0u};
+    constexpr int kMode = AIRAN_LDPC_MODE_FP16;
+    auto launch = [&](auto kernel, const RaggedLdpcList &l) {
+        if (l.count > 0)
+            hipLaunchKernelGGL(kernel, dim3(l.count), dim3(kCheckThreads), 0, s, cw, bits, nullptr, iters_out, d, cbs,
+                               grants, l.list);
+    };
+    launch(LdpcCheckPairKernel<kMode, kRows, 384, true>, many);
+    launch(LdpcCheckPairKernel<kMode, kFewRows, 384, true>, few);
+    launch(LdpcCheckPairKernel<kMode, kRows, 0, true>, other);
     return LaunchStatus();
 }
 
-int32_t InitLdpcScratch()
+uint32_t LdpcFewRows() { return kFewRows; }
+
+int32_t InitLdpcTables()
 {
-    // The decoder's constant tables too, so that a caller who ran
-    // airan_InitDevice launches nothing but the decoder afterwards.
-    int32_t st = LoadTable();
-    if (st == AIRAN_OK) st = LoadLiftTable();
-    if (st != AIRAN_OK) return st;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return AIRAN_LAUNCH_FAILED;
-    std::lock_guard<std::mutex> lock(g_table_mutex);
-    if (g_scratch_ptr[dev] != nullptr) return AIRAN_OK;
-    void *p = nullptr;
-    if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || p == nullptr) return AIRAN_LAUNCH_FAILED;
-    g_scratch_ptr[dev] = p;
-    return AIRAN_OK;
+    // So that a caller who ran airan_InitDevice launches nothing but the
+    // decoder afterwards.
+    const int32_t st = LoadLiftTable();
+    return st == AIRAN_OK ? LoadEdgeTable() : st;
 }
 
 int32_t LaunchLdpcFromCodeword(const Geom &g, const AiranTbPlanV1 &p, const RateMatchDescriptor *desc,

@@ -50,9 +50,7 @@ struct RaggedCb {
     uint32_t grant;
     uint32_t e, k0, ncb, cw_symbol_offset;  // rate matching (within the grant's codeword)
     uint32_t z, kprime, filler, k, rows;    // decoder
-    uint64_t lam_off;                       // int16 [68 z]
     uint64_t bits_off;                      // int8 [k]
-    uint64_t ws_off;                        // decoder message state (uint2), rows > 8
     uint32_t crc_cb, len_tb, poly_tb, xpow; // CRC24B length (0 / 24), TB CRC and this block's shift
 };
 

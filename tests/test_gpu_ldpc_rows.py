@@ -1,0 +1,68 @@
+"""The decoder kernel of one code block per workgroup (REF mode, more than 8
+active rows, unaligned buffers) bit for bit against the oracle where it can go
+wrong: every lifting size (the halves of 12 .. 192 words), the row counts at
+which its unrolled rows, its two register arrays and its kernels end, buffers
+of any alignment, a K that is no multiple of 4, and int16 inputs large enough
+for REF mode's growing posteriors to reach infinity and NaN."""
+import numpy as np
+import pytest
+
+from oracle_lib import load_oracle, ptr
+from puschrx import abi, ops
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+def _check(lam, n, z, k, iters, rows, mode, early, offset=0, want_lam=True):
+    oracle = load_oracle()
+    ref = lam.copy()
+    bits, it = np.zeros(n * k, np.int8), np.zeros(n, np.uint8)
+    oracle.or_ldpc_decode(z, n, ptr(ref), mode, iters, rows, k, 1 if early else 0, ptr(bits), ptr(it))
+    dev = torch.zeros(lam.size + offset, dtype=torch.int16, device="cuda")
+    dev[offset:] = torch.from_numpy(lam).cuda()
+    got, lam_out, git = ops.ldpc_decode(dev[offset:], n, z, k, iters, rows, mode, early, want_lam=want_lam)
+    torch.cuda.synchronize()
+    assert np.array_equal(git.cpu().numpy(), it)
+    assert np.array_equal(got.cpu().numpy(), bits)
+    if want_lam:
+        assert np.array_equal(lam_out.cpu().numpy(), ref)
+
+
+def _llrs(z, n, rows, ebno, seed):
+    oracle, rng = load_oracle(), np.random.default_rng(seed)
+    out = np.zeros((n, 68 * z), np.int16)
+    var = 1.0 / (2.0 * 22 / (20 + rows) * 10 ** (0.1 * ebno))
+    for row in out:
+        info, cw = rng.integers(0, 2, 22 * z, dtype=np.uint8), np.zeros(68 * z, np.uint8)
+        oracle.or_ldpc_encode(z, ptr(info), ptr(cw))
+        y = 1.0 - 2.0 * cw + rng.normal(0, np.sqrt(var), cw.size)
+        row[:] = np.clip(np.rint(2 * y / var * 256), -5120, 5120)
+        row[: 2 * z] = 0
+        row[(22 + rows) * z:] = 0
+    return out.reshape(-1)
+
+
+@pytest.mark.parametrize("mode", [abi.LDPC_MODE_REF, abi.LDPC_MODE_FP16])
+@pytest.mark.parametrize("z,rows", [(24, 46), (48, 12), (96, 9), (192, 43), (384, 4), (384, 9), (384, 10), (384, 11),
+                                    (384, 41), (384, 42), (384, 43)])
+def test_rows_and_lifting_sizes(gpu_stream, mode, z, rows):
+    for early, ebno in ((True, 3.0), (False, 1.0)):
+        _check(_llrs(z, 5, rows, ebno, z + rows), 5, z, 22 * z, 6, rows, mode, early)
+
+
+@pytest.mark.parametrize("offset", [1, 2])
+@pytest.mark.parametrize("rows", [6, 17])
+def test_alignment_and_odd_k(gpu_stream, offset, rows):
+    z = 384
+    _check(_llrs(z, 3, rows, 3.0, 5), 3, z, 22 * z - 3, 5, rows, abi.LDPC_MODE_FP16, True, offset=offset)
+
+
+@pytest.mark.parametrize("mode", [abi.LDPC_MODE_REF, abi.LDPC_MODE_FP16])
+@pytest.mark.parametrize("rows", [9, 46])
+def test_full_range_inputs(gpu_stream, mode, rows):
+    """Bits and iterations only: the clamped posterior of a NaN is no number."""
+    rng = np.random.default_rng(rows)
+    lam = rng.integers(-32768, 32768, (4, 68 * 96)).astype(np.int16)
+    lam[3] = np.where(rng.integers(0, 2, 68 * 96), 32767, -32768)
+    _check(lam.reshape(-1), 4, 96, 22 * 96, 20, rows, mode, True, want_lam=False)
