@@ -350,6 +350,20 @@ void DropGraph(AiranPuschChain *c)
     c->graph_stream = nullptr;
 }
 
+// CRC of every code block and transport block (plans with CRCs), with the
+// tables and block shifts that Create built.
+int32_t EnqueueCrc(AiranPuschChain *c, uint32_t tbs, hipStream_t s)
+{
+    if (!c->crc) return AIRAN_OK;
+    airan::CrcJob crc{};
+    const int32_t st = airan::CrcJobSetup(c->plan, c->cb_ok, reinterpret_cast<uint32_t *>(c->crc_ws), &crc);
+    if (st != AIRAN_OK) return st;
+    crc.xpow = c->crc_xpow;
+    airan::LaunchCbCrc(c->bits, crc, c->plan.K, tbs * c->plan.C, CrcTables(c), s);
+    airan::LaunchCrcFinish(reinterpret_cast<const uint32_t *>(c->crc_ws), c->tb_ok, tbs, c->plan.C, s);
+    return airan::LaunchStatus();
+}
+
 int32_t EnqueueStages(AiranPuschChain *c, const void *iq, const uint16_t *slot_no, uint32_t slots, hipStream_t s,
                       bool timed)
 {
@@ -419,16 +433,7 @@ int32_t EnqueueStages(AiranPuschChain *c, const void *iq, const uint16_t *slot_n
                                            c->opts.early_stop != 0, c->bits, c->iters, c->ldpc_queue, s);
         if (st != AIRAN_OK) return st;
         mark();
-        if (c->crc) {
-            airan::CrcJob crc{};
-            if ((st = airan::CrcJobSetup(c->plan, c->cb_ok, reinterpret_cast<uint32_t *>(c->crc_ws), &crc)) !=
-                AIRAN_OK)
-                return st;
-            crc.xpow = c->crc_xpow;
-            airan::LaunchCbCrc(c->bits, crc, c->plan.K, ncb, CrcTables(c), s);
-            airan::LaunchCrcFinish(reinterpret_cast<const uint32_t *>(c->crc_ws), c->tb_ok, tbs, c->plan.C, s);
-            if ((st = airan::LaunchStatus()) != AIRAN_OK) return st;
-        }
+        if ((st = EnqueueCrc(c, tbs, s)) != AIRAN_OK) return st;
         mark();
         return AIRAN_OK;
     }
@@ -452,11 +457,7 @@ int32_t EnqueueStages(AiranPuschChain *c, const void *iq, const uint16_t *slot_n
     st = airan_ldpc_decode_Enqueue(&la, c->ldpc_ws, c->ldpc_ws_bytes);
     if (st != AIRAN_OK) return st;
     mark();
-    if (c->crc) {
-        st = airan_crc_check_Enqueue(&c->plan, tbs, c->bits, c->cb_ok, c->tb_ok, nullptr, c->crc_ws,
-                                     c->crc_ws_bytes, s);
-        if (st != AIRAN_OK) return st;
-    }
+    if ((st = EnqueueCrc(c, tbs, s)) != AIRAN_OK) return st;
     mark();
     return AIRAN_OK;
 }
@@ -564,7 +565,7 @@ int32_t airan_pusch_chain_Create(const PuschMimoConfig *config, const AiranTbPla
         // The CRC check's tables, after the TB remainder parts in crc_ws.
         airan::CrcJob job{};
         if ((st = airan::CrcJobSetup(p, nullptr, nullptr, &job)) != AIRAN_OK) return fail(st);
-        airan::LaunchCrcTables(job, p.K, CrcTables(c), nullptr);
+        airan::LaunchCrcTables(job, p.K, static_cast<uint32_t>(ncb), CrcTables(c), nullptr);
         if (hipDeviceSynchronize() != hipSuccess || airan::LaunchStatus() != AIRAN_OK)
             return fail(AIRAN_LAUNCH_FAILED);
     }

@@ -88,16 +88,8 @@ struct CrcDev {
     uint32_t poly_tb, len_tb;
 };
 
-__global__ void __launch_bounds__(256) ZeroKernel(uint32_t *p, uint32_t n)
-{
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) p[t] = 0;
-}
-
-constexpr uint32_t kCrcW = 24;           // bits per thread and block
-constexpr uint32_t kCrcThreads = 384;     // 24 * 384 >= 8448, the largest K
-constexpr uint32_t kCrcMaxLen = 24;
-static_assert(airan::kCrcTableBytes >= 2 * kCrcMaxLen * kCrcThreads * sizeof(uint32_t), "mask table size");
+// ------------------------------------------------------- one block per group
+constexpr uint32_t kChunkThreads = 320;  // 32 positions each: 10240 >= 8448, the largest K
 
 // The four 0/1 bytes of w as 4 bits, the first byte highest.
 __device__ inline uint32_t Pack4(uint32_t w)
@@ -105,134 +97,79 @@ __device__ inline uint32_t Pack4(uint32_t w)
     return (((w & 0x01010101u) * 0x08040201u) >> 24) & 0xfu;
 }
 
-// Masks of one CRC for positions [w0, w0 + 24) of an n-bit message;
-// pw[e] = x^(len + e) mod g.  Positions >= n get no bits.
-__device__ inline void CrcMasks(const uint32_t *pw, uint32_t poly, uint32_t len, uint32_t n, uint32_t w0,
-                                uint32_t (&m)[kCrcMaxLen])
+// v(x) p(x) mod g for the 32-bit polynomial v and a residue p, by Horner's
+// rule with the residues left-aligned (the top bit is the sign bit).
+__device__ inline uint32_t CrcMul32(uint32_t v, uint32_t p, uint32_t poly, uint32_t len)
 {
+    const uint32_t sh = 32u - len, pl = p << sh, gl = poly << sh;
+    int32_t r = 0;
 #pragma unroll
-    for (uint32_t k = 0; k < kCrcMaxLen; ++k) m[k] = 0;
-    if (w0 >= n) return;
-    const uint32_t last = min(n - w0, kCrcW) - 1;  // last position that counts
-    uint32_t p = pw[n - 1 - (w0 + last)];          // its term; earlier ones are times x
-    const uint32_t top = 1u << (len - 1), mask = (top << 1) - 1u;
-#pragma unroll
-    for (int jj = kCrcW - 1; jj >= 0; --jj) {
-        if (static_cast<uint32_t>(jj) > last) continue;
-#pragma unroll
-        for (uint32_t k = 0; k < kCrcMaxLen; ++k) m[k] |= ((p >> k) & 1u) << (kCrcW - 1 - jj);
-        p = ((p << 1) & mask) ^ ((p & top) ? poly : 0u);
+    for (int i = 31; i >= 0; --i) {
+        const uint32_t top = static_cast<uint32_t>(r >> 31) & gl;
+        const uint32_t bit = static_cast<uint32_t>(static_cast<int32_t>(v << (31 - i)) >> 31) & pl;
+        r = static_cast<int32_t>((static_cast<uint32_t>(r) << 1) ^ top ^ bit);
     }
+    return static_cast<uint32_t>(r) >> sh;
 }
 
-// Remainder share of the 24 bits v (first position highest) under masks m.
-__device__ inline uint32_t CrcApply(uint32_t v, const uint32_t (&m)[kCrcMaxLen])
+// Remainders of one block by a workgroup of kChunkThreads: rb of its first nb
+// bits (CRC24B), ra of its first na (the TB CRC).  Thread t takes positions
+// [32 t, 32 t + 32): their bits as a polynomial times x^(len + bits after
+// them), tabulated in pow_*.  The result is valid in thread 0.
+__device__ inline void CrcBlockRemainders(const int8_t *__restrict__ b, uint32_t K, uint32_t nb, uint32_t na,
+                                          const uint32_t *__restrict__ pow_b, const uint32_t *__restrict__ pow_tb,
+                                          uint32_t poly_tb, uint32_t len_tb, uint32_t *rb_out, uint32_t *ra_out)
 {
-    uint32_t r = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < kCrcMaxLen; ++k) r |= (__popc(v & m[k]) & 1u) << k;
-    return r;
-}
-
-// The masks of both CRCs for every thread slot: masks[k][t] (CRC24B rows
-// k < 24, then the TB CRC's), built once per plan.
-__global__ void __launch_bounds__(kCrcThreads) CrcMaskKernel(airan::CrcJob c, uint32_t *__restrict__ masks)
-{
-    const uint32_t t = threadIdx.x, w0 = kCrcW * t;
-    uint32_t mb[kCrcMaxLen], ma[kCrcMaxLen];
-    CrcMasks(c.pow_b, airan::kCrcPolyB, 24, c.crc_cb ? c.kprime : 0u, w0, mb);
-    CrcMasks(c.pow_tb, c.poly_tb, c.len_tb, c.L, w0, ma);
-#pragma unroll
-    for (uint32_t k = 0; k < kCrcMaxLen; ++k) {
-        masks[k * kCrcThreads + t] = mb[k];
-        masks[(kCrcMaxLen + k) * kCrcThreads + t] = ma[k];
-    }
-}
-
-constexpr uint32_t kCrcBatch = 4;  // blocks a workgroup checks together
-
-// bits: int8 0/1 per bit, [cb][K].  Persistent: workgroup b checks blocks
-// kCrcBatch at a time (b kCrcBatch, ..., then G kCrcBatch further on) with
-// kCrcThreads threads, thread t owning positions [24 t, 24 t + 24) and
-// holding their masks (CrcMaskKernel) in registers; the batch's loads are in
-// flight together and threads 0 .. kCrcBatch - 1 finish its blocks.
-__global__ void __launch_bounds__(kCrcThreads) CbCrcKernel(const int8_t *__restrict__ bits, airan::CrcJob c,
-                                                          uint32_t K, uint32_t num_cb,
-                                                          const uint32_t *__restrict__ masks)
-{
-    const uint32_t t = threadIdx.x, w0 = kCrcW * t;
-    uint32_t mb[kCrcMaxLen], ma[kCrcMaxLen];
-#pragma unroll
-    for (uint32_t k = 0; k < kCrcMaxLen; ++k) {
-        mb[k] = masks[k * kCrcThreads + t];
-        ma[k] = masks[(kCrcMaxLen + k) * kCrcThreads + t];
-    }
-    // Three 8-byte loads when the block base and w0 are 8-aligned and the
-    // slice lies inside the block.
-    const bool vec = (K % 8u) == 0 && (reinterpret_cast<uintptr_t>(bits) & 7u) == 0 && w0 + kCrcW <= K;
-    const bool any = w0 < c.kprime;
-    __shared__ uint32_t red[kCrcBatch][2][kCrcThreads / 64];
-    for (uint32_t base = blockIdx.x * kCrcBatch; base < num_cb; base += gridDim.x * kCrcBatch) {
-        uint32_t v[kCrcBatch];
-        if (vec) {
-            // Unconditional loads (clamped block, own slice or the block's
-            // first), masked at use, so the batch is in flight together.
-            uint2 q[kCrcBatch][3];
-#pragma unroll
-            for (uint32_t u = 0; u < kCrcBatch; ++u) {
-                const uint32_t cbu = min(base + u, num_cb - 1);
-                const uint2 *p = reinterpret_cast<const uint2 *>(bits + static_cast<size_t>(cbu) * K + (any ? w0 : 0u));
-                q[u][0] = p[0];
-                q[u][1] = p[1];
-                q[u][2] = p[2];
-            }
-#pragma unroll
-            for (uint32_t u = 0; u < kCrcBatch; ++u) {
-                v[u] = Pack4(q[u][0].x) << 20 | Pack4(q[u][0].y) << 16 | Pack4(q[u][1].x) << 12 |
-                       Pack4(q[u][1].y) << 8 | Pack4(q[u][2].x) << 4 | Pack4(q[u][2].y);
-                if (!any || base + u >= num_cb) v[u] = 0;
-            }
+    __shared__ uint32_t red[2][kChunkThreads / 64];
+    const uint32_t t = threadIdx.x, p0 = 32u * t, n = max(nb, na);
+    uint32_t v = 0;
+    if (p0 < n) {
+        if (K % 16u == 0 && (reinterpret_cast<uintptr_t>(b) & 15u) == 0) {
+            const uint4 lo = *reinterpret_cast<const uint4 *>(b + p0);
+            const uint4 hi = p0 + 16u < K ? *reinterpret_cast<const uint4 *>(b + p0 + 16) : make_uint4(0, 0, 0, 0);
+            v = Pack4(lo.x) << 28 | Pack4(lo.y) << 24 | Pack4(lo.z) << 20 | Pack4(lo.w) << 16 | Pack4(hi.x) << 12 |
+                Pack4(hi.y) << 8 | Pack4(hi.z) << 4 | Pack4(hi.w);
         } else {
-#pragma unroll
-            for (uint32_t u = 0; u < kCrcBatch; ++u) {
-                v[u] = 0;
-                if (!any || base + u >= num_cb) continue;
-                const int8_t *b = bits + static_cast<size_t>(base + u) * K + w0;
-                for (uint32_t j = 0; j < kCrcW && w0 + j < K; ++j)
-                    v[u] |= static_cast<uint32_t>(b[j] & 1) << (kCrcW - 1 - j);
-            }
+            for (uint32_t j = 0; j < 32u && p0 + j < n; ++j) v |= static_cast<uint32_t>(b[p0 + j] & 1) << (31u - j);
         }
-        uint32_t rb[kCrcBatch], ra[kCrcBatch];
-#pragma unroll
-        for (uint32_t u = 0; u < kCrcBatch; ++u) {
-            rb[u] = CrcApply(v[u], mb);
-            ra[u] = CrcApply(v[u], ma);
-        }
-        for (int off = 32; off > 0; off >>= 1) {
-#pragma unroll
-            for (uint32_t u = 0; u < kCrcBatch; ++u) {
-                rb[u] ^= __shfl_xor(rb[u], off);
-                ra[u] ^= __shfl_xor(ra[u], off);
-            }
-        }
-        if ((t & 63u) == 0) {
-#pragma unroll
-            for (uint32_t u = 0; u < kCrcBatch; ++u) {
-                red[u][0][t >> 6] = rb[u];
-                red[u][1][t >> 6] = ra[u];
-            }
-        }
-        __syncthreads();
-        if (t < kCrcBatch && base + t < num_cb) {
-            uint32_t xb = 0, xa = 0;
-            for (uint32_t w = 0; w < blockDim.x / 64u; ++w) {
-                xb ^= red[t][0][w];
-                xa ^= red[t][1][w];
-            }
-            airan::CrcFinishBlock(c, base + t, xb, xa);
-        }
-        __syncthreads();
     }
+    auto part = [&](uint32_t len_msg, const uint32_t *pw, uint32_t poly, uint32_t len) {
+        if (p0 >= len_msg) return 0u;
+        const uint32_t m = min(32u, len_msg - p0);
+        return CrcMul32(v >> (32u - m), pw[len_msg - p0 - m], poly, len);
+    };
+    uint32_t rb = part(nb, pow_b, airan::kCrcPolyB, 24u), ra = part(na, pow_tb, poly_tb, len_tb);
+    for (int off = 32; off > 0; off >>= 1) {
+        rb ^= __shfl_xor(rb, off);
+        ra ^= __shfl_xor(ra, off);
+    }
+    if ((t & 63u) == 0) {
+        red[0][t >> 6] = rb;
+        red[1][t >> 6] = ra;
+    }
+    __syncthreads();
+    rb = ra = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kChunkThreads / 64u; ++w) {
+        rb ^= red[0][w];
+        ra ^= red[1][w];
+    }
+    *rb_out = rb;
+    *ra_out = ra;
+}
+
+// bits: int8 0/1 per bit, [cb][K], any K and alignment; a workgroup per block.
+// About 500 VALU instructions a wave, no table but the powers: 129 blocks take
+// 5.2 us (latency), where the matrix product's few workgroups of 32 blocks
+// take 16 (see kCrcMfmaMin).
+__global__ void __launch_bounds__(kChunkThreads) CbCrcKernel(const int8_t *__restrict__ bits, airan::CrcJob c,
+                                                            uint32_t K)
+{
+    const uint32_t cb = blockIdx.x;
+    uint32_t rb, ra;
+    CrcBlockRemainders(bits + static_cast<size_t>(cb) * K, K, c.crc_cb ? c.kprime : 0u, c.L, c.pow_b, c.pow_tb,
+                       c.poly_tb, c.len_tb, &rb, &ra);
+    if (threadIdx.x == 0) airan::CrcFinishBlock(c, cb, rb, ra);
 }
 
 // The same products on the matrix cores when K is a multiple of 32: the
@@ -373,55 +310,39 @@ __global__ void __launch_bounds__(256) PackKernel(const int8_t *__restrict__ bit
 // Ragged batch: one workgroup per code block of any grant.  The block's
 // CRC24B remainder over its K' bits and the remainder of its part of the
 // TB (its first K' - crc_cb bits) as the last bits of a message, shifted by
-// x^(bits after it in its TB) mod g_TB (the host's per-block `xpow`).
-__global__ void __launch_bounds__(256) RaggedCrcKernel(const int8_t *__restrict__ bits,
-                                                       const airan::RaggedCb *__restrict__ cbs,
-                                                       const uint32_t *__restrict__ pow_b,
-                                                       const uint32_t *__restrict__ pow_a,
-                                                       const uint32_t *__restrict__ pow_16,
-                                                       uint8_t *__restrict__ cb_ok, uint32_t *__restrict__ tb_part)
+// x^(bits after it in its TB) mod g_TB (the host's per-block `xpow`).  2282
+// blocks in 16.5 us; with two table loads per set bit it took 49.
+__global__ void __launch_bounds__(kChunkThreads) RaggedCrcKernel(const int8_t *__restrict__ bits,
+                                                                const airan::RaggedCb *__restrict__ cbs,
+                                                                const uint32_t *__restrict__ pow_b,
+                                                                const uint32_t *__restrict__ pow_a,
+                                                                const uint32_t *__restrict__ pow_16,
+                                                                uint8_t *__restrict__ cb_ok,
+                                                                uint32_t *__restrict__ tb_part)
 {
-    const airan::RaggedCb c = cbs[blockIdx.x];
-    const int8_t *b = bits + c.bits_off;
-    const uint32_t n = c.kprime, L = c.kprime - c.crc_cb;
-    const uint32_t *pw = c.len_tb == 24 ? pow_a : pow_16;
-    uint32_t rb = 0, ra = 0;
-    for (uint32_t j = threadIdx.x; j < n; j += blockDim.x) {
-        if (b[j] != 0) {
-            if (c.crc_cb) rb ^= pow_b[n - 1 - j];
-            if (j < L) ra ^= pw[L - 1 - j];
-        }
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        rb ^= __shfl_xor(rb, off);
-        ra ^= __shfl_xor(ra, off);
-    }
-    __shared__ uint32_t part[2][4];
-    if ((threadIdx.x & 63u) == 0) {
-        part[0][threadIdx.x / 64] = rb;
-        part[1][threadIdx.x / 64] = ra;
-    }
-    __syncthreads();
+    const airan::RaggedCb &c = cbs[blockIdx.x];
+    uint32_t rb, ra;
+    CrcBlockRemainders(bits + c.bits_off, c.k, c.crc_cb ? c.kprime : 0u, c.kprime - c.crc_cb, pow_b,
+                       c.len_tb == 24 ? pow_a : pow_16, c.poly_tb, c.len_tb, &rb, &ra);
     if (threadIdx.x == 0) {
-        rb = part[0][0] ^ part[0][1] ^ part[0][2] ^ part[0][3];
-        ra = part[1][0] ^ part[1][1] ^ part[1][2] ^ part[1][3];
         cb_ok[blockIdx.x] = c.crc_cb ? static_cast<uint8_t>(rb == 0) : static_cast<uint8_t>(1);
         tb_part[blockIdx.x] = airan::CrcMulMod(ra, c.xpow, c.poly_tb, c.len_tb);
     }
 }
 
-// tb_ok[t] = 1 when the parts of TB t's code blocks (first[t] .. first[t] +
-// count[t] - 1) XOR to zero.
+// tb_ok of TB blockIdx.x (one wave): the parts of its code blocks (first[t] ..
+// first[t] + count[t] - 1) XOR to zero.
 __global__ void __launch_bounds__(64) RaggedCrcFinishKernel(const uint32_t *__restrict__ tb_part,
                                                             const uint32_t *__restrict__ first,
                                                             const uint32_t *__restrict__ count,
-                                                            uint8_t *__restrict__ tb_ok, uint32_t num_tbs)
+                                                            uint8_t *__restrict__ tb_ok)
 {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= num_tbs) return;
+    const uint32_t t = blockIdx.x, n = count[t];
+    const uint32_t *p = tb_part + first[t];
     uint32_t x = 0;
-    for (uint32_t r = 0; r < count[t]; ++r) x ^= tb_part[first[t] + r];
-    tb_ok[t] = x == 0 ? 1 : 0;
+    for (uint32_t r = threadIdx.x; r < n; r += 64) x ^= p[r];
+    for (int off = 32; off > 0; off >>= 1) x ^= __shfl_xor(x, off);
+    if (threadIdx.x == 0) tb_ok[t] = x == 0 ? 1 : 0;
 }
 
 }  // namespace
@@ -463,10 +384,9 @@ int32_t LaunchCrcRagged(const RaggedCb *cbs, uint32_t num_cb, const int8_t *bits
     const int32_t st = EnsureTables(&t);
     if (st != AIRAN_OK) return st;
     if (num_cb == 0 || num_tbs == 0) return AIRAN_INVALID_ARGUMENT;
-    hipLaunchKernelGGL(RaggedCrcKernel, dim3(num_cb), dim3(256), 0, s, bits, cbs, t->pow_b, t->pow_a, t->pow_16,
+    hipLaunchKernelGGL(RaggedCrcKernel, dim3(num_cb), dim3(kChunkThreads), 0, s, bits, cbs, t->pow_b, t->pow_a, t->pow_16,
                        cb_ok, tb_part);
-    hipLaunchKernelGGL(RaggedCrcFinishKernel, dim3(CeilDiv(num_tbs, 64)), dim3(64), 0, s, tb_part, tb_first,
-                       tb_count, tb_ok, num_tbs);
+    hipLaunchKernelGGL(RaggedCrcFinishKernel, dim3(num_tbs), dim3(64), 0, s, tb_part, tb_first, tb_count, tb_ok);
     return LaunchStatus();
 }
 
@@ -485,51 +405,38 @@ int32_t CrcJobSetup(const AiranTbPlanV1 &p, uint8_t *cb_ok, uint32_t *tb_part, C
     return AIRAN_OK;
 }
 
-void LaunchCrcZero(uint32_t *words, uint32_t n, hipStream_t s)
-{
-    hipLaunchKernelGGL(ZeroKernel, dim3(CeilDiv(n, 256)), dim3(256), 0, s, words, n);
-}
+// Blocks from which the matrix product (32 blocks per workgroup) is the faster
+// check.  A workgroup per block against it, K = 8448: 129 blocks 5.2 / 16.1 us,
+// 2064 blocks 15.7 / 19.0 us, 8256 blocks 42.9 / 31.9 us; lines through these
+// cross near 3000.
+constexpr uint32_t kCrcMfmaMin = 3000;
 
 // The matrix-core path needs whole position pairs and aligned 16-byte loads.
-bool CrcMfmaEligible(const void *bits, uint32_t K, const void *tables)
+bool CrcMfmaEligible(const void *bits, uint32_t K, uint32_t num_cb, const void *tables)
 {
-    return K % 32 == 0 && ((reinterpret_cast<uintptr_t>(bits) | reinterpret_cast<uintptr_t>(tables)) & 15u) == 0;
+    return num_cb >= kCrcMfmaMin && K % 32 == 0 &&
+           ((reinterpret_cast<uintptr_t>(bits) | reinterpret_cast<uintptr_t>(tables)) & 15u) == 0;
 }
 
-void LaunchCrcTables(const CrcJob &c, uint32_t K, void *tables, hipStream_t s)
+// The fragment table of the matrix product, where a check of num_cb blocks
+// would take it.
+void LaunchCrcTables(const CrcJob &c, uint32_t K, uint32_t num_cb, void *tables, hipStream_t s)
 {
-    if (K % 32 == 0) {
-        const uint32_t P = K / 32;
-        static_assert(kCrcTableBytes >= 2 * (8448 / 32) * 64 * sizeof(uint4), "fragment table size");
-        hipLaunchKernelGGL(CrcFragKernel, dim3(CeilDiv(2 * P * 64, 256)), dim3(256), 0, s, c, P,
-                           static_cast<uint4 *>(tables));
-    }
-    // The masks of the VALU path follow the fragment table (used when the
-    // bits are not 16-byte aligned).
-    hipLaunchKernelGGL(CrcMaskKernel, dim3(1), dim3(kCrcThreads), 0, s, c,
-                       reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(tables) + kCrcFragBytes));
+    if (K % 32 != 0 || num_cb < kCrcMfmaMin) return;
+    const uint32_t P = K / 32;
+    static_assert(kCrcTableBytes >= 2 * (8448 / 32) * 64 * sizeof(uint4), "fragment table size");
+    hipLaunchKernelGGL(CrcFragKernel, dim3(CeilDiv(2 * P * 64, 256)), dim3(256), 0, s, c, P,
+                       static_cast<uint4 *>(tables));
 }
 
 void LaunchCbCrc(const int8_t *bits, const CrcJob &c, uint32_t K, uint32_t num_cb, const void *tables,
                  hipStream_t s)
 {
-    if (CrcMfmaEligible(bits, K, tables)) {
+    if (CrcMfmaEligible(bits, K, num_cb, tables))
         hipLaunchKernelGGL(CrcMfmaKernel, dim3(CeilDiv(num_cb, kCrcCols)), dim3(kCrcWaves * 64), 0, s, bits, c, K,
                            num_cb, static_cast<const uint4 *>(tables));
-        return;
-    }
-    const uint32_t *masks = reinterpret_cast<const uint32_t *>(static_cast<const uint8_t *>(tables) + kCrcFragBytes);
-    // One resident wave of workgroups (the masks are built once per workgroup).
-    uint32_t cap = 1024;
-    int dev = 0, cus = 0, per_cu = 0;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void *>(CbCrcKernel),
-                                                     static_cast<int>(kCrcThreads), 0) == hipSuccess &&
-        cus > 0 && per_cu > 0)
-        cap = static_cast<uint32_t>(cus) * static_cast<uint32_t>(per_cu);
-    const uint32_t grid = std::max(1u, std::min(CeilDiv(num_cb, kCrcBatch), cap));
-    hipLaunchKernelGGL(CbCrcKernel, dim3(grid), dim3(kCrcThreads), 0, s, bits, c, K, num_cb, masks);
+    else
+        hipLaunchKernelGGL(CbCrcKernel, dim3(num_cb), dim3(kChunkThreads), 0, s, bits, c, K);
 }
 
 void LaunchCrcFinish(const uint32_t *tb_part, uint8_t *tb_ok, uint32_t num_tbs, uint32_t C, hipStream_t s)
@@ -541,7 +448,7 @@ void LaunchCrcFinish(const uint32_t *tb_part, uint8_t *tb_ok, uint32_t num_tbs, 
 
 extern "C" size_t airan_crc_check_WorkspaceBytes(uint32_t num_tbs)
 {
-    // Per-block TB remainder parts, then the check masks.
+    // Per-block TB remainder parts, then the matrix product's table.
     return airan::CrcTableOffset(num_tbs) + airan::kCrcTableBytes;
 }
 
@@ -566,7 +473,7 @@ extern "C" int32_t airan_crc_check_Enqueue(const AiranTbPlanV1 *p, uint32_t num_
                      p->Kprime - p->crc_cb, d.poly_tb, d.len_tb};
     hipStream_t s = static_cast<hipStream_t>(stream);
     void *tables = static_cast<uint8_t *>(workspace) + airan::CrcTableOffset(num_tbs);
-    airan::LaunchCrcTables(c, p->K, tables, s);
+    airan::LaunchCrcTables(c, p->K, num_tbs * p->C, tables, s);
     airan::LaunchCbCrc(static_cast<const int8_t *>(bits), c, p->K, num_tbs * p->C, tables, s);
     airan::LaunchCrcFinish(static_cast<const uint32_t *>(workspace), static_cast<uint8_t *>(tb_ok), num_tbs, p->C, s);
     if (tb_bytes != nullptr) {
