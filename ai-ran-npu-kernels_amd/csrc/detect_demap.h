@@ -10,49 +10,50 @@
 
 namespace airan {
 
-__device__ inline int16_t SatNeg16(int v) { return static_cast<int16_t>(v == -32768 ? 32767 : -v); }
-
 // xh / ne: the RE's LMMSE outputs; gw: the scrambling bits from this RE's
-// first codeword bit on (bit l * qm + b for layer l, bit plane b); out: the
-// RE's first codeword position in bit plane 0 (planes cw_stride apart).
-// QM > 0 fixes the modulation at compile time.
+// first codeword bit on (bit l * QM + b for layer l, bit plane b); out: bit
+// plane 0 (uniform; planes cw_stride apart), pos: the RE's first codeword
+// position.  The LLRs (at most 2560 in magnitude) stay packed by axis, plane 2 k in the low
+// and 2 k + 1 in the high half, and leave as one NL-element store per plane.
 template <int NL, int QM>
-__device__ inline void DemapStore(const Cf (&xh)[4], const float (&ne)[4], uint32_t qm_rt, __half floor16,
-                                  uint64_t gw, int16_t *out, uint32_t cw_stride)
+__device__ inline void DemapStore(const Cf (&xh)[4], const float (&ne)[4], __half floor16, uint64_t gw, int16_t *out,
+                                  uint32_t pos, uint32_t cw_stride)
 {
-    const uint32_t qm = QM > 0 ? static_cast<uint32_t>(QM) : qm_rt, m = qm / 2;
+    constexpr int M = QM / 2;
+    // l QM + b < NL QM <= 32: the RE's bits are the low word's.
     const uint32_t g32 = static_cast<uint32_t>(gw);
-    // LLRs of all layers first, then one contiguous NL-element store per bit
-    // plane (the thread's REs are adjacent within a plane).
-    int16_t v[8][NL];
+    s16x2_t v[M][NL];
 #pragma unroll
     for (int l = 0; l < NL; ++l) {
-        const __half xr16 = __float2half_rn(xh[l].r), xi16 = __float2half_rn(xh[l].i);
+        const h16x2_t x = {static_cast<_Float16>(xh[l].r), static_cast<_Float16>(xh[l].i)};
         __half ne16 = __float2half_rn(ne[l]);
         if (__half2float(ne16) < __half2float(floor16)) ne16 = floor16;
-        int llr[8];
-        QamSymbolLlrs(qm, xr16, xi16, ne16, llr);
+        s16x2_t w[M];
+        QamSymbolPair<QM>(x, ne16, w);
 #pragma unroll
-        for (uint32_t b = 0; b < 8; ++b) {
-            const uint32_t stream = (b & 1u) ? m + b / 2 : b / 2;
-            const int x = b < qm ? llr[stream] : 0;
-            // l qm + b < NL qm <= 32: the RE's bits are the low word's.
-            const bool flip = (g32 >> (static_cast<uint32_t>(l) * qm + b)) & 1u;
-            v[b][l] = flip ? SatNeg16(x) : static_cast<int16_t>(x);
+        for (int k = 0; k < M; ++k) {
+            // Times 4, or -4 where the scrambling bit is set.
+            const uint32_t b = g32 >> (l * QM + 2 * k);
+            const s16x2_t bit = __builtin_bit_cast(s16x2_t, (b & 1u) | (b & 2u) << 15);
+            const s16x2_t four = {4, 4};
+            v[k][l] = w[k] * (bit * static_cast<short>(-8) + four);
         }
     }
-    for (uint32_t b = 0; b < qm; ++b) {
-        int16_t *o = out + static_cast<size_t>(b) * cw_stride;
+    auto half = [](s16x2_t x, int q) { return static_cast<uint32_t>(static_cast<uint16_t>(q ? x.y : x.x)); };
+#pragma unroll
+    for (int b = 0; b < QM; ++b) {
+        int16_t *plane = out + static_cast<size_t>(b) * cw_stride;
+        const s16x2_t *p = v[b / 2];
+        const uint32_t at = 2u * pos;
         if constexpr (NL == 4) {
-            *reinterpret_cast<uint2 *>(o) =
-                make_uint2(static_cast<uint16_t>(v[b][0]) | static_cast<uint32_t>(static_cast<uint16_t>(v[b][1])) << 16,
-                           static_cast<uint16_t>(v[b][2]) | static_cast<uint32_t>(static_cast<uint16_t>(v[b][3])) << 16);
+            typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+            *PlaneAt(reinterpret_cast<u32x2_t *>(plane), at) =
+                u32x2_t{half(p[0], b & 1) | half(p[1], b & 1) << 16, half(p[2], b & 1) | half(p[3], b & 1) << 16};
         } else if constexpr (NL == 2) {
-            *reinterpret_cast<uint32_t *>(o) =
-                static_cast<uint16_t>(v[b][0]) | static_cast<uint32_t>(static_cast<uint16_t>(v[b][1])) << 16;
+            *PlaneAt(reinterpret_cast<uint32_t *>(plane), at) = half(p[0], b & 1) | half(p[1], b & 1) << 16;
         } else {
 #pragma unroll
-            for (int l = 0; l < NL; ++l) o[l] = v[b][l];
+            for (int l = 0; l < NL; ++l) *PlaneAt(plane, at + 2u * l) = static_cast<int16_t>(half(p[l], b & 1));
         }
     }
 }

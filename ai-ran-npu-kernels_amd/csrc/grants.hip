@@ -46,7 +46,7 @@ __global__ void __launch_bounds__(256) GrantGoldKernel(uint32_t *__restrict__ bi
 // Detection + QAM demap + layer demap + descramble of one RE of one grant:
 // the single-grant chain's fused detector (per-RE LMMSE on the vector
 // units, no_eff floor, the qam256_demod arithmetic, Gold descrambling).
-template <int NL>
+template <int NL, int QM>
 __device__ inline void RaggedDetectRe(const RaggedGrant &gr, uint32_t ds, uint32_t sc, const __half *__restrict__ rx_re,
                                       const __half *__restrict__ rx_im, const __half *__restrict__ h_re,
                                       const __half *__restrict__ h_im, const __half *__restrict__ noise,
@@ -58,25 +58,26 @@ __device__ inline void RaggedDetectRe(const RaggedGrant &gr, uint32_t ds, uint32
     for (uint32_t r = 0; r < nr; ++r) s += __half2float(noise[gr.noise_off + r]);
     const float no = __half2float(__float2half_rn(s * (1.0f / static_cast<float>(nr))));
     const size_t plane = static_cast<size_t>(g.nsym) * g.pad;
-    const size_t off = static_cast<size_t>(g.data_sym[ds]) * g.pad + sc;
+    const uint32_t off = 2u * (g.data_sym[ds] * g.pad + sc);
+    const __half *hr_g = h_re + gr.h_off, *hi_g = h_im + gr.h_off, *yr_g = rx_re + gr.rx_off, *yi_g = rx_im + gr.rx_off;
     auto loadh = [&](int r, int l) {
-        const size_t i = gr.h_off + (static_cast<size_t>(r) * NL + l) * plane + off;
-        return Cf{__half2float(h_re[i]), __half2float(h_im[i])};
+        const size_t p = (static_cast<size_t>(r) * NL + l) * plane;
+        return Cf{airan::LoadAt(hr_g + p, off), airan::LoadAt(hi_g + p, off)};
     };
     auto loady = [&](int r) {
-        const size_t i = gr.rx_off + static_cast<size_t>(r) * plane + off;
-        return Cf{__half2float(rx_re[i]), __half2float(rx_im[i])};
+        const size_t p = static_cast<size_t>(r) * plane;
+        return Cf{airan::LoadAt(yr_g + p, off), airan::LoadAt(yi_g + p, off)};
     };
     Cf xh[4];
     float ne[4];
     airan::Detect<NL>(static_cast<int>(nr), no, loadh, loady, xh, ne);
     const uint32_t re = ds * g.used + sc;
-    const uint64_t bit0 = static_cast<uint64_t>(re) * NL * g.qm;
+    const uint64_t bit0 = static_cast<uint64_t>(re) * NL * QM;
     const uint32_t *gb = gold + gr.gold_off;
     const uint32_t w0 = static_cast<uint32_t>(bit0 >> 5);
     const uint64_t gw = (static_cast<uint64_t>(gb[w0]) | (static_cast<uint64_t>(gb[w0 + 1]) << 32)) >> (bit0 & 31u);
-    airan::DemapStore<NL, 0>(xh, ne, g.qm, __ushort_as_half(static_cast<uint16_t>(gr.floor16)), gw,
-                             cw + gr.cw_off + static_cast<size_t>(re) * NL, g.cw_stride);
+    airan::DemapStore<NL, QM>(xh, ne, __ushort_as_half(static_cast<uint16_t>(gr.floor16)), gw, cw + gr.cw_off, re * NL,
+                              g.cw_stride);
 }
 
 // One workgroup per tile (grant, data symbol, blockDim.x subcarriers).
@@ -94,11 +95,23 @@ __global__ void __launch_bounds__(256) RaggedDetectKernel(const __half *__restri
     const RaggedGrant &gr = grants[t.grant];
     const uint32_t sc = t.sc0 + threadIdx.x;
     if (sc >= gr.g.used) return;
-    switch (gr.g.nl) {
-    case 1: RaggedDetectRe<1>(gr, t.ds, sc, rx_re, rx_im, h_re, h_im, noise, gold, cw); break;
-    case 2: RaggedDetectRe<2>(gr, t.ds, sc, rx_re, rx_im, h_re, h_im, noise, gold, cw); break;
-    case 3: RaggedDetectRe<3>(gr, t.ds, sc, rx_re, rx_im, h_re, h_im, noise, gold, cw); break;
-    default: RaggedDetectRe<4>(gr, t.ds, sc, rx_re, rx_im, h_re, h_im, noise, gold, cw); break;
+    // Uniform over the workgroup.
+    auto run = [&](auto nl, auto qm) {
+        RaggedDetectRe<decltype(nl)::value, decltype(qm)::value>(gr, t.ds, sc, rx_re, rx_im, h_re, h_im, noise, gold, cw);
+    };
+    auto layers = [&](auto qm) {
+        switch (gr.g.nl) {
+        case 1: run(std::integral_constant<int, 1>{}, qm); break;
+        case 2: run(std::integral_constant<int, 2>{}, qm); break;
+        case 3: run(std::integral_constant<int, 3>{}, qm); break;
+        default: run(std::integral_constant<int, 4>{}, qm); break;
+        }
+    };
+    switch (gr.g.qm) {
+    case 2: layers(std::integral_constant<int, 2>{}); break;
+    case 4: layers(std::integral_constant<int, 4>{}); break;
+    case 6: layers(std::integral_constant<int, 6>{}); break;
+    default: layers(std::integral_constant<int, 8>{}); break;
     }
 }
 

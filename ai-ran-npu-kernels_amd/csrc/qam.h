@@ -112,4 +112,68 @@ __device__ inline void QamSymbolLlrs(uint32_t qm, __half xr, __half xi, __half n
     }
 }
 
+// ------------------------------------------------- packed (I, Q) demapper
+typedef short s16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 h16x2_t __attribute__((ext_vector_type(2)));
+
+// The LLRs of one symbol in the units above divided by 4, the I axis in the
+// low and the Q axis in the high half: w[k] holds streams k and Qm/2 + k.
+// Closed forms of the max-log over the 2^(Qm/2) levels for every modulation
+// (equal to AxisExhaustive for every integer u in +-1000 and t >= 0), with
+// cl_i = min(|u|, 2 i t); every coefficient is a multiple of 4, so the clip
+// to +-2560 is one to +-640 here.  From t = 1024 on each LLR is clipped or
+// constant in t (2 i t >= |u|, and the t terms exceed the clip), so t is
+// limited there and all sums fit 16 bits.
+template <int QM>
+__device__ inline void AxisPair(s16x2_t u, s16x2_t t, s16x2_t (&w)[QM / 2])
+{
+    constexpr int M = QM / 2;
+    const s16x2_t a = __builtin_elementwise_max(u, -u), t2 = t + t;
+    s16x2_t cl[8], kt = t2, sum = {0, 0};
+#pragma unroll
+    for (int i = 1; i < (1 << (M - 1)); ++i) {
+        cl[i] = __builtin_elementwise_min(a, kt);
+        sum += cl[i];
+        kt += t2;
+    }
+    const s16x2_t neg = u >> 15;  // -1 where u < 0
+    w[0] = ((sum ^ neg) - neg) - u * static_cast<short>(1 << (M - 1));
+    if constexpr (M == 2) w[1] = a - t2;
+    if constexpr (M == 3) {
+        w[1] = (a + a + cl[1]) - (t2 * static_cast<short>(3) + cl[3]);
+        w[2] = (t2 + a) - (cl[2] + cl[2]);
+    }
+    if constexpr (M == 4) {
+        w[1] = (a * static_cast<short>(4) + (cl[1] + cl[2] + cl[3])) - (t2 * static_cast<short>(10) + (cl[5] + cl[6] + cl[7]));
+        w[2] = (t2 * static_cast<short>(3) + (a + a) + cl[3] + cl[5]) - (cl[4] * static_cast<short>(4) + cl[1] + cl[7]);
+        w[3] = (t2 + a) + (cl[4] - cl[2] - cl[6]) * static_cast<short>(2);
+    }
+    const s16x2_t hi = {640, 640}, lo = {-640, -640};
+#pragma unroll
+    for (int k = 0; k < M; ++k) w[k] = __builtin_elementwise_max(__builtin_elementwise_min(w[k], hi), lo);
+}
+
+// QamUT and AxisPair of one symbol (x = (I, Q) in fp16).  The fp16 quotients
+// D / n by the hardware reciprocal: rounded to fp16 they equal the division's
+// for every fp16 n and each of the eight constants (checked by exhaustion).
+// The limits of u apply before its rounding (integers, so the same), the
+// order of max and min giving a NaN u = -1000 as QamUT does.
+template <int QM>
+__device__ inline void QamSymbolPair(h16x2_t x, __half n, s16x2_t (&w)[QM / 2])
+{
+    uint16_t dq, d2q;
+    QamConsts(QM, &dq, &d2q);
+    float nf = __half2float(n);
+    if (!(nf >= 6.103515625e-05f) || !isfinite(nf)) nf = 6.103515625e-05f;
+    const float rn = __builtin_amdgcn_rcpf(nf);
+    const _Float16 scale = static_cast<_Float16>(__half2float(__ushort_as_half(dq)) * rn);
+    const float thr = static_cast<float>(static_cast<_Float16>(__half2float(__ushort_as_half(d2q)) * rn));
+    const h16x2_t s2 = {scale, scale}, lim = {static_cast<_Float16>(1000.0f), static_cast<_Float16>(1000.0f)};
+    const h16x2_t p = __builtin_elementwise_min(__builtin_elementwise_max(x * s2, -lim), lim);
+    const s16x2_t u = __builtin_convertvector(__builtin_elementwise_rint(p), s16x2_t);
+    const short t = static_cast<short>(rintf(fminf(thr, 1024.0f)));
+    const s16x2_t tt = {t, t};
+    AxisPair<QM>(u, tt, w);
+}
+
 }  // namespace airan
