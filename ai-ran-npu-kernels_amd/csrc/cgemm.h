@@ -52,9 +52,12 @@ __device__ inline uint32_t Bf16Bits(float x)
     return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
 }
 
+// No contraction: a product that the caller passes is rounded to fp32 before it
+// is split, in every kernel alike.
 template <int S>
 __device__ inline void Bf16Parts(float x, uint32_t *part)
 {
+#pragma clang fp contract(off)
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         part[s] = Bf16Bits(x);

@@ -19,7 +19,14 @@
 // uncorrelated, each observed on a comb of spacing 4 (offsets comb and
 // comb + 2); each gets its own comb-model filter and h0,1 = (g+ +- g-) / 2.
 //
-// The eigen-factors of every observation model are built once per grant
+// Models that differ only in their comb offset share one base: R_pp depends on
+// the observations' number and spacing alone, and R_hp on the distance between
+// subcarrier and observation, so the model of offset o is the base of offset 0
+// with its rows shifted by o (four models at rank 4, two of a pair or of two
+// combs).  The base is stored once, over the subcarriers the shifts reach, and
+// the models' columns are stacked in one product against it.
+//
+// The eigen-factors of every base are built once per grant
 // shape in FP64 on the device (covariances by a kernel, rocSOLVER zheevd,
 // rocBLAS zgemm); the noise-dependent parts are applied per slot, with the
 // noise estimated from the energy outside the kept eigenspace.
@@ -56,22 +63,29 @@ constexpr uint32_t kProjKTile = 128;
 // receive antenna, DMRS symbol) x kInterpTile subcarriers.
 constexpr uint32_t kInterpTile = 128;
 
-// One observation model: n observations at offset + step * p.
-struct CeModelFactors {
-    uint32_t n = 0;      // observations
-    uint32_t step = 0;   // subcarrier spacing of the observations (2 or 4)
-    uint32_t offset = 0;
-    uint32_t in_a = 0;   // z = h_ls[in_a] + sign_b * h_ls[in_b]
-    uint32_t in_b = 0;
-    float sign_b = 0.0f;
-    uint32_t rank = 0;   // stored eigenpairs (multiple of 16; columns >= kept are zero)
-    uint32_t kept = 0;   // eigenpairs actually kept
-    float2 *bt = nullptr;  // [n][rank]    bt[p][k] = conj(U[p][k])
-    float *a2 = nullptr;   // [rank][used] |(R_hp U)[sc][k]|^2, subcarrier contiguous
-    uint16_t *a16 = nullptr;  // R_hp U, 2-part fragment planes: rows sc < AlignUp(used, kInterpTile), K = rank
+// A base: n observations at step * p, estimated at the subcarriers r - max_off,
+// r < rows = used + max_off (max_off: the largest comb offset of its models).
+struct CeBaseFactors {
+    uint32_t n = 0;        // observations
+    uint32_t step = 0;     // subcarrier spacing of the observations (2 or 4)
+    uint32_t max_off = 0;
+    uint32_t rows = 0;
+    uint32_t q0 = 0, nq = 0;  // its models q0 .. q0 + nq - 1
+    uint32_t rank = 0;     // stored eigenpairs (multiple of 16; columns >= kept are zero)
+    uint32_t kept = 0;     // eigenpairs actually kept
+    float *a2 = nullptr;   // [rank][rows] |(R_hp U)[r][k]|^2, subcarrier contiguous
+    uint16_t *a16 = nullptr;  // R_hp U, 2-part fragment planes: r < AlignUp(rows, kInterpTile), K = rank
     uint16_t *w16 = nullptr;  // conj(U) transposed, 3-part fragment planes: rows k < AlignUp(rank, kProjKTile),
                               // K = AlignUp(n, 16) observations (zero beyond n)
     float *lam = nullptr;  // [rank] eigenvalues (1 for padded columns)
+};
+
+// One observation model: its base and comb offset, and its observations
+// z = h_ls[in_a] + sign_b * h_ls[in_b].
+struct CeModel {
+    uint32_t base = 0, offset = 0;
+    uint32_t in_a = 0, in_b = 0;
+    float sign_b = 0.0f;
 };
 
 }  // namespace
@@ -80,8 +94,10 @@ struct LmmseFilter {
     int device;
     Geom g;
     LmmseFilterParamsV1 params;
-    uint32_t nm;                       // observation models
-    CeModelFactors model[kMaxModels];
+    uint32_t nb;                       // bases
+    CeBaseFactors base[kMaxModels];
+    uint32_t nm;                       // observation models, each base's adjacent
+    CeModel model[kMaxModels];
     int32_t layer_model[4][2];         // models of layer l (second = -1 for a comb model)
     float layer_sign[4];               // h_l = (g_a + sign g_b) / 2 for an FD-OCC pair
     float rt[14][4];                   // J0(2 pi f_d (s - d_j) T) per symbol and DMRS symbol
@@ -139,10 +155,12 @@ __global__ void __launch_bounds__(256) PackBtKernel(const double2 *__restrict__ 
     bt[static_cast<size_t>(p) * rank + k] = o;
 }
 
+// Subcarriers i0 .. used - 1 of av go to rows i + shift of at (rows columns).
 __global__ void __launch_bounds__(256) PackAtKernel(const double2 *__restrict__ av, float2 *__restrict__ at,
-                                                    uint32_t used, uint32_t rank, uint32_t kept)
+                                                    uint32_t used, uint32_t i0, uint32_t shift, uint32_t rows,
+                                                    uint32_t kept)
 {
-    const uint32_t sc = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t sc = i0 + blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t k = blockIdx.y;
     if (sc >= used) return;
     float2 o = make_float2(0.0f, 0.0f);
@@ -151,7 +169,7 @@ __global__ void __launch_bounds__(256) PackAtKernel(const double2 *__restrict__ 
         const double2 e = av[sc + static_cast<size_t>(kept - 1 - k) * used];
         o = make_float2(static_cast<float>(e.x), static_cast<float>(e.y));
     }
-    at[static_cast<size_t>(k) * used + sc] = o;
+    at[static_cast<size_t>(k) * rows + sc + shift] = o;
 }
 
 // a16 = at transposed into bf16 fragment planes (rows sc < sc_pad, zero
@@ -191,24 +209,41 @@ __global__ void __launch_bounds__(256) PackW16Kernel(const float2 *__restrict__ 
 }
 
 // ---------------------------------------------------------------- apply
-struct CeModelDev {
-    const float2 *bt;
+struct CeBaseDev {
     const float *a2;
     const uint16_t *a16;
     const uint16_t *w16;
     const float *lam;
-    uint32_t n, rank, kept, in_a, in_b;
+    uint32_t n, rank, kept, rows, q0, nq;
+};
+
+struct CeModelDev {
+    uint32_t base, shift;  // subcarrier sc is the base's row sc + shift
+    uint32_t in_a, in_b;
     float sign_b;
 };
 
 struct CeApply {
-    uint32_t nr, nl, nm, ndmrs, pilot_pad, used, pad, nsym;
+    uint32_t nr, nl, nm, nb, ndmrs, pilot_pad, used, pad, nsym;
+    CeBaseDev b[kMaxModels];
     CeModelDev m[kMaxModels];
     int32_t layer_model[4][2];
     float layer_sign[4];
     float rt[14][4];
     float rtt[4][4];
 };
+
+// A base's columns (rows of its products): row = (model * slots + slot) *
+// NR*D + col, model counted from q0.
+struct CeRow {
+    uint32_t q, slot, col;
+};
+__device__ inline CeRow RowOf(const CeApply &c, const CeBaseDev &bd, uint32_t slots, uint32_t row)
+{
+    const uint32_t ncol = c.nr * c.ndmrs, ms = row / ncol, mi = ms / slots;
+    return {bd.q0 + mi, ms - mi * slots, row - ms * ncol};
+}
+__host__ __device__ inline uint32_t BaseRows(uint32_t nq, uint32_t slots, uint32_t ncol) { return nq * slots * ncol; }
 
 // Workspace layout for `slots` slots (each part 256-byte aligned):
 //   stats  [slots][4]                       fp32  relative noise n_q
@@ -219,12 +254,13 @@ struct CeApply {
 //   hf     [slots][models][NR*D][used]      c64   frequency estimate (unscaled)
 //   tp     [kProjSplits][slots][models][NR*D][kMaxRank]  c64  partial U^H z
 //          over one of kProjSplits fixed ranges of the observations
-//   zb     [models][zb_stride]               bf16  z in 3-part fragment planes:
-//          rows n = slot * NR*D + col < npad (zero beyond slots * NR*D),
-//          K = AlignUp(n_q, 16) observations (zero beyond n_q)
+//   zb     [models][zb_stride]               bf16  z in 3-part fragment planes,
+//          a base's rows (RowOf) from its first model's part on, K =
+//          AlignUp(n, 16) observations (zero beyond n)
 //   tb     [models][TbModelElems]            bf16  t / (lam_k + n_q) in fragment
-//          planes: rows n = slot * NR*D + col < AlignUp(slots * NR*D,
-//          kInterpTile) (zero beyond), K = the model's rank
+//          planes, the same rows, K = the base's rank
+// Rows beyond a base's last are not written: a row of a product depends on
+// that row alone, and theirs are not stored.
 struct CeWs {
     float *stats;
     double *energy;
@@ -238,6 +274,10 @@ struct CeWs {
     size_t zb_stride;  // bf16 per model in zb
     uint32_t npad;     // rows of tb and zb per model
 };
+
+// A base's rows against the row tile of the 128-row products: below this many
+// the 32-row forms are the faster (see CeInterpRowsBody).
+constexpr uint32_t kSmallRows = 256;
 
 size_t Align256(size_t b) { return (b + 255) / 256 * 256; }
 
@@ -282,10 +322,10 @@ size_t CeWsLayout(const Geom &g, uint32_t slots, uint8_t *base, CeWs *w)
     return off;
 }
 
-__device__ inline float2 LoadZ(const __half *hr, const __half *hi, const CeApply &c, const CeModelDev &md,
+__device__ inline float2 LoadZ(const __half *hr, const __half *hi, const CeApply &c, const CeModelDev &md, uint32_t n,
                                uint32_t slot, uint32_t col, uint32_t p)
 {
-    if (p >= md.n) return make_float2(0.0f, 0.0f);
+    if (p >= n) return make_float2(0.0f, 0.0f);
     const uint32_t rx = col / c.ndmrs, d = col - rx * c.ndmrs;
     const size_t ha = (((static_cast<size_t>(slot) * c.nr + rx) * c.nl + md.in_a) * c.ndmrs + d) * c.pilot_pad + p;
     float2 v = make_float2(__half2float(hr[ha]), __half2float(hi[ha]));
@@ -307,29 +347,29 @@ __device__ inline void ProjRange(uint32_t n, uint32_t part, uint32_t *p0, uint32
     *len = b - a;
 }
 
-// zb[q] = z[slot, col][p] in 3-part fragment planes (rows n = slot * NR*D +
-// col, zero for n >= slots * NR*D and p >= n_q), one thread per row and 8
-// observations.  Grid (npad * AlignUp(max n, 16) / 8 / 256, models).
+// zb = z[slot, col][p] of every model in 3-part fragment planes, one thread per
+// row and 8 observations (zero for p >= n).  Grid (rows * AlignUp(max n, 16) /
+// 8 / 256, bases).
 __device__ __forceinline__ void CeZSplitKernelBody(const __half *__restrict__ hr, const __half *__restrict__ hi,
                                                       const CeWs &w, uint32_t slots, const CeApply &c, uint32_t bx, uint32_t by)
 {
-    const uint32_t q = by;
-    const CeModelDev &md = c.m[q];
+    const CeBaseDev &bd = c.b[by];
     const uint32_t e = bx * blockDim.x + threadIdx.x;
-    const uint32_t n = e % w.npad, p0 = (e / w.npad) * 8u;
-    const uint32_t pk = airan::AlignUp(md.n, 16u);
+    const uint32_t rows = BaseRows(bd.nq, slots, c.nr * c.ndmrs);
+    const uint32_t n = e % rows, p0 = (e / rows) * 8u;
+    const uint32_t pk = airan::AlignUp(bd.n, 16u);
     if (p0 >= pk) return;
-    const uint32_t ncol = c.nr * c.ndmrs;
     float2 v[8];
 #pragma unroll
     for (uint32_t j = 0; j < 8; ++j) v[j] = make_float2(0.0f, 0.0f);
-    if (n < slots * ncol) {
+    {
         // LoadZ of observations p0 .. p0 + 7 with 16-byte loads (p0 and
         // pilot_pad are multiples of 8 and p0 + 8 <= pk <= pilot_pad).
-        const uint32_t slot = n / ncol, col = n - slot * ncol;
-        const uint32_t rx = col / c.ndmrs, d = col - rx * c.ndmrs;
+        const CeRow cr = RowOf(c, bd, slots, n);
+        const CeModelDev &md = c.m[cr.q];
+        const uint32_t rx = cr.col / c.ndmrs, d = cr.col - rx * c.ndmrs;
         auto row = [&](uint32_t layer) {
-            return (((static_cast<size_t>(slot) * c.nr + rx) * c.nl + layer) * c.ndmrs + d) * c.pilot_pad + p0;
+            return (((static_cast<size_t>(cr.slot) * c.nr + rx) * c.nl + layer) * c.ndmrs + d) * c.pilot_pad + p0;
         };
         auto h8 = [](const __half *base, size_t off, float *out) {
             const uint4 u = *reinterpret_cast<const uint4 *>(base + off);
@@ -353,9 +393,9 @@ __device__ __forceinline__ void CeZSplitKernelBody(const __half *__restrict__ hr
         }
 #pragma unroll
         for (uint32_t j = 0; j < 8; ++j)
-            if (p0 + j < md.n) v[j] = make_float2(ar[j], ai[j]);
+            if (p0 + j < bd.n) v[j] = make_float2(ar[j], ai[j]);
     }
-    airan::StoreFrag8<3>(w.zb + q * w.zb_stride, n, p0, pk / 16u, v);
+    airan::StoreFrag8<3>(w.zb + bd.q0 * w.zb_stride, n, p0, pk / 16u, v);
 }
 __global__ void __launch_bounds__(256) CeZSplitKernel(const __half *__restrict__ hr, const __half *__restrict__ hi,
                                                       CeWs w, uint32_t slots, CeApply c)
@@ -365,70 +405,101 @@ __global__ void __launch_bounds__(256) CeZSplitKernel(const __half *__restrict__
 
 // tp[part][slot, q][col][k] = sum_{p in range(part)} z[slot, col][p] conj(U[p][k])
 // on split bf16 MFMA with 3 parts (fp32-accurate products, which the
-// subspace noise estimate needs): C = ZB W^T with rows n (slot, col) and
-// columns k.  Workgroup: 64 rows x kProjKTile eigenvectors of one (model,
-// split), four waves of 32 x 64 (1 x 2 blocks of 32 x 32).  Linear grid of
-// 8 * per_xcd workgroups; each XCD takes a contiguous range of tiles ordered
-// (model, split) major, so the operands of one (model, split) -- about 2 MB
-// at 273 PRB and 64 slots -- are read through one L2.
+// subspace noise estimate needs): C = ZB W^T with a base's rows n (RowOf) and
+// columns k.  Workgroup: RB * 32 rows x kProjKTile eigenvectors of one (base,
+// split): RB = 2, four waves of 32 x 64, or, for a base of few rows, RB = 1,
+// four waves of 32 x 32.  The operands of the next steps of 16 observations are
+// loaded while a step's products run.  Linear grid of 8 * per_xcd workgroups per
+// base; each XCD takes a contiguous range of tiles ordered split major, so
+// the operands of one split are read through one L2.
+template <uint32_t RB>
 __device__ __forceinline__ void CeProjectMfmaKernelBody(const CeWs &w, uint32_t slots, const CeApply &c, uint32_t k_tiles,
                                                               uint32_t per_xcd, uint32_t bx, uint32_t by)
 {
+    constexpr uint32_t KB = RB;  // 32-eigenvector blocks per wave
     const uint32_t tile = (bx & 7u) * per_xcd + (bx >> 3);
-    const uint32_t per_split = (w.npad / 64u) * k_tiles;
-    if (tile >= c.nm * kProjSplits * per_split) return;
-    const uint32_t qs = tile / per_split, rest = tile - qs * per_split;
-    const uint32_t q = qs / kProjSplits, part = qs - q * kProjSplits;
-    const CeModelDev &md = c.m[q];
+    const CeBaseDev &bd = c.b[by];
+    const uint32_t ncol = c.nr * c.ndmrs, N = BaseRows(bd.nq, slots, ncol);
+    if ((N < kSmallRows) != (RB == 1)) return;  // the other form's
+    const uint32_t per_split = (N + 32u * RB - 1u) / (32u * RB) * k_tiles;
+    if (tile >= kProjSplits * per_split) return;
+    const uint32_t part = tile / per_split, rest = tile - part * per_split;
     const uint32_t kt = rest % k_tiles, nt = rest / k_tiles;
-    if (kt * kProjKTile >= md.rank) return;
+    if (kt * kProjKTile >= bd.rank) return;
     uint32_t p0, len;
-    ProjRange(md.n, part, &p0, &len);
+    ProjRange(bd.n, part, &p0, &len);
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t nb = nt * 2u + (wave & 1u);
-    const uint32_t kb0 = kt * (kProjKTile / 32u) + (wave >> 1) * 2u;
-    const uint32_t pblocks = airan::AlignUp(md.n, 16u) / 16u;
-    const uint16_t *za = w.zb + q * w.zb_stride;
-    f32x16_t acc_r[2], acc_i[2];
+    const uint32_t nb = RB == 2 ? nt * 2u + (wave & 1u) : nt;
+    const uint32_t kb0 = kt * (kProjKTile / 32u) + (RB == 2 ? (wave >> 1) * 2u : wave);
+    const uint32_t pblocks = airan::AlignUp(bd.n, 16u) / 16u;
+    const uint16_t *za = w.zb + bd.q0 * w.zb_stride;
+    f32x16_t acc_r[KB], acc_i[KB];
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (uint32_t b = 0; b < KB; ++b)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc_r[b][i] = acc_i[b][i] = 0.0f;
     const uint32_t pb_begin = p0 / 16u, pb_end = (p0 + len + 15u) / 16u;
     auto load = [&](uint32_t pb, airan::CFrag<3> &fa, airan::CFrag<3> *fb) {
         fa = airan::LoadFrag<3>(za + (static_cast<size_t>(nb) * pblocks + pb) * airan::FragBlock<3>(), lane);
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
-            fb[b] = airan::LoadFrag<3>(md.w16 + (static_cast<size_t>(kb0 + b) * pblocks + pb) * airan::FragBlock<3>(),
+        for (uint32_t b = 0; b < KB; ++b)
+            fb[b] = airan::LoadFrag<3>(bd.w16 + (static_cast<size_t>(kb0 + b) * pblocks + pb) * airan::FragBlock<3>(),
                                        lane);
     };
-    for (uint32_t pb = pb_begin; pb < pb_end; ++pb) {
-        airan::CFrag<3> fa, fb[2];
-        load(pb, fa, fb);
-        const uint4 nai[3] = {airan::NegBf16x8(fa.p[3]), airan::NegBf16x8(fa.p[4]), airan::NegBf16x8(fa.p[5])};
+    // Steps whose operands are in flight: three for RB = 1 (few workgroups, bound
+    // by latency: 9 slots of 106 PRB 8.2 us against 11.7 with two); for RB = 2 the
+    // next one's beside this one's, whose registers leave three waves per SIMD
+    // (64 slots of 273 PRB: 42 us, 46 with two steps in two register sets).
+    constexpr uint32_t kDepth = RB == 1 ? 3 : 1;
+    airan::CFrag<3> fa[kDepth], fb[kDepth][KB];
+    auto step = [&](const airan::CFrag<3> &a, const airan::CFrag<3> *b) {
+        const uint4 nai[3] = {airan::NegBf16x8(a.p[3]), airan::NegBf16x8(a.p[4]), airan::NegBf16x8(a.p[5])};
 #pragma unroll
-        for (int b = 0; b < 2; ++b) airan::CMfmaSplit<3>(acc_r[b], acc_i[b], fa, nai, fb[b]);
+        for (uint32_t i = 0; i < KB; ++i) airan::CMfmaSplit<3>(acc_r[i], acc_i[i], a, nai, b[i]);
+    };
+    if (pb_begin < pb_end) {
+#pragma unroll
+        for (uint32_t u = 0; u < kDepth; ++u) load(min(pb_begin + u, pb_end - 1u), fa[u], fb[u]);
     }
-    const uint32_t ncol = c.nr * c.ndmrs, N = slots * ncol;
-    float2 *tp = w.tp + static_cast<size_t>(part) * slots * c.nm * ncol * kMaxRank;
+    for (uint32_t pb = pb_begin; pb < pb_end; pb += kDepth) {
+        if constexpr (RB == 1) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-        const uint32_t k = (kb0 + b) * 32u + (lane & 31u);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const uint32_t n = nb * 32u + 8u * (i / 4) + 4u * (lane >> 5) + (i & 3);
-            if (n < N && k < md.rank) {
-                const uint32_t slot = n / ncol, col = n - slot * ncol;
-                tp[((static_cast<size_t>(slot) * c.nm + q) * ncol + col) * kMaxRank + k] =
-                    make_float2(acc_r[b][i], acc_i[b][i]);
+            for (uint32_t u = 0; u < kDepth; ++u) {
+                if (pb + u < pb_end) step(fa[u], fb[u]);
+                load(min(pb + u + kDepth, pb_end - 1u), fa[u], fb[u]);
             }
+        } else {
+            airan::CFrag<3> na, nf[KB];
+            load(min(pb + 1u, pb_end - 1u), na, nf);
+            step(fa[0], fb[0]);
+            fa[0] = na;
+#pragma unroll
+            for (uint32_t b = 0; b < KB; ++b) fb[0][b] = nf[b];
         }
     }
+    float2 *tp = w.tp + static_cast<size_t>(part) * slots * c.nm * ncol * kMaxRank;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const uint32_t n = nb * 32u + 8u * (i / 4) + 4u * (lane >> 5) + (i & 3);
+        if (n >= N) continue;
+        const CeRow r = RowOf(c, bd, slots, n);
+        float2 *o = tp + ((static_cast<size_t>(r.slot) * c.nm + r.q) * ncol + r.col) * kMaxRank;
+#pragma unroll
+        for (uint32_t b = 0; b < KB; ++b) {
+            const uint32_t k = (kb0 + b) * 32u + (lane & 31u);
+            if (k < bd.rank) o[k] = make_float2(acc_r[b][i], acc_i[b][i]);
+        }
+    }
+}
+__global__ void __launch_bounds__(256, 2) CeProjectSmallKernel(CeWs w, uint32_t slots, CeApply c, uint32_t k_tiles,
+                                                               uint32_t per_xcd)
+{
+    CeProjectMfmaKernelBody<1>(w, slots, c, k_tiles, per_xcd, blockIdx.x, blockIdx.y);
 }
 __global__ void __launch_bounds__(256, 2) CeProjectMfmaKernel(CeWs w, uint32_t slots, CeApply c, uint32_t k_tiles,
                                                               uint32_t per_xcd)
 {
-    CeProjectMfmaKernelBody(w, slots, c, k_tiles, per_xcd, blockIdx.x, blockIdx.y);
+    CeProjectMfmaKernelBody<2>(w, slots, c, k_tiles, per_xcd, blockIdx.x, blockIdx.y);
 }
 
 // Column energies: |z|^2 over the observations and |u|^2 over the kept
@@ -437,7 +508,7 @@ __global__ void __launch_bounds__(256, 2) CeProjectMfmaKernel(CeWs w, uint32_t s
 // in split order, and t is stored for the kernels after.  Grid
 // slots * models * NR*D.
 __device__ __forceinline__ void CeEnergyKernelBody(const __half *__restrict__ hr, const __half *__restrict__ hi,
-                                                      const CeWs &w, const CeApply &c, uint32_t slots, uint32_t bx, uint32_t by)
+                                                      const CeWs &w, const CeApply &c, uint32_t slots, uint32_t bx)
 {
     __shared__ double red[2][4];
     const uint32_t ncol = c.nr * c.ndmrs;
@@ -445,15 +516,13 @@ __device__ __forceinline__ void CeEnergyKernelBody(const __half *__restrict__ hr
     const uint32_t col = b % ncol, sq = b / ncol;
     const uint32_t q = sq % c.nm, slot = sq / c.nm;
     const CeModelDev &md = c.m[q];
+    const CeBaseDev &bd = c.b[md.base];
     double ez = 0.0, eu = 0.0;
-    for (uint32_t p = threadIdx.x; p < md.n; p += blockDim.x) {
-        const float2 v = LoadZ(hr, hi, c, md, slot, col, p);
-        ez += static_cast<double>(v.x) * v.x + static_cast<double>(v.y) * v.y;
-    }
     const size_t total = static_cast<size_t>(slots) * c.nm * kMaxRank * ncol;
     const size_t e0 = (static_cast<size_t>(sq) * ncol + col) * kMaxRank;
-    for (uint32_t k = threadIdx.x; k < md.rank; k += blockDim.x) {
+    for (uint32_t k = threadIdx.x; k < bd.rank; k += blockDim.x) {
         float2 u = w.tp[e0 + k];
+#pragma unroll
         for (uint32_t part = 1; part < kProjSplits; ++part) {
             const float2 v = w.tp[static_cast<size_t>(part) * total + e0 + k];
             u.x += v.x;
@@ -461,6 +530,10 @@ __device__ __forceinline__ void CeEnergyKernelBody(const __half *__restrict__ hr
         }
         w.t[e0 + k] = u;
         eu += static_cast<double>(u.x) * u.x + static_cast<double>(u.y) * u.y;
+    }
+    for (uint32_t p = threadIdx.x; p < bd.n; p += blockDim.x) {
+        const float2 v = LoadZ(hr, hi, c, md, bd.n, slot, col, p);
+        ez += static_cast<double>(v.x) * v.x + static_cast<double>(v.y) * v.y;
     }
     for (int off = 32; off > 0; off >>= 1) {
         ez += __shfl_xor(ez, off);
@@ -480,11 +553,11 @@ __device__ __forceinline__ void CeEnergyKernelBody(const __half *__restrict__ hr
 __global__ void __launch_bounds__(256) CeEnergyKernel(const __half *__restrict__ hr, const __half *__restrict__ hi,
                                                       CeWs w, CeApply c, uint32_t slots)
 {
-    CeEnergyKernelBody(hr, hi, w, c, slots, blockIdx.x, blockIdx.y);
+    CeEnergyKernelBody(hr, hi, w, c, slots, blockIdx.x);
 }
 
-// Noise and per-model statistics of one slot (thread 0, fp64, fixed order),
-// then inv[slot, q][k] = 1 / (lam_k + n_q) by all threads.
+// Noise and per-model statistics of one slot, then its scaled columns.
+//
 // Every observation z carries the per-RE noise sigma^2 (comb: y r*; FD-OCC
 // pair: h_ls0 +- h_ls1, each the mean of two).  The noise lies in the
 // complement of the kept eigenspace: per Rx, sigma^2 = sum_{q,d} (|z|^2 -
@@ -492,88 +565,123 @@ __global__ void __launch_bounds__(256) CeEnergyKernel(const __half *__restrict__
 // which the channel's frequency selectivity inflates, is the fallback below
 // kMinNoiseDims dimensions.  P_q = mean |z|^2 - sigma^2 and the filter's
 // relative noise n_q = sigma^2 / P_q -> stats[4 slot + q];
-// noise_out[slot][rx] = fp16(sigma^2_rx) when non-null.
-__device__ __forceinline__ void CeStatsKernelBody(const __half *__restrict__ noise_in,
-                                                     __half *__restrict__ noise_out, const CeWs &w, const CeApply &c, uint32_t bx, uint32_t by)
+// noise_out[slot][rx] = fp16(sigma^2_rx) when non-null.  inv[slot, q][k] =
+// 1 / (lam_k + n_q) and tb = t inv in 2-part fragment planes, 8 eigenvectors
+// per thread.
+//
+// A workgroup per slot and kScaleRank eigenvectors: each forms the slot's
+// statistics itself (a lane per antenna, a wave per model; fp64, fixed order),
+// so that they need no launch of their own; the first stores them.  64 slots,
+// 4 Rx, 273 PRB 11 us (19 in two launches, the
+// statistics being one thread's serial sums), 23 slots of 64 Rx, 133 PRB
+// 43 against 120.
+constexpr uint32_t kScaleRank = 64;
+constexpr uint32_t kScaleParts = kMaxRank / kScaleRank;
+constexpr uint32_t kMaxCols = 64 * 4;  // NR * D
+__device__ __forceinline__ void CeScaleKernelBody(const __half *__restrict__ noise_in, __half *__restrict__ noise_out,
+                                                     const CeWs &w, const CeApply &c, uint32_t slots, uint32_t bx)
 {
+    __shared__ double energy[kMaxModels * kMaxCols * 2];
+    __shared__ double s2rx[64], eh[kMaxModels];
     __shared__ float nq[kMaxModels];
-    // The slot's energies staged in LDS by all threads, so thread 0's serial
-    // sums read LDS instead of waiting on one global load at a time.
-    constexpr uint32_t kStage = 2 * kMaxModels * 32;
-    __shared__ double stage[kStage];
-    const uint32_t slot = bx;
-    const uint32_t ncol = c.nr * c.ndmrs;
-    const uint32_t n_e = 2 * c.nm * ncol;
-    const double *eg = w.energy + 2 * static_cast<size_t>(slot) * c.nm * ncol;
-    if (n_e <= kStage) {
-        for (uint32_t t = threadIdx.x; t < n_e; t += blockDim.x) stage[t] = eg[t];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        const double *e = n_e <= kStage ? stage : eg;
+    const uint32_t slot = bx / kScaleParts, part = bx - slot * kScaleParts;
+    uint32_t max_rank = 0;
+    for (uint32_t b = 0; b < c.nb; ++b) max_rank = max(max_rank, c.b[b].rank);
+    if (part * kScaleRank >= max_rank) return;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t ncol = c.nr * c.ndmrs, ncols = c.nm * ncol;
+    const double *eg = w.energy + 2 * static_cast<size_t>(slot) * ncols;
+    for (uint32_t t = threadIdx.x; t < 2 * ncols; t += blockDim.x) energy[t] = eg[t];
+    __syncthreads();
+    if (wave == 0 && lane < c.nr) {
+        const uint32_t rx = lane;
         double dims = 0.0;
-        for (uint32_t q = 0; q < c.nm; ++q) dims += static_cast<double>(c.m[q].n - c.m[q].kept) * c.ndmrs;
-        double s2_sum = 0.0;
-        for (uint32_t rx = 0; rx < c.nr; ++rx) {
-            double s2;
-            if (dims >= kMinNoiseDims) {
-                double res = 0.0;
-                for (uint32_t q = 0; q < c.nm; ++q)
-                    for (uint32_t d = 0; d < c.ndmrs; ++d) {
-                        const double *x = e + 2 * (static_cast<size_t>(q) * ncol + rx * c.ndmrs + d);
-                        res += fmax(x[0] - x[1], 0.0);
-                    }
-                s2 = res / dims;
-            } else {
-                s2 = __half2float(noise_in[static_cast<size_t>(slot) * c.nr + rx]);
-            }
-            if (noise_out) noise_out[static_cast<size_t>(slot) * c.nr + rx] = __float2half_rn(static_cast<float>(s2));
-            s2_sum += s2;
+        for (uint32_t q = 0; q < c.nm; ++q)
+            dims += static_cast<double>(c.b[c.m[q].base].n - c.b[c.m[q].base].kept) * c.ndmrs;
+        double s2;
+        if (dims >= kMinNoiseDims) {
+            double res = 0.0;
+            for (uint32_t q = 0; q < c.nm; ++q)
+                for (uint32_t d = 0; d < c.ndmrs; ++d) {
+                    const double *x = energy + 2 * (q * ncol + rx * c.ndmrs + d);
+                    res += fmax(x[0] - x[1], 0.0);
+                }
+            s2 = res / dims;
+        } else {
+            s2 = __half2float(noise_in[static_cast<size_t>(slot) * c.nr + rx]);
         }
-        const double s2 = s2_sum / c.nr;
-        for (uint32_t q = 0; q < c.nm; ++q) {
-            double eh = 0.0;
-            for (uint32_t col = 0; col < ncol; ++col) eh += e[2 * (static_cast<size_t>(q) * ncol + col)];
-            const double mean = eh / (static_cast<double>(ncol) * c.m[q].n);
-            const double p = fmax(mean - s2, 1e-3 * mean + 1e-30);
-            const float v = static_cast<float>(s2 / p);
-            w.stats[4 * slot + q] = v;
-            nq[q] = v;
-        }
+        if (noise_out && part == 0)
+            noise_out[static_cast<size_t>(slot) * c.nr + rx] = __float2half_rn(static_cast<float>(s2));
+        s2rx[rx] = s2;
+    }
+    if (wave < c.nm) {
+        double s = 0.0;
+        for (uint32_t col = lane; col < ncol; col += 64) s += energy[2 * (wave * ncol + col)];
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+        if (lane == 0) eh[wave] = s;
     }
     __syncthreads();
-    for (uint32_t q = 0; q < c.nm; ++q)
-        for (uint32_t k = threadIdx.x; k < c.m[q].rank; k += blockDim.x)
-            w.inv[(static_cast<size_t>(slot) * c.nm + q) * kMaxRank + k] = 1.0f / (c.m[q].lam[k] + nq[q]);
+    if (threadIdx.x < c.nm) {
+        const uint32_t q = threadIdx.x;
+        double s2_sum = 0.0;
+        for (uint32_t rx = 0; rx < c.nr; ++rx) s2_sum += s2rx[rx];
+        const double s2 = s2_sum / c.nr;
+        const double mean = eh[q] / (static_cast<double>(ncol) * c.b[c.m[q].base].n);
+        const double p = fmax(mean - s2, 1e-3 * mean + 1e-30);
+        const float v = static_cast<float>(s2 / p);
+        if (part == 0) w.stats[4 * slot + q] = v;
+        nq[q] = v;
+    }
+    __syncthreads();
+    // Columns fastest: the lanes of a model's columns write adjacent rows of
+    // the fragment planes.
+    for (uint32_t e = threadIdx.x; e < ncols * (kScaleRank / 8u); e += blockDim.x) {
+        const uint32_t i = e % ncols, k0 = part * kScaleRank + e / ncols * 8u;
+        const uint32_t q = i / ncol, col = i - q * ncol;
+        const CeBaseDev &bd = c.b[c.m[q].base];
+        if (k0 >= bd.rank) continue;
+        const size_t sq = static_cast<size_t>(slot) * c.nm + q;
+        float2 v[8];
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) {
+            const float2 x = w.t[(sq * ncol + col) * kMaxRank + k0 + j];
+            const float s = 1.0f / (bd.lam[k0 + j] + nq[q]);
+            if (col == 0) w.inv[sq * kMaxRank + k0 + j] = s;
+            v[j] = make_float2(x.x * s, x.y * s);
+        }
+        airan::StoreFrag8<2>(w.tb + bd.q0 * TbModelElems(w.npad), ((q - bd.q0) * slots + slot) * ncol + col, k0,
+                             bd.rank / 16u, v);
+    }
 }
-__global__ void __launch_bounds__(256) CeStatsKernel(const __half *__restrict__ noise_in,
-                                                     __half *__restrict__ noise_out, CeWs w, CeApply c)
+__global__ void __launch_bounds__(256) CeScaleKernel(const __half *__restrict__ noise_in, __half *__restrict__ noise_out,
+                                                     CeWs w, CeApply c, uint32_t slots)
 {
-    CeStatsKernelBody(noise_in, noise_out, w, c, blockIdx.x, blockIdx.y);
+    CeScaleKernelBody(noise_in, noise_out, w, c, slots, blockIdx.x);
 }
 
 // hhat_var[slot, q][sc] = sum_k |A[k][sc]|^2 / (lam_k + n_q) (ref.py:109-111)
 // on fp32 MFMA (v_mfma_f32_32x32x2f32, exact fp32 products): a workgroup per
-// 32 slots x 32 subcarriers of one model, its four waves taking fixed
+// 32 rows x 32 columns of one base, its four waves taking fixed
 // quarters of the rank (in steps of 16) and their partial sums added in
-// wave order.  Lane l takes A[slot l % 32][k + l / 32] = 1 / (lam + n) and
-// B[k + l / 32][sc l % 32] = |A|^2; accumulator i holds slot
-// 8 (i / 4) + 4 (l / 32) + i % 4.  Rows past `slots` and subcarriers past
-// `used` read clamped (valid) addresses and are not stored.  Grid: slot
-// tiles fastest (they share the |A|^2 tile), then subcarrier tiles, then
-// models.
-__device__ __forceinline__ void CeHvMfmaKernelBody(const CeWs &w, uint32_t slots, const CeApply &c, uint32_t slot_tiles,
-                                                      uint32_t sc_tiles, uint32_t bx, uint32_t by)
+// wave order.  Lane l takes A[row l % 32][k + l / 32] = 1 / (lam + n) and
+// B[k + l / 32][column l % 32] = |A|^2; accumulator i holds row
+// 8 (i / 4) + 4 (l / 32) + i % 4.  A base's (model, slot) pairs are the rows,
+// its rows r = sc + shift the columns; rows and columns past the last read
+// clamped (valid) addresses and are not stored.  Grid: row tiles fastest (they
+// share the |A|^2 tile), then column tiles; y: bases.
+__device__ __forceinline__ void CeHvMfmaKernelBody(const CeWs &w, uint32_t slots, const CeApply &c, uint32_t bx, uint32_t by)
 {
     __shared__ float part[3][16][64];
-    const uint32_t st = bx % slot_tiles, rest = bx / slot_tiles;
-    const uint32_t ct = rest % sc_tiles, q = rest / sc_tiles;
-    const CeModelDev &md = c.m[q];
+    const CeBaseDev &bd = c.b[by];
+    const uint32_t pairs = bd.nq * slots, row_tiles = (pairs + 31u) / 32u;
+    const uint32_t st = bx % row_tiles, ct = bx / row_tiles;
+    if (ct * 32u >= bd.rows) return;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, r = lane & 31u, kh = lane >> 5;
-    const uint32_t slot = min(st * 32u + r, slots - 1u), sc = min(ct * 32u + r, c.used - 1u);
-    const float *ia = w.inv + (static_cast<size_t>(slot) * c.nm + q) * kMaxRank + kh;
-    const float *ba = md.a2 + static_cast<size_t>(kh) * c.used + sc;
-    const uint32_t steps = md.rank / 16u;
+    const uint32_t pr = min(st * 32u + r, pairs - 1u), col = ct * 32u + r, cc = min(col, bd.rows - 1u);
+    const uint32_t mi = pr / slots;
+    const float *ia = w.inv + (static_cast<size_t>(pr - mi * slots) * c.nm + bd.q0 + mi) * kMaxRank + kh;
+    const float *ba = bd.a2 + static_cast<size_t>(kh) * bd.rows + cc;
+    const uint32_t steps = bd.rank / 16u;
     f32x16_t acc;
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
@@ -582,7 +690,7 @@ __device__ __forceinline__ void CeHvMfmaKernelBody(const CeWs &w, uint32_t slots
 #pragma unroll
         for (uint32_t u = 0; u < 8; ++u) {
             av[u] = ia[k0 + 2u * u];
-            bv[u] = ba[static_cast<size_t>(k0 + 2u * u) * c.used];
+            bv[u] = ba[static_cast<size_t>(k0 + 2u * u) * bd.rows];
         }
 #pragma unroll
         for (uint32_t u = 0; u < 8; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[u], bv[u], acc, 0, 0, 0);
@@ -595,56 +703,23 @@ __device__ __forceinline__ void CeHvMfmaKernelBody(const CeWs &w, uint32_t slots
     if (wave > 0) return;
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = ((acc[i] + part[0][i][lane]) + part[1][i][lane]) + part[2][i][lane];
-    const uint32_t col = ct * 32u + r;
-    if (col >= c.used) return;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-        const uint32_t s = st * 32u + 8u * (i / 4) + 4u * kh + (i & 3);
-        if (s < slots) w.hv[(static_cast<size_t>(s) * c.nm + q) * c.used + col] = acc[i];
+        const uint32_t p = st * 32u + 8u * (i / 4) + 4u * kh + (i & 3);
+        if (p >= pairs) continue;
+        const uint32_t m = p / slots, q = bd.q0 + m, sc = col - c.m[q].shift;  // wraps below zero
+        if (sc < c.used) w.hv[(static_cast<size_t>(p - m * slots) * c.nm + q) * c.used + sc] = acc[i];
     }
 }
-__global__ void __launch_bounds__(256) CeHvMfmaKernel(CeWs w, uint32_t slots, CeApply c, uint32_t slot_tiles,
-                                                      uint32_t sc_tiles)
+__global__ void __launch_bounds__(256) CeHvMfmaKernel(CeWs w, uint32_t slots, CeApply c)
 {
-    CeHvMfmaKernelBody(w, slots, c, slot_tiles, sc_tiles, blockIdx.x, blockIdx.y);
-}
-
-// tb[q] = t[slot, q][col][k] / (lam_k + n_q) in 2-part fragment planes, row
-// n = slot * NR*D + col (zero for n >= slots * NR*D), one thread per row and
-// 8 eigenvectors.  Grid (npad * kMaxRank / 8 / 256, models).
-__device__ __forceinline__ void CeScaleSplitKernelBody(const CeWs &w, uint32_t slots, const CeApply &c, uint32_t bx, uint32_t by)
-{
-    const uint32_t q = by;
-    const CeModelDev &md = c.m[q];
-    const uint32_t e = bx * blockDim.x + threadIdx.x;
-    const uint32_t n = e % w.npad, k0 = (e / w.npad) * 8u;
-    if (k0 >= md.rank) return;
-    const uint32_t ncol = c.nr * c.ndmrs;
-    float2 v[8];
-    if (n < slots * ncol) {
-        const uint32_t slot = n / ncol, col = n - slot * ncol;
-        const size_t sq = static_cast<size_t>(slot) * c.nm + q;
-#pragma unroll
-        for (uint32_t j = 0; j < 8; ++j) {
-            const float2 x = w.t[(sq * ncol + col) * kMaxRank + k0 + j];
-            const float s = w.inv[sq * kMaxRank + k0 + j];
-            v[j] = make_float2(x.x * s, x.y * s);
-        }
-    } else {
-#pragma unroll
-        for (uint32_t j = 0; j < 8; ++j) v[j] = make_float2(0.0f, 0.0f);
-    }
-    airan::StoreFrag8<2>(w.tb + q * TbModelElems(w.npad), n, k0, md.rank / 16u, v);
-}
-__global__ void __launch_bounds__(256) CeScaleSplitKernel(CeWs w, uint32_t slots, CeApply c)
-{
-    CeScaleSplitKernelBody(w, slots, c, blockIdx.x, blockIdx.y);
+    CeHvMfmaKernelBody(w, slots, c, blockIdx.x, blockIdx.y);
 }
 
 // hf[slot, q][col][sc] = sum_k (t[slot, q][col][k] / (lam_k + n_q)) A[k][sc]
-// on split bf16 MFMA with 2 parts: C = TB A^T with rows n (slot, col) and
-// columns sc.  Workgroup: a kInterpTile x kInterpTile tile of one model, four
-// waves of 64 x 64 (2 x 2 blocks of 32 x 32).  Per K-step of 16 the tile's
+// on split bf16 MFMA with 2 parts: C = TB A^T with a base's rows n (RowOf) and
+// columns r = sc + shift.  Workgroup: a kInterpTile x kInterpTile tile of one
+// base, four waves of 64 x 64 (2 x 2 blocks of 32 x 32).  Per K-step of 16 the tile's
 // 4 row blocks and 4 subcarrier blocks (32 planes of 1 KB) are copied to
 // LDS by the direct global -> LDS path, double-buffered: the next step's
 // copies are in flight while this step's MFMAs run, and every fragment is
@@ -653,22 +728,23 @@ __global__ void __launch_bounds__(256) CeScaleSplitKernel(CeWs w, uint32_t slots
 // range of tiles with the row tiles of one subcarrier tile adjacent: the
 // subcarrier-side operand is read once per XCD, the small row-side operand
 // stays in every L2.  Linear grid of 8 * per_xcd.
-__device__ __forceinline__ void CeInterpMfmaKernelBody(const CeWs &w, uint32_t slots, const CeApply &c, uint32_t sc_tiles,
-                                                          uint32_t per_xcd, uint32_t bx, uint32_t by)
+__device__ __forceinline__ void CeInterpMfmaKernelBody(const CeWs &w, uint32_t slots, const CeApply &c, uint32_t per_xcd,
+                                                          uint32_t bx, uint32_t by)
 {
     __shared__ uint4 stage[2][8][4][64];  // [buffer][block: 4 row, 4 subcarrier][plane][lane]
-    const uint32_t xcd = bx & 7u, j = bx >> 3;
-    const uint32_t n_tiles = w.npad / kInterpTile;
-    const uint32_t tile = xcd * per_xcd + j;
-    if (tile >= c.nm * sc_tiles * n_tiles) return;
-    const uint32_t nt = tile % n_tiles, rest = tile / n_tiles;
-    const uint32_t st = rest % sc_tiles, q = rest / sc_tiles;
-    const CeModelDev &md = c.m[q];
+    const CeBaseDev &bd = c.b[by];
+    const uint32_t ncol = c.nr * c.ndmrs, N = BaseRows(bd.nq, slots, ncol);
+    if (N < kSmallRows) return;  // the 32-row form's
+    const uint32_t n_tiles = (N + kInterpTile - 1u) / kInterpTile;
+    const uint32_t sc_tiles = (bd.rows + kInterpTile - 1u) / kInterpTile;
+    const uint32_t tile = (bx & 7u) * per_xcd + (bx >> 3);
+    if (tile >= sc_tiles * n_tiles) return;
+    const uint32_t nt = tile % n_tiles, st = tile / n_tiles;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t nrow0 = (nt * kInterpTile) / 32u, nsc0 = (st * kInterpTile) / 32u;
     const uint32_t nb0 = nrow0 + (wave & 1u) * 2u, sb0 = nsc0 + (wave >> 1) * 2u;
-    const uint32_t kb_count = md.rank / 16u;
-    const uint16_t *ta = w.tb + q * TbModelElems(w.npad);
+    const uint32_t kb_count = bd.rank / 16u;
+    const uint16_t *ta = w.tb + bd.q0 * TbModelElems(w.npad);
     f32x16_t acc_r[2][2], acc_i[2][2];
 #pragma unroll
     for (int a = 0; a < 2; ++a)
@@ -684,7 +760,7 @@ __device__ __forceinline__ void CeInterpMfmaKernelBody(const CeWs &w, uint32_t s
             const uint32_t g = 2u * wave + jb;
             const uint16_t *src =
                 g < 4u ? ta + (static_cast<size_t>(nrow0 + g) * kb_count + kb) * airan::FragBlock<2>()
-                       : md.a16 + (static_cast<size_t>(nsc0 + g - 4u) * kb_count + kb) * airan::FragBlock<2>();
+                       : bd.a16 + (static_cast<size_t>(nsc0 + g - 4u) * kb_count + kb) * airan::FragBlock<2>();
 #pragma unroll
             for (uint32_t p = 0; p < 4; ++p) airan::PlaneToLds(src + p * airan::kFragPlane, &stage[buf][g][p][0], lane);
         }
@@ -715,27 +791,86 @@ __device__ __forceinline__ void CeInterpMfmaKernelBody(const CeWs &w, uint32_t s
         }
         __syncthreads();  // buffer cur is refilled by the next step's copies
     }
-    const uint32_t ncol = c.nr * c.ndmrs, N = slots * ncol;
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-            const uint32_t sc = (sb0 + b) * 32u + (lane & 31u);
+        for (int i = 0; i < 16; ++i) {
+            const uint32_t n = (nb0 + a) * 32u + 8u * (i / 4) + 4u * (lane >> 5) + (i & 3);
+            if (n >= N) continue;
+            const CeRow r = RowOf(c, bd, slots, n);
+            float2 *o = w.hf + ((static_cast<size_t>(r.slot) * c.nm + r.q) * ncol + r.col) * c.used;
+            const uint32_t shift = c.m[r.q].shift;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const uint32_t n = (nb0 + a) * 32u + 8u * (i / 4) + 4u * (lane >> 5) + (i & 3);
-                if (n < N && sc < c.used) {
-                    const uint32_t slot = n / ncol, col = n - slot * ncol;
-                    w.hf[((static_cast<size_t>(slot) * c.nm + q) * ncol + col) * c.used + sc] =
-                        make_float2(acc_r[a][b][i], acc_i[a][b][i]);
-                }
+            for (int b = 0; b < 2; ++b) {
+                const uint32_t sc = (sb0 + b) * 32u + (lane & 31u) - shift;  // wraps below zero
+                if (sc < c.used) o[sc] = make_float2(acc_r[a][b][i], acc_i[a][b][i]);
             }
         }
 }
-__global__ void __launch_bounds__(256, 2) CeInterpMfmaKernel(CeWs w, uint32_t slots, CeApply c, uint32_t sc_tiles,
-                                                          uint32_t per_xcd)
+__global__ void __launch_bounds__(256, 2) CeInterpMfmaKernel(CeWs w, uint32_t slots, CeApply c, uint32_t per_xcd)
 {
-    CeInterpMfmaKernelBody(w, slots, c, sc_tiles, per_xcd, blockIdx.x, blockIdx.y);
+    CeInterpMfmaKernelBody(w, slots, c, per_xcd, blockIdx.x, blockIdx.y);
+}
+
+// The same product for a base of few rows (below kSmallRows: a slot or a few,
+// the shapes of a ragged batch): workgroup 32 rows x kInterpTile columns, a
+// wave per 32 x 32 block with its operands straight from memory, three K-steps
+// in flight.  Every element is the same ordered sum as in the 128-row form.
+// One 273-PRB slot (32 rows) 15 us against 38 of 128-row tiles, 96
+// ragged grants 162 against 548 (a 128-row tile per 8 columns and model,
+// and four copies of the filter).
+__device__ __forceinline__ void CeInterpSmallKernelBody(const CeWs &w, uint32_t slots, const CeApply &c, uint32_t per_xcd,
+                                                           uint32_t bx, uint32_t by)
+{
+    const CeBaseDev &bd = c.b[by];
+    const uint32_t ncol = c.nr * c.ndmrs, N = BaseRows(bd.nq, slots, ncol);
+    if (N >= kSmallRows) return;  // the 128-row form's
+    const uint32_t n_tiles = (N + 31u) / 32u, sc_tiles = (bd.rows + kInterpTile - 1u) / kInterpTile;
+    const uint32_t tile = (bx & 7u) * per_xcd + (bx >> 3);
+    if (tile >= sc_tiles * n_tiles) return;
+    const uint32_t nb = tile % n_tiles, st = tile / n_tiles;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t sb = st * (kInterpTile / 32u) + wave;
+    const uint32_t kb_count = bd.rank / 16u;
+    const uint16_t *ta = w.tb + bd.q0 * TbModelElems(w.npad) +
+                         static_cast<size_t>(nb) * kb_count * airan::FragBlock<2>();
+    const uint16_t *aa = bd.a16 + static_cast<size_t>(sb) * kb_count * airan::FragBlock<2>();
+    f32x16_t acc_r, acc_i;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc_r[i] = acc_i[i] = 0.0f;
+    constexpr uint32_t kDepth = 3;
+    airan::CFrag<2> fa[kDepth], fb[kDepth];
+    auto load = [&](uint32_t kb, uint32_t u) {
+        const uint32_t k = min(kb, kb_count - 1u);
+        fa[u] = airan::LoadFrag<2>(ta + static_cast<size_t>(k) * airan::FragBlock<2>(), lane);
+        fb[u] = airan::LoadFrag<2>(aa + static_cast<size_t>(k) * airan::FragBlock<2>(), lane);
+    };
+#pragma unroll
+    for (uint32_t u = 0; u < kDepth; ++u) load(u, u);
+    for (uint32_t kb = 0; kb < kb_count; kb += kDepth) {
+#pragma unroll
+        for (uint32_t u = 0; u < kDepth; ++u) {
+            if (kb + u < kb_count) {
+                const uint4 nai[2] = {airan::NegBf16x8(fa[u].p[2]), airan::NegBf16x8(fa[u].p[3])};
+                airan::CMfmaSplit<2>(acc_r, acc_i, fa[u], nai, fb[u]);
+            }
+            load(kb + u + kDepth, u);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const uint32_t n = nb * 32u + 8u * (i / 4) + 4u * (lane >> 5) + (i & 3);
+        if (n >= N) continue;
+        const CeRow r = RowOf(c, bd, slots, n);
+        const uint32_t sc = sb * 32u + (lane & 31u) - c.m[r.q].shift;  // wraps below zero
+        if (sc < c.used)
+            w.hf[((static_cast<size_t>(r.slot) * c.nm + r.q) * ncol + r.col) * c.used + sc] =
+                make_float2(acc_r[i], acc_i[i]);
+    }
+}
+__global__ void __launch_bounds__(256) CeInterpSmallKernel(CeWs w, uint32_t slots, CeApply c, uint32_t per_xcd)
+{
+    CeInterpSmallKernelBody(w, slots, c, per_xcd, blockIdx.x, blockIdx.y);
 }
 
 // (R_tt + e I) for D DMRS symbols, eliminated once (no pivoting; the matrix
@@ -795,22 +930,29 @@ __device__ inline void Rescale(float hv, float *scale, float *err2)
     *err2 = fmaxf(s * (s - 1.0f) * hv + (1.0f - s) + s * err, 0.0f);
 }
 
+constexpr uint32_t kPostRx = 8;
+
 // Rescale (per model), pair combination h = (g_a + sign g_b) / 2 with
 // relative error (err_a + err_b) / 2, and time interpolation over the D DMRS
-// symbols.  One thread per subcarrier of one (slot, layer) = blockIdx.y.
-// Writes H[slot][rx][l][sym][sc] fp16 for sc < pad (zero beyond used).
+// symbols.  One thread per subcarrier of one (slot, layer, kPostRx receive
+// antennas) = blockIdx.y.  Writes H[slot][rx][l][sym][sc] fp16 for sc < pad
+// (zero beyond used).  Bound by the writes: 64 slots, 4 Rx, 273 PRB 312 MB in 60
+// us; 23 slots, 64 Rx, 133 PRB 185 us, where one thread for all antennas
+// left 2.5 workgroups per CU and took 307.
 template <int D>
 __device__ __forceinline__ void CePostKernelBody(const CeWs &w, __half *__restrict__ out_r, __half *__restrict__ out_i,
                                                     uint32_t out_layers, const CeApply &c, uint32_t bx, uint32_t by)
 {
     const uint32_t sc = bx * blockDim.x + threadIdx.x;
-    const uint32_t slot = by / c.nl, l = by - slot * c.nl;
+    const uint32_t chunks = (c.nr + kPostRx - 1u) / kPostRx, sl = by / chunks;
+    const uint32_t rx0 = (by - sl * chunks) * kPostRx, rx1 = min(c.nr, rx0 + kPostRx);
+    const uint32_t slot = sl / c.nl, l = sl - slot * c.nl;
     if (sc >= c.pad) return;
     const size_t plane = static_cast<size_t>(c.nsym) * c.pad;
     out_r += static_cast<size_t>(slot) * c.nr * out_layers * plane;
     out_i += static_cast<size_t>(slot) * c.nr * out_layers * plane;
     if (sc >= c.used) {
-        for (uint32_t rx = 0; rx < c.nr; ++rx)
+        for (uint32_t rx = rx0; rx < rx1; ++rx)
             for (uint32_t s = 0; s < c.nsym; ++s) {
                 const size_t o = (static_cast<size_t>(rx) * out_layers + l) * plane + static_cast<size_t>(s) * c.pad + sc;
                 out_r[o] = __ushort_as_half(0);
@@ -839,7 +981,7 @@ __device__ __forceinline__ void CePostKernelBody(const CeWs &w, __half *__restri
 #pragma unroll
     for (uint32_t s = 0; s < 14; ++s)
         if (s < c.nsym) ts.Solve(c.rt[s], tw[s]);
-    for (uint32_t rx = 0; rx < c.nr; ++rx) {
+    for (uint32_t rx = rx0; rx < rx1; ++rx) {
         float2 hf[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) {
@@ -881,19 +1023,19 @@ void FreeDev(void *p)
     if (p != nullptr) (void)hipFree(p);
 }
 
-// Eigen-factors of one observation model (FP64 on the device).
-int32_t BuildModel(const Geom &g, const LmmseFilterParamsV1 &prm, hipStream_t stream, CeModelFactors *out)
+// Eigen-factors of one base (FP64 on the device).
+int32_t BuildBase(const LmmseFilterParamsV1 &prm, hipStream_t stream, CeBaseFactors *out)
 {
     ObsGeom o{};
     o.n = out->n;
     o.step = out->step;
-    o.offset = out->offset;
-    o.used = g.used;
+    o.used = out->rows - out->max_off;
     o.scs_tau = prm.scs_hz * prm.tau_s;
-    const uint32_t n = o.n;
+    const uint32_t n = o.n, rows = out->rows, used = o.used;
     if (n == 0 || n > kMaxObs) return AIRAN_UNSUPPORTED_PROFILE;
     double2 *rpp = nullptr, *rhp = nullptr, *av = nullptr;
     float2 *at = nullptr;  // (R_hp U) transposed, [rank][used], packed into a16 / a2
+    float2 *bt = nullptr;  // conj(U), [n][rank], packed into w16
     double *eig = nullptr, *work = nullptr;
     rocblas_int *info = nullptr;
     rocblas_handle handle = nullptr;
@@ -905,6 +1047,7 @@ int32_t BuildModel(const Geom &g, const LmmseFilterParamsV1 &prm, hipStream_t st
         FreeDev(rhp);
         FreeDev(av);
         FreeDev(at);
+        FreeDev(bt);
         FreeDev(eig);
         FreeDev(work);
         FreeDev(info);
@@ -914,12 +1057,11 @@ int32_t BuildModel(const Geom &g, const LmmseFilterParamsV1 &prm, hipStream_t st
         return AIRAN_LAUNCH_FAILED;
     };
     if (hipMalloc(&rpp, sizeof(double2) * n * n) != hipSuccess ||
-        hipMalloc(&rhp, sizeof(double2) * static_cast<size_t>(g.used) * n) != hipSuccess ||
+        hipMalloc(&rhp, sizeof(double2) * static_cast<size_t>(used) * n) != hipSuccess ||
         hipMalloc(&eig, sizeof(double) * n) != hipSuccess || hipMalloc(&work, sizeof(double) * n) != hipSuccess ||
         hipMalloc(&info, sizeof(rocblas_int)) != hipSuccess)
         return fail();
     hipLaunchKernelGGL(BuildRppKernel, dim3(airan::CeilDiv(n, 256), n), dim3(256), 0, stream, rpp, o);
-    hipLaunchKernelGGL(BuildRhpKernel, dim3(airan::CeilDiv(g.used, 256), n), dim3(256), 0, stream, rhp, o);
     if (!CheckRocblas(rocblas_create_handle(&handle)) || !CheckRocblas(rocblas_set_stream(handle, stream)))
         return fail();
     if (!CheckRocblas(rocsolver_zheevd(handle, rocblas_evect_original, rocblas_fill_lower,
@@ -938,37 +1080,47 @@ int32_t BuildModel(const Geom &g, const LmmseFilterParamsV1 &prm, hipStream_t st
     }
     kept = std::max<uint32_t>(kept, 1);
     const uint32_t rank = airan::AlignUp(kept, 16);
-    // av = R_hp (used x n) * V[:, n-kept .. n-1] (n x kept), column-major.
-    if (hipMalloc(&av, sizeof(double2) * static_cast<size_t>(g.used) * kept) != hipSuccess) return fail();
-    const rocblas_double_complex one{1.0, 0.0}, zero{0.0, 0.0};
-    if (!CheckRocblas(rocblas_zgemm(handle, rocblas_operation_none, rocblas_operation_none,
-                                    static_cast<rocblas_int>(g.used), static_cast<rocblas_int>(kept),
-                                    static_cast<rocblas_int>(n), &one,
-                                    reinterpret_cast<const rocblas_double_complex *>(rhp),
-                                    static_cast<rocblas_int>(g.used),
-                                    reinterpret_cast<const rocblas_double_complex *>(rpp) + static_cast<size_t>(n - kept) * n,
-                                    static_cast<rocblas_int>(n), &zero,
-                                    reinterpret_cast<rocblas_double_complex *>(av),
-                                    static_cast<rocblas_int>(g.used))))
+    if (hipMalloc(&av, sizeof(double2) * static_cast<size_t>(used) * kept) != hipSuccess ||
+        hipMalloc(&at, sizeof(float2) * static_cast<size_t>(rank) * rows) != hipSuccess)
         return fail();
+    // av = R_hp (used x n) * V[:, n-kept .. n-1] (n x kept), column-major, for
+    // the largest offset (rows 0 .. used - 1) and for offset 0 (the rest: its
+    // last subcarriers), each the product that a model of that offset has, so
+    // that a model's values do not depend on what it shares the base with.
+    const rocblas_double_complex one{1.0, 0.0}, zero{0.0, 0.0};
+    for (uint32_t pass = 0; pass < (out->max_off > 0 ? 2u : 1u); ++pass) {
+        o.offset = pass == 0 ? out->max_off : 0u;
+        hipLaunchKernelGGL(BuildRhpKernel, dim3(airan::CeilDiv(used, 256), n), dim3(256), 0, stream, rhp, o);
+        if (!CheckRocblas(rocblas_zgemm(handle, rocblas_operation_none, rocblas_operation_none,
+                                        static_cast<rocblas_int>(used), static_cast<rocblas_int>(kept),
+                                        static_cast<rocblas_int>(n), &one,
+                                        reinterpret_cast<const rocblas_double_complex *>(rhp),
+                                        static_cast<rocblas_int>(used),
+                                        reinterpret_cast<const rocblas_double_complex *>(rpp) +
+                                            static_cast<size_t>(n - kept) * n,
+                                        static_cast<rocblas_int>(n), &zero,
+                                        reinterpret_cast<rocblas_double_complex *>(av),
+                                        static_cast<rocblas_int>(used))))
+            return fail();
+        const uint32_t i0 = pass == 0 ? 0u : used - std::min(used, out->max_off);
+        hipLaunchKernelGGL(PackAtKernel, dim3(airan::CeilDiv(used - i0, 256), rank), dim3(256), 0, stream, av, at, used,
+                           i0, pass == 0 ? 0u : out->max_off, rows, kept);
+    }
     out->rank = rank;
     out->kept = kept;
-    if (hipMalloc(&out->bt, sizeof(float2) * static_cast<size_t>(n) * rank) != hipSuccess ||
-        hipMalloc(&at, sizeof(float2) * static_cast<size_t>(rank) * g.used) != hipSuccess ||
-        hipMalloc(&out->a2, sizeof(float) * static_cast<size_t>(rank) * g.used) != hipSuccess ||
+    if (hipMalloc(&bt, sizeof(float2) * static_cast<size_t>(n) * rank) != hipSuccess ||
+        hipMalloc(&out->a2, sizeof(float) * static_cast<size_t>(rank) * rows) != hipSuccess ||
         hipMalloc(&out->lam, sizeof(float) * rank) != hipSuccess)
         return fail();
-    hipLaunchKernelGGL(PackBtKernel, dim3(airan::CeilDiv(rank, 256), n), dim3(256), 0, stream, rpp, out->bt, n,
+    hipLaunchKernelGGL(PackBtKernel, dim3(airan::CeilDiv(rank, 256), n), dim3(256), 0, stream, rpp, bt, n,
                        rank, kept);
-    hipLaunchKernelGGL(PackAtKernel, dim3(airan::CeilDiv(g.used, 256), rank), dim3(256), 0, stream, av, at,
-                       g.used, rank, kept);
-    const uint32_t sc_pad = airan::AlignUp(g.used, kInterpTile);
+    const uint32_t sc_pad = airan::AlignUp(rows, kInterpTile);
     if (hipMalloc(&out->a16, sizeof(uint16_t) * 4 * static_cast<size_t>(sc_pad) * rank) != hipSuccess) return fail();
     hipLaunchKernelGGL(PackA16Kernel, dim3(airan::CeilDiv(sc_pad * (rank / 8), 256)), dim3(256), 0, stream, at,
-                       out->a16, out->a2, g.used, sc_pad, rank);
+                       out->a16, out->a2, rows, sc_pad, rank);
     const uint32_t k_pad = airan::AlignUp(rank, kProjKTile), pk = airan::AlignUp(n, 16u);
     if (hipMalloc(&out->w16, sizeof(uint16_t) * 6 * static_cast<size_t>(k_pad) * pk) != hipSuccess) return fail();
-    hipLaunchKernelGGL(PackW16Kernel, dim3(airan::CeilDiv(k_pad * (pk / 8), 256)), dim3(256), 0, stream, out->bt,
+    hipLaunchKernelGGL(PackW16Kernel, dim3(airan::CeilDiv(k_pad * (pk / 8), 256)), dim3(256), 0, stream, bt,
                        out->w16, n, rank, k_pad);
     std::vector<float> lam_f(rank, 1.0f);  // padded columns: zero factors, unit eigenvalue
     for (uint32_t k = 0; k < kept; ++k) lam_f[k] = static_cast<float>(std::max(lam_host[n - 1 - k], 0.0));
@@ -979,27 +1131,37 @@ int32_t BuildModel(const Geom &g, const LmmseFilterParamsV1 &prm, hipStream_t st
     return AIRAN_OK;
 }
 
-// Observation models of a grant, in layer order: a layer alone on its comb
-// gets one comb model (step 2); the first layer of an FD-OCC pair creates the
-// pair's two models g+ (offset comb) and g- (offset comb + 2), step 4.  The
+// Observation models of a grant, in layer order (so the models of a base are
+// adjacent: there are two combs, each one layer's or one pair's): a layer alone
+// on its comb gets one comb model (step 2); the first layer of an FD-OCC pair
+// creates the pair's two models g+ (offset comb) and g- (offset comb + 2), step 4.  The
 // pair's layer with FD-OCC signs (+,+) (port 1000 or 1002) is h_ls "a".
 void PlanModels(const Geom &g, const PuschMimoConfig &cfg, LmmseFilter *f)
 {
-    f->nm = 0;
+    f->nb = f->nm = 0;
     bool done[4] = {};
     for (uint32_t l = 0; l < g.nl; ++l) {
         if (done[l]) continue;
+        // The base of `step` and n observations, extended to the model's offset.
+        auto add = [&](uint32_t n, uint32_t step, uint32_t offset, uint32_t in_a, uint32_t in_b, float sign_b) {
+            uint32_t b = 0;
+            while (b < f->nb && f->base[b].step != step) ++b;
+            CeBaseFactors &bf = f->base[b];
+            if (b == f->nb) {
+                ++f->nb;
+                bf.n = n;
+                bf.step = step;
+                bf.q0 = f->nm;
+            }
+            ++bf.nq;
+            bf.max_off = std::max(bf.max_off, offset);
+            f->model[f->nm++] = {b, offset, in_a, in_b, sign_b};
+        };
         if (!g.occ[l]) {
-            CeModelFactors &m = f->model[f->nm];
-            m.n = g.n_dmrs_re;
-            m.step = 2;
-            m.offset = g.comb[l];
-            m.in_a = m.in_b = l;
-            m.sign_b = 0.0f;
             f->layer_model[l][0] = static_cast<int32_t>(f->nm);
             f->layer_model[l][1] = -1;
             f->layer_sign[l] = 1.0f;
-            ++f->nm;
+            add(g.n_dmrs_re, 2, g.comb[l], l, l, 0.0f);
             done[l] = true;
             continue;
         }
@@ -1008,22 +1170,15 @@ void PlanModels(const Geom &g, const PuschMimoConfig &cfg, LmmseFilter *f)
             if (g.comb[q] == g.comb[l]) partner = q;
         const bool l_plus = cfg.dmrs_ports[l] == 1000 || cfg.dmrs_ports[l] == 1002;
         const uint32_t lp = l_plus ? l : partner, lm = l_plus ? partner : l;
-        for (int sgn = 0; sgn < 2; ++sgn) {
-            CeModelFactors &m = f->model[f->nm + sgn];
-            m.n = g.n_occ;
-            m.step = 4;
-            m.offset = g.comb[l] + 2u * sgn;
-            m.in_a = lp;
-            m.in_b = lm;
-            m.sign_b = sgn == 0 ? 1.0f : -1.0f;
-        }
         f->layer_model[lp][0] = f->layer_model[lm][0] = static_cast<int32_t>(f->nm);
         f->layer_model[lp][1] = f->layer_model[lm][1] = static_cast<int32_t>(f->nm + 1);
         f->layer_sign[lp] = 1.0f;
         f->layer_sign[lm] = -1.0f;
-        f->nm += 2;
+        add(g.n_occ, 4, g.comb[l], lp, lm, 1.0f);
+        add(g.n_occ, 4, g.comb[l] + 2u, lp, lm, -1.0f);
         done[lp] = done[lm] = true;
     }
+    for (uint32_t b = 0; b < f->nb; ++b) f->base[b].rows = g.used + f->base[b].max_off;
 }
 
 CeApply MakeApply(const LmmseFilter &f)
@@ -1038,9 +1193,14 @@ CeApply MakeApply(const LmmseFilter &f)
     c.used = g.used;
     c.pad = g.pad;
     c.nsym = g.nsym;
+    c.nb = f.nb;
+    for (uint32_t b = 0; b < f.nb; ++b) {
+        const CeBaseFactors &m = f.base[b];
+        c.b[b] = CeBaseDev{m.a2, m.a16, m.w16, m.lam, m.n, m.rank, m.kept, m.rows, m.q0, m.nq};
+    }
     for (uint32_t q = 0; q < f.nm; ++q) {
-        const CeModelFactors &m = f.model[q];
-        c.m[q] = CeModelDev{m.bt, m.a2, m.a16, m.w16, m.lam, m.n, m.rank, m.kept, m.in_a, m.in_b, m.sign_b};
+        const CeModel &m = f.model[q];
+        c.m[q] = CeModelDev{m.base, f.base[m.base].max_off - m.offset, m.in_a, m.in_b, m.sign_b};
     }
     std::memcpy(c.layer_model, f.layer_model, sizeof(c.layer_model));
     std::memcpy(c.layer_sign, f.layer_sign, sizeof(c.layer_sign));
@@ -1072,7 +1232,7 @@ namespace {
 // by binary search over the block prefix sums and runs the step's body with
 // the job's arguments and its block coordinates within the job's grid, so
 // each job computes exactly what its own LaunchCeApply would.
-constexpr int kCeSteps = 8;  // ZSplit, Project, Energy, Stats, Hv, ScaleSplit, Interp, Post
+constexpr int kCeSteps = 8;  // ZSplit, Project, Energy, Hv, Interp, InterpSmall, Post, Scale
 
 struct CeJobDev {
     CeApply c;
@@ -1080,7 +1240,7 @@ struct CeJobDev {
     const __half *hr, *hi, *noise_in;
     __half *noise_out, *out_re, *out_im;
     uint32_t slots, out_layers;
-    uint32_t k_tiles, proj_per_xcd, hv_slot_tiles, hv_sc_tiles, sc_tiles, interp_per_xcd;
+    uint32_t k_tiles, proj_per_xcd, proj_small_per_xcd, interp_per_xcd, small_per_xcd;
     uint32_t gx[kCeSteps], gy[kCeSteps];
 };
 
@@ -1119,47 +1279,50 @@ __global__ void __launch_bounds__(256, 2) CeProjectGrouped(const CeJobDev *jobs,
 {
     const CeJobBlock jb = LocateJob(jobs, starts, n, 1);
     const CeJobDev &J = *jb.job;
-    CeProjectMfmaKernelBody(J.w, J.slots, J.c, J.k_tiles, J.proj_per_xcd, jb.bx, jb.by);
+    if (BaseRows(J.c.b[jb.by].nq, J.slots, J.c.nr * J.c.ndmrs) < kSmallRows)
+        CeProjectMfmaKernelBody<1>(J.w, J.slots, J.c, J.k_tiles, J.proj_small_per_xcd, jb.bx, jb.by);
+    else
+        CeProjectMfmaKernelBody<2>(J.w, J.slots, J.c, J.k_tiles, J.proj_per_xcd, jb.bx, jb.by);
 }
 
 __global__ void __launch_bounds__(256) CeEnergyGrouped(const CeJobDev *jobs, const uint32_t *starts, uint32_t n)
 {
     const CeJobBlock jb = LocateJob(jobs, starts, n, 2);
     const CeJobDev &J = *jb.job;
-    CeEnergyKernelBody(J.hr, J.hi, J.w, J.c, J.slots, jb.bx, jb.by);
+    CeEnergyKernelBody(J.hr, J.hi, J.w, J.c, J.slots, jb.bx);
 }
 
-__global__ void __launch_bounds__(256) CeStatsGrouped(const CeJobDev *jobs, const uint32_t *starts, uint32_t n)
+__global__ void __launch_bounds__(256) CeScaleGrouped(const CeJobDev *jobs, const uint32_t *starts, uint32_t n)
 {
-    const CeJobBlock jb = LocateJob(jobs, starts, n, 3);
+    const CeJobBlock jb = LocateJob(jobs, starts, n, 7);
     const CeJobDev &J = *jb.job;
-    CeStatsKernelBody(J.noise_in, J.noise_out, J.w, J.c, jb.bx, jb.by);
+    CeScaleKernelBody(J.noise_in, J.noise_out, J.w, J.c, J.slots, jb.bx);
 }
 
 __global__ void __launch_bounds__(256) CeHvGrouped(const CeJobDev *jobs, const uint32_t *starts, uint32_t n)
 {
-    const CeJobBlock jb = LocateJob(jobs, starts, n, 4);
+    const CeJobBlock jb = LocateJob(jobs, starts, n, 3);
     const CeJobDev &J = *jb.job;
-    CeHvMfmaKernelBody(J.w, J.slots, J.c, J.hv_slot_tiles, J.hv_sc_tiles, jb.bx, jb.by);
-}
-
-__global__ void __launch_bounds__(256) CeScaleSplitGrouped(const CeJobDev *jobs, const uint32_t *starts, uint32_t n)
-{
-    const CeJobBlock jb = LocateJob(jobs, starts, n, 5);
-    const CeJobDev &J = *jb.job;
-    CeScaleSplitKernelBody(J.w, J.slots, J.c, jb.bx, jb.by);
+    CeHvMfmaKernelBody(J.w, J.slots, J.c, jb.bx, jb.by);
 }
 
 __global__ void __launch_bounds__(256, 2) CeInterpGrouped(const CeJobDev *jobs, const uint32_t *starts, uint32_t n)
 {
-    const CeJobBlock jb = LocateJob(jobs, starts, n, 6);
+    const CeJobBlock jb = LocateJob(jobs, starts, n, 4);
     const CeJobDev &J = *jb.job;
-    CeInterpMfmaKernelBody(J.w, J.slots, J.c, J.sc_tiles, J.interp_per_xcd, jb.bx, jb.by);
+    CeInterpMfmaKernelBody(J.w, J.slots, J.c, J.interp_per_xcd, jb.bx, jb.by);
+}
+
+__global__ void __launch_bounds__(256) CeInterpSmallGrouped(const CeJobDev *jobs, const uint32_t *starts, uint32_t n)
+{
+    const CeJobBlock jb = LocateJob(jobs, starts, n, 5);
+    const CeJobDev &J = *jb.job;
+    CeInterpSmallKernelBody(J.w, J.slots, J.c, J.small_per_xcd, jb.bx, jb.by);
 }
 
 __global__ void __launch_bounds__(256) CePostGrouped(const CeJobDev *jobs, const uint32_t *starts, uint32_t n)
 {
-    const CeJobBlock jb = LocateJob(jobs, starts, n, 7);
+    const CeJobBlock jb = LocateJob(jobs, starts, n, 6);
     const CeJobDev &J = *jb.job;
     switch (J.c.ndmrs) {
     case 1: CePostKernelBody<1>(J.w, J.out_re, J.out_im, J.out_layers, J.c, jb.bx, jb.by); break;
@@ -1169,31 +1332,37 @@ __global__ void __launch_bounds__(256) CePostGrouped(const CeJobDev *jobs, const
     }
 }
 
-// The grids LaunchCeApply uses for one application.
-void StepGrids(const LmmseFilter &f, const CeWs &w, uint32_t slots, CeJobDev *j)
+// Grids of one application's steps (gx = 0: the step has nothing to do); a
+// base's products take the 128-row or, below kSmallRows rows, the 32-row form.
+void StepGrids(const LmmseFilter &f, uint32_t slots, CeJobDev *j)
 {
     const Geom &g = f.g;
     const uint32_t ncol = g.nr * g.ndmrs;
-    uint32_t max_rank = 0, max_n = 0;
-    for (uint32_t q = 0; q < f.nm; ++q) {
-        max_rank = std::max(max_rank, f.model[q].rank);
-        max_n = std::max(max_n, f.model[q].n);
-    }
+    uint32_t max_rank = 0, z = 0, hv = 0, large = 0, small = 0;
+    for (uint32_t b = 0; b < f.nb; ++b) max_rank = std::max(max_rank, f.base[b].rank);
     j->k_tiles = airan::AlignUp(max_rank, kProjKTile) / kProjKTile;
-    j->proj_per_xcd = airan::CeilDiv(f.nm * kProjSplits * (w.npad / 64) * j->k_tiles, 8);
-    j->hv_slot_tiles = airan::CeilDiv(slots, 32);
-    j->hv_sc_tiles = airan::CeilDiv(g.used, 32);
-    j->sc_tiles = airan::AlignUp(g.used, kInterpTile) / kInterpTile;
-    j->interp_per_xcd = airan::CeilDiv(f.nm * j->sc_tiles * (w.npad / kInterpTile), 8);
-    const uint32_t gx[kCeSteps] = {airan::CeilDiv(static_cast<uint64_t>(w.npad) * airan::AlignUp(max_n, 16u) / 8, 256),
-                                   8 * j->proj_per_xcd,
-                                   slots * f.nm * ncol,
-                                   slots,
-                                   j->hv_slot_tiles * j->hv_sc_tiles * f.nm,
-                                   airan::CeilDiv(static_cast<uint64_t>(w.npad) * kMaxRank / 8, 256),
-                                   8 * j->interp_per_xcd,
-                                   airan::CeilDiv(g.pad, 256)};
-    const uint32_t gy[kCeSteps] = {f.nm, 1, 1, 1, 1, f.nm, 1, slots * g.nl};
+    uint32_t proj = 0, proj_small = 0;
+    for (uint32_t b = 0; b < f.nb; ++b) {
+        const CeBaseFactors &m = f.base[b];
+        const uint32_t rows = BaseRows(m.nq, slots, ncol), sc_tiles = airan::CeilDiv(m.rows, kInterpTile);
+        z = std::max(z, airan::CeilDiv(static_cast<uint64_t>(rows) * airan::AlignUp(m.n, 16u) / 8, 256));
+        hv = std::max(hv, airan::CeilDiv(m.nq * slots, 32) * airan::CeilDiv(m.rows, 32));
+        if (rows < kSmallRows) {
+            proj_small = std::max(proj_small, kProjSplits * airan::CeilDiv(rows, 32) * j->k_tiles);
+            small = std::max(small, sc_tiles * airan::CeilDiv(rows, 32));
+        } else {
+            proj = std::max(proj, kProjSplits * airan::CeilDiv(rows, 64) * j->k_tiles);
+            large = std::max(large, sc_tiles * airan::CeilDiv(rows, kInterpTile));
+        }
+    }
+    j->proj_per_xcd = airan::CeilDiv(proj, 8);
+    j->proj_small_per_xcd = airan::CeilDiv(proj_small, 8);
+    j->interp_per_xcd = airan::CeilDiv(large, 8);
+    j->small_per_xcd = airan::CeilDiv(small, 8);
+    const uint32_t gx[kCeSteps] = {z, 8 * std::max(j->proj_per_xcd, j->proj_small_per_xcd), slots * f.nm * ncol, hv,
+                                   8 * j->interp_per_xcd, 8 * j->small_per_xcd, airan::CeilDiv(g.pad, 256),
+                                   slots * kScaleParts};
+    const uint32_t gy[kCeSteps] = {f.nb, f.nb, 1, f.nb, f.nb, f.nb, slots * g.nl * airan::CeilDiv(g.nr, kPostRx), 1};
     for (int k = 0; k < kCeSteps; ++k) {
         j->gx[k] = gx[k];
         j->gy[k] = gy[k];
@@ -1224,29 +1393,23 @@ int32_t LaunchCeApply(const LmmseFilter *f, const __half *hr, const __half *hi, 
     const CeApply c = MakeApply(*f);
     CeWs w{};
     CeWsLayout(g, slots, static_cast<uint8_t *>(ws), &w);
-    const uint32_t ncol = g.nr * g.ndmrs;
-    uint32_t max_rank = 0;
-    for (uint32_t q = 0; q < f->nm; ++q) max_rank = std::max(max_rank, f->model[q].rank);
-    uint32_t max_n = 0;
-    for (uint32_t q = 0; q < f->nm; ++q) max_n = std::max(max_n, f->model[q].n);
-    hipLaunchKernelGGL(CeZSplitKernel, dim3(CeilDiv(static_cast<uint64_t>(w.npad) * AlignUp(max_n, 16u) / 8, 256),
-                                            f->nm),
-                       dim3(256), 0, s, hr, hi, w, slots, c);
-    const uint32_t k_tiles = AlignUp(max_rank, kProjKTile) / kProjKTile;
-    const uint32_t proj_per_xcd = CeilDiv(f->nm * kProjSplits * (w.npad / 64) * k_tiles, 8);
-    hipLaunchKernelGGL(CeProjectMfmaKernel, dim3(8 * proj_per_xcd), dim3(256), 0, s, w, slots, c, k_tiles,
-                       proj_per_xcd);
-    hipLaunchKernelGGL(CeEnergyKernel, dim3(slots * f->nm * ncol), dim3(256), 0, s, hr, hi, w, c, slots);
-    hipLaunchKernelGGL(CeStatsKernel, dim3(slots), dim3(256), 0, s, noise_in, noise_out, w, c);
-    const uint32_t hv_slot_tiles = CeilDiv(slots, 32), hv_sc_tiles = CeilDiv(g.used, 32);
-    hipLaunchKernelGGL(CeHvMfmaKernel, dim3(hv_slot_tiles * hv_sc_tiles * f->nm), dim3(256), 0, s, w, slots, c,
-                       hv_slot_tiles, hv_sc_tiles);
-    hipLaunchKernelGGL(CeScaleSplitKernel, dim3(CeilDiv(static_cast<uint64_t>(w.npad) * kMaxRank / 8, 256), f->nm),
-                       dim3(256), 0, s, w, slots, c);
-    const uint32_t sc_tiles = AlignUp(g.used, kInterpTile) / kInterpTile;
-    const uint32_t per_xcd = CeilDiv(f->nm * sc_tiles * (w.npad / kInterpTile), 8);
-    hipLaunchKernelGGL(CeInterpMfmaKernel, dim3(8 * per_xcd), dim3(256), 0, s, w, slots, c, sc_tiles, per_xcd);
-    const dim3 pgrid(CeilDiv(g.pad, 256), slots * g.nl);
+    CeJobDev j{};
+    StepGrids(*f, slots, &j);
+    auto grid = [&](int step) { return dim3(j.gx[step], j.gy[step]); };
+    hipLaunchKernelGGL(CeZSplitKernel, grid(0), dim3(256), 0, s, hr, hi, w, slots, c);
+    if (j.proj_per_xcd)
+        hipLaunchKernelGGL(CeProjectMfmaKernel, dim3(8 * j.proj_per_xcd, f->nb), dim3(256), 0, s, w, slots, c, j.k_tiles,
+                           j.proj_per_xcd);
+    if (j.proj_small_per_xcd)
+        hipLaunchKernelGGL(CeProjectSmallKernel, dim3(8 * j.proj_small_per_xcd, f->nb), dim3(256), 0, s, w, slots, c,
+                           j.k_tiles, j.proj_small_per_xcd);
+    hipLaunchKernelGGL(CeEnergyKernel, grid(2), dim3(256), 0, s, hr, hi, w, c, slots);
+    hipLaunchKernelGGL(CeScaleKernel, grid(7), dim3(256), 0, s, noise_in, noise_out, w, c, slots);
+    hipLaunchKernelGGL(CeHvMfmaKernel, grid(3), dim3(256), 0, s, w, slots, c);
+    if (j.interp_per_xcd)
+        hipLaunchKernelGGL(CeInterpMfmaKernel, grid(4), dim3(256), 0, s, w, slots, c, j.interp_per_xcd);
+    if (j.small_per_xcd) hipLaunchKernelGGL(CeInterpSmallKernel, grid(5), dim3(256), 0, s, w, slots, c, j.small_per_xcd);
+    const dim3 pgrid = grid(6);
     switch (g.ndmrs) {
     case 1: hipLaunchKernelGGL(CePostKernel<1>, pgrid, dim3(256), 0, s, w, out_re, out_im, out_layers, c); break;
     case 2: hipLaunchKernelGGL(CePostKernel<2>, pgrid, dim3(256), 0, s, w, out_re, out_im, out_layers, c); break;
@@ -1295,7 +1458,7 @@ int32_t CreateCeGrouped(const CeGroupJob *jobs, uint32_t n, CeGrouped **out)
         d.out_im = jb.out_im;
         d.slots = jb.slots;
         d.out_layers = jb.out_layers;
-        StepGrids(*jb.filter, d.w, jb.slots, &d);
+        StepGrids(*jb.filter, jb.slots, &d);
         for (int k = 0; k < kCeSteps; ++k) {
             starts[static_cast<size_t>(k) * (n + 1) + i] = static_cast<uint32_t>(acc[k]);
             acc[k] += static_cast<uint64_t>(d.gx[k]) * d.gy[k];
@@ -1330,11 +1493,11 @@ int32_t LaunchCeGrouped(const CeGrouped *g, hipStream_t s)
     if (g->total[0]) hipLaunchKernelGGL(CeZSplitGrouped, dim3(g->total[0]), dim3(256), 0, s, j, st, n);
     if (g->total[1]) hipLaunchKernelGGL(CeProjectGrouped, dim3(g->total[1]), dim3(256), 0, s, j, st, n);
     if (g->total[2]) hipLaunchKernelGGL(CeEnergyGrouped, dim3(g->total[2]), dim3(256), 0, s, j, st, n);
-    if (g->total[3]) hipLaunchKernelGGL(CeStatsGrouped, dim3(g->total[3]), dim3(256), 0, s, j, st, n);
-    if (g->total[4]) hipLaunchKernelGGL(CeHvGrouped, dim3(g->total[4]), dim3(256), 0, s, j, st, n);
-    if (g->total[5]) hipLaunchKernelGGL(CeScaleSplitGrouped, dim3(g->total[5]), dim3(256), 0, s, j, st, n);
-    if (g->total[6]) hipLaunchKernelGGL(CeInterpGrouped, dim3(g->total[6]), dim3(256), 0, s, j, st, n);
-    if (g->total[7]) hipLaunchKernelGGL(CePostGrouped, dim3(g->total[7]), dim3(256), 0, s, j, st, n);
+    if (g->total[7]) hipLaunchKernelGGL(CeScaleGrouped, dim3(g->total[7]), dim3(256), 0, s, j, st, n);
+    if (g->total[3]) hipLaunchKernelGGL(CeHvGrouped, dim3(g->total[3]), dim3(256), 0, s, j, st, n);
+    if (g->total[4]) hipLaunchKernelGGL(CeInterpGrouped, dim3(g->total[4]), dim3(256), 0, s, j, st, n);
+    if (g->total[5]) hipLaunchKernelGGL(CeInterpSmallGrouped, dim3(g->total[5]), dim3(256), 0, s, j, st, n);
+    if (g->total[6]) hipLaunchKernelGGL(CePostGrouped, dim3(g->total[6]), dim3(256), 0, s, j, st, n);
     return LaunchStatus();
 }
 
@@ -1448,8 +1611,8 @@ int32_t airan_channel_est_lmmse_CreateFilter(const PuschMimoConfig *config, cons
     f->params = *params;
     PlanModels(g, *config, f);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    for (uint32_t q = 0; q < f->nm; ++q) {
-        st = BuildModel(g, *params, s, &f->model[q]);
+    for (uint32_t b = 0; b < f->nb; ++b) {
+        st = BuildBase(*params, s, &f->base[b]);
         if (st != AIRAN_OK) {
             airan_channel_est_lmmse_DestroyFilter(f);
             return st;
@@ -1473,12 +1636,11 @@ int32_t airan_channel_est_lmmse_CreateFilter(const PuschMimoConfig *config, cons
 void airan_channel_est_lmmse_DestroyFilter(LmmseFilter *f)
 {
     if (f == nullptr) return;
-    for (uint32_t q = 0; q < kMaxModels; ++q) {
-        FreeDev(f->model[q].bt);
-        FreeDev(f->model[q].a2);
-        FreeDev(f->model[q].a16);
-        FreeDev(f->model[q].w16);
-        FreeDev(f->model[q].lam);
+    for (CeBaseFactors &b : f->base) {
+        FreeDev(b.a2);
+        FreeDev(b.a16);
+        FreeDev(b.w16);
+        FreeDev(b.lam);
     }
     delete f;
 }
@@ -1486,7 +1648,7 @@ void airan_channel_est_lmmse_DestroyFilter(LmmseFilter *f)
 uint32_t airan_channel_est_lmmse_FilterRank(const LmmseFilter *f, uint32_t layer)
 {
     if (f == nullptr || layer >= f->g.nl) return 0;
-    return f->model[f->layer_model[layer][0]].kept;
+    return f->base[f->model[f->layer_model[layer][0]].base].kept;
 }
 
 size_t airan_channel_est_lmmse_WorkspaceBytes(const PuschMimoConfig *config)
