@@ -192,7 +192,7 @@ struct AiranGrantBatch {
     };
     std::vector<FftGroup> ffts;
     RaggedItem *gen_items = nullptr, *ls_items = nullptr, *noise_items = nullptr;
-    uint32_t n_gen = 0, n_ls = 0, n_noise = 0, max_ref_pad = 0, max_pilot_pad = 0, max_dmrs = 0;
+    uint32_t n_gen = 0, n_ls = 0, n_noise = 0, max_pilot_pad = 0, max_dmrs = 0;
     RaggedTile *tiles = nullptr;
     uint32_t n_tiles = 0, tile = 256;
     std::vector<RaggedTile> host_tiles_src;  // (grant, ds, used) per row, for rebuilding tiles
@@ -264,7 +264,7 @@ int32_t EnqueueStages(AiranGrantBatch *b, const void *iq, hipStream_t s)
             AIRAN_OK)
             return st;
     if ((st = airan::LaunchDmrsRagged(b->grants, b->gen_items, b->n_gen, b->ls_items, b->n_ls, b->noise_items,
-                                      b->n_noise, b->max_ref_pad, b->max_pilot_pad, b->max_dmrs, b->rx_re, b->rx_im,
+                                      b->n_noise, b->max_pilot_pad, b->max_dmrs, b->rx_re, b->rx_im,
                                       b->ref_re, b->ref_im, b->hls_re, b->hls_im, b->noise_ls, s)) != AIRAN_OK)
         return st;
     if ((st = airan::LaunchCeGrouped(b->ce_grouped, s)) != AIRAN_OK) return st;
@@ -435,7 +435,6 @@ int32_t airan_pusch_grants_Create(const PuschMimoConfig *configs, const AiranTbP
             for (uint32_t l = 0; l < g.nl; ++l) ls.push_back({i, r, l});
         for (uint32_t r = 0; r < g.nr; ++r) nz.push_back({i, r, 0});
         for (uint32_t ds = 0; ds < g.ndata; ++ds) b->host_tiles_src.push_back({i, ds, g.used});
-        b->max_ref_pad = std::max(b->max_ref_pad, g.ref_pad);
         b->max_pilot_pad = std::max(b->max_pilot_pad, g.pilot_pad);
         b->max_dmrs = std::max(b->max_dmrs, g.ndmrs);
         const uint32_t rows = airan_ldpc_ActiveRows(&p);

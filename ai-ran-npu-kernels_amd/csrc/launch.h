@@ -123,7 +123,7 @@ int32_t LaunchOfdmRagged(uint32_t fft, uint32_t iq_format, const RaggedStream *s
 // and noise (items (grant, rx)); the max_* bound the grids.
 int32_t LaunchDmrsRagged(const RaggedGrant *grants, const RaggedItem *gen_items, uint32_t n_gen,
                          const RaggedItem *ls_items, uint32_t n_ls, const RaggedItem *noise_items, uint32_t n_noise,
-                         uint32_t max_ref_pad, uint32_t max_pilot_pad, uint32_t max_dmrs, const __half *rx_re,
+                         uint32_t max_pilot_pad, uint32_t max_dmrs, const __half *rx_re,
                          const __half *rx_im, __half *ref_re, __half *ref_im, __half *h_re, __half *h_im,
                          __half *noise, hipStream_t s);
 // c_init of DMRS symbol `symbol` of cfg (mimo_dmrs_gen.cpp:38-45).

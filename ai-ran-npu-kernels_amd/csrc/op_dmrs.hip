@@ -41,96 +41,70 @@ __device__ inline uint32_t DevDmrsCinit(uint32_t slot_number, uint32_t symbol, u
 }
 
 // r(m) = ((1-2c(2m)) + j(1-2c(2m+1)))/sqrt(2) (mimo_dmrs_gen_kernel.cpp:163),
-// times w_f = (-1)^m on ports 1001/1003.  A thread owns 16 consecutive m.
-// Grid (m blocks, D, slots * L).  slot_no == nullptr: one reference from
-// d.cinit; else one reference per slot ([slots][L][D][ref_pad]), its c_init
-// from the slot's number slot_no[slot].
-// 16 consecutive pilots m0 .. m0 + 15 of one reference [ref_pad] at `base`:
-// pilot m of DMRS c_init `cinit` (Gold offset `off`), zero past n_dmrs_re.
-__device__ inline void DmrsGen16(uint16_t *__restrict__ re, uint16_t *__restrict__ im, size_t base, uint32_t m0,
-                                 uint32_t ref_pad, uint32_t n_dmrs_re, uint32_t cinit, uint32_t off, bool wf_odd)
+// times w_f = (-1)^m on ports 1001/1003; zero past n_dmrs_re.  One reference
+// row [ref_pad] at `re`, `im` by one workgroup, 8 pilots a thread; 16-byte
+// stores where the row allows them (ref_pad is a multiple of 128).
+//
+// Bound by latency: a 273-PRB row is 6.6 KB.  The row's Gold bits come from
+// one GoldSpan (11 barriers) instead of a jump per thread; a workgroup per
+// layer derives its symbol's bits again rather than store four layers in
+// turn.  64 full-carrier slots of 4 layers (27 MB written): 17 -> 6.5 us, one
+// slot 12.5 -> 5.2 us.
+__device__ inline void DmrsRow(uint16_t *__restrict__ re, uint16_t *__restrict__ im, uint32_t ref_pad,
+                               uint32_t n_dmrs_re, uint32_t cinit, uint32_t off, bool wf_odd)
 {
-    const uint16_t pos = 0x39a8, neg = 0xb9a8;  // fp16(+-0.70710678)
-    const uint32_t bits = airan::GoldWordAt(cinit, 2ull * (m0 + off));
+    __shared__ uint32_t x1[airan::kGoldSpanWords + 2], x2[airan::kGoldSpanWords + 2];
+    const uint32_t first = airan::GoldSpan(x1, x2, cinit, 2ull * off, 2u * n_dmrs_re);
+    const bool vec = ((reinterpret_cast<uintptr_t>(re) | reinterpret_cast<uintptr_t>(im)) & 15u) == 0;
+    const uint32_t pos = 0x39a8u, flip = 0x8000u;  // fp16(0.70710678), its sign
+    for (uint32_t m0 = 8u * threadIdx.x; m0 < ref_pad; m0 += 8u * blockDim.x) {
+        // Pilots in pairs (m, m + 1), m even: w_f = -1 negates the second.
+        const uint32_t bits = m0 < n_dmrs_re ? airan::BitsAt(x1, first + 2u * m0) : 0u;
+        uint32_t wr[4], wi[4];
 #pragma unroll
-    for (uint32_t j = 0; j < 16; ++j) {
-        const uint32_t m = m0 + j;
-        if (m >= ref_pad) break;
-        uint16_t vr = 0, vi = 0;
-        if (m < n_dmrs_re) {
-            vr = ((bits >> (2 * j)) & 1u) ? neg : pos;
-            vi = ((bits >> (2 * j + 1)) & 1u) ? neg : pos;
-            if (wf_odd && (m & 1u)) {
-                vr ^= 0x8000u;
-                vi ^= 0x8000u;
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t m = m0 + 2u * k, c = bits >> (4u * k);
+            const uint32_t have = (m < n_dmrs_re ? 0xffffu : 0u) | (m + 1u < n_dmrs_re ? 0xffff0000u : 0u);
+            const uint32_t one = (pos | pos << 16) ^ (wf_odd ? flip << 16 : 0u);
+            wr[k] = (one ^ (c & 1u ? flip : 0u) ^ (c & 4u ? flip << 16 : 0u)) & have;
+            wi[k] = (one ^ (c & 2u ? flip : 0u) ^ (c & 8u ? flip << 16 : 0u)) & have;
+        }
+        if (vec) {
+            *reinterpret_cast<uint4 *>(re + m0) = uint4{wr[0], wr[1], wr[2], wr[3]};
+            *reinterpret_cast<uint4 *>(im + m0) = uint4{wi[0], wi[1], wi[2], wi[3]};
+        } else {
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j) {
+                re[m0 + j] = static_cast<uint16_t>(wr[j / 2] >> (16u * (j & 1u)));
+                im[m0 + j] = static_cast<uint16_t>(wi[j / 2] >> (16u * (j & 1u)));
             }
         }
-        re[base + m] = vr;
-        im[base + m] = vi;
     }
 }
 
-// Grid (m blocks, D, slots): the layers of a (slot, DMRS symbol) share one
-// Gold sequence (they differ in w_f only), so a thread derives the word of
-// its 16 pilots once and writes every layer's 16 values; vec: the outputs
-// are 16-byte aligned (ref_pad is a multiple of 128, so are all the rows),
-// which allows 16-byte stores.
+// Grid (L, D, slots).  slot_no == nullptr: one reference from d.cinit; else
+// one reference per slot ([slots][L][D][ref_pad]), its c_init from the slot's
+// number slot_no[slot].
 __global__ void __launch_bounds__(256) DmrsGenKernel(uint16_t *__restrict__ re, uint16_t *__restrict__ im,
-                                                     const uint16_t *__restrict__ slot_no, DmrsGenDev d,
-                                                     uint32_t vec)
+                                                     const uint16_t *__restrict__ slot_no, DmrsGenDev d)
 {
-    const uint32_t m0 = (blockIdx.x * blockDim.x + threadIdx.x) * 16;
-    if (m0 >= d.ref_pad) return;
-    const uint32_t dd = blockIdx.y, slot = blockIdx.z;
+    const uint32_t l = blockIdx.x, dd = blockIdx.y, slot = blockIdx.z;
     const uint32_t cinit = slot_no == nullptr ? d.cinit[dd] : DevDmrsCinit(slot_no[slot], d.sym[dd], d.nid, d.nscid);
-    if (!vec) {
-        for (uint32_t l = 0; l < d.nl; ++l) {
-            const size_t base = ((static_cast<size_t>(slot) * d.nl + l) * d.ndmrs + dd) * d.ref_pad;
-            DmrsGen16(re, im, base, m0, d.ref_pad, d.n_dmrs_re, cinit, d.off, d.wf_odd[l] != 0);
-        }
-        return;
-    }
-    // Pilots m0 .. m0 + 15 (m0 is a multiple of 16 and ref_pad of 128: all
-    // below ref_pad) as fp16 pairs, w_f = +1; pilots past n_dmrs_re are +0.
-    const uint32_t pos = 0x39a8u, neg = 0xb9a8u;  // fp16(+-0.70710678)
-    const uint32_t bits = m0 < d.n_dmrs_re ? airan::GoldWordAt(cinit, 2ull * (m0 + d.off)) : 0u;
-    uint32_t wr[8], wi[8], odd[8];
-#pragma unroll
-    for (uint32_t k = 0; k < 8; ++k) {
-        const uint32_t m = m0 + 2u * k;
-        const bool v0 = m < d.n_dmrs_re, v1 = m + 1u < d.n_dmrs_re;
-        const uint32_t r0 = v0 ? ((bits >> (4u * k)) & 1u ? neg : pos) : 0u;
-        const uint32_t i0 = v0 ? ((bits >> (4u * k + 1u)) & 1u ? neg : pos) : 0u;
-        const uint32_t r1 = v1 ? ((bits >> (4u * k + 2u)) & 1u ? neg : pos) : 0u;
-        const uint32_t i1 = v1 ? ((bits >> (4u * k + 3u)) & 1u ? neg : pos) : 0u;
-        wr[k] = r0 | r1 << 16;
-        wi[k] = i0 | i1 << 16;
-        odd[k] = v1 ? 0x80000000u : 0u;  // w_f = -1 negates the odd pilot m + 1
-    }
-    for (uint32_t l = 0; l < d.nl; ++l) {
-        const uint32_t f = d.wf_odd[l] != 0 ? ~0u : 0u;
-        const size_t base = ((static_cast<size_t>(slot) * d.nl + l) * d.ndmrs + dd) * d.ref_pad + m0;
-        uint4 *pr = reinterpret_cast<uint4 *>(re + base), *pi = reinterpret_cast<uint4 *>(im + base);
-        pr[0] = uint4{wr[0] ^ (odd[0] & f), wr[1] ^ (odd[1] & f), wr[2] ^ (odd[2] & f), wr[3] ^ (odd[3] & f)};
-        pr[1] = uint4{wr[4] ^ (odd[4] & f), wr[5] ^ (odd[5] & f), wr[6] ^ (odd[6] & f), wr[7] ^ (odd[7] & f)};
-        pi[0] = uint4{wi[0] ^ (odd[0] & f), wi[1] ^ (odd[1] & f), wi[2] ^ (odd[2] & f), wi[3] ^ (odd[3] & f)};
-        pi[1] = uint4{wi[4] ^ (odd[4] & f), wi[5] ^ (odd[5] & f), wi[6] ^ (odd[6] & f), wi[7] ^ (odd[7] & f)};
-    }
+    const size_t base = ((static_cast<size_t>(slot) * d.nl + l) * d.ndmrs + dd) * d.ref_pad;
+    DmrsRow(re + base, im + base, d.ref_pad, d.n_dmrs_re, cinit, d.off, d.wf_odd[l] != 0);
 }
 
-// Ragged batch: item = (grant, layer); grid (m blocks of the largest grant,
-// D max, items).
+// Ragged batch: item = (grant, layer); grid (1, D max, items).
 __global__ void __launch_bounds__(256) RaggedDmrsGenKernel(uint16_t *__restrict__ re, uint16_t *__restrict__ im,
                                                            const airan::RaggedGrant *__restrict__ grants,
                                                            const airan::RaggedItem *__restrict__ items)
 {
     const airan::RaggedItem it = items[blockIdx.z];
     const airan::RaggedGrant &gr = grants[it.grant];
-    const uint32_t m0 = (blockIdx.x * blockDim.x + threadIdx.x) * 16;
     const uint32_t dd = blockIdx.y;
-    if (m0 >= gr.g.ref_pad || dd >= gr.g.ndmrs) return;
+    if (dd >= gr.g.ndmrs) return;
     const size_t base = gr.ref_off + (static_cast<size_t>(it.a) * gr.g.ndmrs + dd) * gr.g.ref_pad;
-    DmrsGen16(re, im, base, m0, gr.g.ref_pad, gr.g.n_dmrs_re, gr.dmrs_cinit[dd], gr.dmrs_off, gr.wf_odd[it.a] != 0);
+    DmrsRow(re + base, im + base, gr.g.ref_pad, gr.g.n_dmrs_re, gr.dmrs_cinit[dd], gr.dmrs_off, gr.wf_odd[it.a] != 0);
 }
 
 // channel_est/mimo_dmrs_ls/mimo_dmrs_ls_kernel.cpp:146-177,301-331: h = y x*
@@ -335,12 +309,12 @@ uint32_t HostDmrsCinit(const PuschMimoConfig &cfg, uint32_t symbol) { return Dmr
 
 int32_t LaunchDmrsRagged(const RaggedGrant *grants, const RaggedItem *gen_items, uint32_t n_gen,
                          const RaggedItem *ls_items, uint32_t n_ls, const RaggedItem *noise_items, uint32_t n_noise,
-                         uint32_t max_ref_pad, uint32_t max_pilot_pad, uint32_t max_dmrs, const __half *rx_re,
+                         uint32_t max_pilot_pad, uint32_t max_dmrs, const __half *rx_re,
                          const __half *rx_im, __half *ref_re, __half *ref_im, __half *h_re, __half *h_im,
                          __half *noise, hipStream_t s)
 {
     if (n_gen == 0 || n_ls == 0 || n_noise == 0) return AIRAN_INVALID_ARGUMENT;
-    hipLaunchKernelGGL(RaggedDmrsGenKernel, dim3(CeilDiv(CeilDiv(max_ref_pad, 16), 256), max_dmrs, n_gen), dim3(256),
+    hipLaunchKernelGGL(RaggedDmrsGenKernel, dim3(1, max_dmrs, n_gen), dim3(256),
                        0, s, reinterpret_cast<uint16_t *>(ref_re), reinterpret_cast<uint16_t *>(ref_im), grants,
                        gen_items);
     hipLaunchKernelGGL(RaggedDmrsLsKernel, dim3(CeilDiv(max_pilot_pad, 256), max_dmrs, n_ls), dim3(256), 0, s, rx_re,
@@ -355,10 +329,8 @@ int32_t LaunchDmrsGenSlots(const PuschMimoConfig &cfg, const Geom &g, const uint
 {
     if (slot_no == nullptr || slots == 0) return AIRAN_INVALID_ARGUMENT;
     const DmrsGenDev d = GenDev(cfg, g);
-    const dim3 grid(CeilDiv(CeilDiv(g.ref_pad, 16), 256), g.ndmrs, slots);
-    const uint32_t vec = ((reinterpret_cast<uintptr_t>(ref_re) | reinterpret_cast<uintptr_t>(ref_im)) & 15u) == 0;
-    hipLaunchKernelGGL(DmrsGenKernel, grid, dim3(256), 0, s, reinterpret_cast<uint16_t *>(ref_re),
-                       reinterpret_cast<uint16_t *>(ref_im), slot_no, d, vec);
+    hipLaunchKernelGGL(DmrsGenKernel, dim3(g.nl, g.ndmrs, slots), dim3(256), 0, s, reinterpret_cast<uint16_t *>(ref_re),
+                       reinterpret_cast<uint16_t *>(ref_im), slot_no, d);
     return LaunchStatus();
 }
 
@@ -446,10 +418,8 @@ int32_t airan_mimo_dmrs_gen_Enqueue(MimoDmrsGenRuntimeV1 *runtime, const MimoDmr
     Geom g;
     airan::DeriveGeom(*a->config, &g);
     const DmrsGenDev d = airan::GenDev(*a->config, g);
-    dim3 grid(airan::CeilDiv(airan::CeilDiv(g.ref_pad, 16), 256), g.ndmrs, 1);
-    const uint32_t vec = ((reinterpret_cast<uintptr_t>(a->dmrs_re) | reinterpret_cast<uintptr_t>(a->dmrs_im)) & 15u) == 0;
-    hipLaunchKernelGGL(DmrsGenKernel, grid, dim3(256), 0, static_cast<hipStream_t>(a->stream),
-                       static_cast<uint16_t *>(a->dmrs_re), static_cast<uint16_t *>(a->dmrs_im), nullptr, d, vec);
+    hipLaunchKernelGGL(DmrsGenKernel, dim3(g.nl, g.ndmrs, 1), dim3(256), 0, static_cast<hipStream_t>(a->stream),
+                       static_cast<uint16_t *>(a->dmrs_re), static_cast<uint16_t *>(a->dmrs_im), nullptr, d);
     return airan::LaunchStatus();
 }
 
