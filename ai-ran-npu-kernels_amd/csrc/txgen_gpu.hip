@@ -16,9 +16,9 @@
 //   DmrsGridKernel  the DMRS symbols of every layer: the slot's DMRS on the
 //       layer's comb (FD-OCC sign on ports 1001/1003), zero on the other.
 //   ChannelOfdmKernel  one workgroup per (slot, Rx, symbol): y = sum_l H x_l
-//       with H = sum_taps g e^(-j 2 pi f tau) on the used subcarriers, an
-//       inverse FFT of 128 .. 4096 points in LDS, the cyclic prefix and AWGN
-//       from a counter-based generator, written as IQ.
+//       with H = sum_taps g e^(-j 2 pi f tau) on the used subcarriers, a
+//       4096-point (or smaller) radix-2 IFFT in LDS, the cyclic prefix and
+//       AWGN from a counter-based generator, written as IQ.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -28,7 +28,7 @@
 #include "airan_ldpc_bg1.h"
 #include "airan_pusch_tx.h"
 #include "common.h"
-#include "fft.h"
+#include "crc.h"
 #include "gold.h"
 
 using airan::DevGeom;
@@ -41,6 +41,7 @@ constexpr uint32_t kPolyB = 0x800063u;   // CRC24B
 constexpr uint32_t kPoly16 = 0x1021u;    // CRC16
 constexpr uint32_t kTbChunkBits = 64, kCbChunkBits = 160;
 constexpr uint32_t kMaxZ = 384;
+constexpr uint32_t kMaxFft = 4096;
 
 struct TxPlan {
     uint32_t Z, C, K, kprime, per_cb, crc_cb, crc_tb, tbs, filler, ncb, q0, G, e_low, e_high, n_low;
@@ -545,7 +546,7 @@ __global__ void __launch_bounds__(256) DmrsGridKernel(DmrsArgs a, const uint16_t
 
 // ------------------------------------------------- channel + OFDM + noise
 struct ChanArgs {
-    uint32_t nr, nl, used, taps, samples, iq_float;
+    uint32_t nr, nl, used, fft, log2n, taps, samples, iq_float;
     uint32_t cp[14], start[14];
     float scs, sigma, inv_sqrt_n;
     uint64_t seed;
@@ -571,157 +572,84 @@ __device__ inline float2 Gauss2(uint64_t key)
     return make_float2(rad * cs, rad * sn);
 }
 
-// e^(-j 2 pi cyc), the phase reduced to (-1/2, 1/2] cycles in fp64; the part
-// of it that fp32 does not hold enters to first order.
-__device__ inline float2 Phasor(double cyc)
-{
-    const double frac = cyc - rint(cyc);
-    const float hi = static_cast<float>(frac), lo = 6.283185307f * static_cast<float>(frac - hi);
-    float sn, cs;
-    sincospif(2.0f * hi, &sn, &cs);
-    return make_float2(cs - sn * lo, -(sn + cs * lo));
-}
-
 // Workgroup (slot, rx, symbol).  grid: complex64 [slots][L][14][used];
 // gains complex64 [slots][NR][L][taps][14]; delays [slots][taps].
-//
-// A bin's phasor of tap tau is P[a] Q[b] with bin = 64 a + b: a wave works on
-// 64 bins of one a, so that a lane's b never changes and the products
-// gain P[a] of all layers and taps are formed once per wave (by its lanes) and
-// read back as broadcasts: 16 multiply-adds per bin and tap for 4 layers,
-// and 64 + N/64 sincos per tap in place of N.  The inverse DFT is the
-// demodulator's radix-16 Stockham FFT on conjugates (N = 4096: the first pass
-// takes the bins from the registers they were computed in).  Bound by vector
-// instructions: 16 full-carrier slots, 4 Rx, 16 taps (896 symbols): 144 ->
-// 66 us against a sincos per bin and tap and a radix-2 transform.
-template <int LOGN>
 __global__ void __launch_bounds__(256) ChannelOfdmKernel(const float2 *__restrict__ grid,
                                                          const float2 *__restrict__ gains,
-                                                         const float *__restrict__ delays, ChanArgs a,
+                                                         const float *__restrict__ delays,
+                                                         const float2 *__restrict__ twiddle, ChanArgs a,
                                                          void *__restrict__ iq)
 {
-    using namespace airan::fft;
-    constexpr uint32_t N = 1u << LOGN, TPS = N / 16, A = N / 64, B = (N + 255) / 256;
-    constexpr uint32_t kTaps = 32;
-    constexpr uint32_t kTables = 2 * kTaps * (64 + A) + 4 * 8 * kTaps, kFft = 2 * (N + N / 16);
-    __shared__ __align__(16) float mem[kTables > kFft ? kTables : kFft];
-    float2 *P = reinterpret_cast<float2 *>(mem), *Q = P + kTaps * A;  // [tap][a], [tap][b]
+    __shared__ float2 buf[kMaxFft];
+    __shared__ float2 gs[4][32];  // this symbol's tap gains per layer
+    __shared__ double tau[32];
     const uint32_t sym = blockIdx.x % 14u, rest = blockIdx.x / 14u;
     const uint32_t rx = rest % a.nr, slot = rest / a.nr;
-    const uint32_t t = threadIdx.x, lane = t & 63u;
-    float4 *gw = reinterpret_cast<float4 *>(Q + kTaps * 64) + (t >> 6) * 2 * kTaps;  // this wave's [tap][layer] gain P[a]
-    const float *tau = delays + static_cast<size_t>(slot) * a.taps;
-    for (uint32_t k = t; k < a.taps * (64u + A); k += 256u) {
-        const bool fine = k < a.taps * 64u;
-        const uint32_t i = fine ? k : k - a.taps * 64u, tp = fine ? i / 64u : i / A, x = fine ? i % 64u : i % A;
-        // Bins from N/2 on are the negative frequencies.
-        const int32_t bin = fine ? static_cast<int32_t>(x) : 64 * static_cast<int32_t>(x >= A / 2 ? x - A : x);
-        const float2 v = Phasor(static_cast<double>(bin) * static_cast<double>(a.scs) * static_cast<double>(tau[tp]));
-        (fine ? Q : P)[tp * (fine ? 64u : A) + x] = v;
+    const uint32_t t = threadIdx.x, n = a.fft;
+    for (uint32_t k = t; k < a.nl * a.taps; k += blockDim.x) {
+        const uint32_t l = k / a.taps, tp = k % a.taps;
+        gs[l][tp] = gains[((((static_cast<size_t>(slot) * a.nr + rx) * a.nl + l) * a.taps + tp) * 14u) + sym];
     }
-    // Lane 4 tp' + l of a wave: the gains of layer l, taps tp' and tp' + 16.
-    float2 g[2] = {make_float2(0.0f, 0.0f), make_float2(0.0f, 0.0f)};
-#pragma unroll
-    for (uint32_t h = 0; h < 2u; ++h) {
-        const uint32_t l = lane & 3u, tp = (lane >> 2) + 16u * h;
-        if (l < a.nl && tp < a.taps)
-            g[h] = gains[((((static_cast<size_t>(slot) * a.nr + rx) * a.nl + l) * a.taps + tp) * 14u) + sym];
-    }
+    for (uint32_t k = t; k < a.taps; k += blockDim.x) tau[k] = delays[static_cast<size_t>(slot) * a.taps + k];
     __syncthreads();
     const uint32_t half = a.used / 2u;
     const size_t gplane = static_cast<size_t>(14) * a.used;
     const float2 *gx = grid + static_cast<size_t>(slot) * a.nl * gplane + static_cast<size_t>(sym) * a.used;
-    float2 v[16];  // conjugates of the bins t + 256 m
-#pragma unroll
-    for (uint32_t m = 0; m < 16u; ++m) {
-        v[m] = make_float2(0.0f, 0.0f);
-        const uint32_t k = t + 256u * m;
-        if (m >= B || k >= N) continue;
+    for (uint32_t k = t; k < n; k += blockDim.x) {
         // Bin k carries subcarrier u = (k + used/2) mod N when u < used.
-        const uint32_t u = (k + half) & (N - 1u);
-        if (__ballot(u < a.used) == 0) continue;
-        float2 x[4];
-#pragma unroll
-        for (uint32_t l = 0; l < 4u; ++l)
-            x[l] = l < a.nl && u < a.used ? gx[static_cast<size_t>(l) * gplane + u] : make_float2(0.0f, 0.0f);
-        // gain P[a] of this wave's 64 bins (a uniform).
-        const uint32_t ka = __builtin_amdgcn_readfirstlane(k >> 6);
-#pragma unroll
-        for (uint32_t h = 0; h < 2u; ++h) {
-            const uint32_t tp = (lane >> 2) + 16u * h;
-            if (16u * h < a.taps) {
-                const float2 p = tp < a.taps ? P[tp * A + ka] : make_float2(0.0f, 0.0f);
-                reinterpret_cast<float2 *>(gw)[4u * tp + (lane & 3u)] =
-                    make_float2(g[h].x * p.x - g[h].y * p.y, g[h].x * p.y + g[h].y * p.x);
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        float hr[4] = {0.0f, 0.0f, 0.0f, 0.0f}, hi[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (uint32_t tp = 0; tp < a.taps; ++tp) {
-            const float2 q = Q[tp * 64u + lane];
-            const float4 g01 = gw[2u * tp], g23 = gw[2u * tp + 1u];
-            const float gr[4] = {g01.x, g01.z, g23.x, g23.z}, gi[4] = {g01.y, g01.w, g23.y, g23.w};
-#pragma unroll
-            for (uint32_t l = 0; l < 4u; ++l) {
-                hr[l] += gr[l] * q.x - gi[l] * q.y;
-                hi[l] += gr[l] * q.y + gi[l] * q.x;
-            }
-        }
+        const uint32_t u = (k + half) & (n - 1u);
         float2 y = make_float2(0.0f, 0.0f);
+        if (u < a.used) {
+            const double f = (static_cast<double>(u) - static_cast<double>(half)) * static_cast<double>(a.scs);
+            float hr[4] = {0.0f, 0.0f, 0.0f, 0.0f}, hi[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (uint32_t tp = 0; tp < a.taps; ++tp) {
+                // e^(-j 2 pi f tau), the phase reduced to (-1/2, 1/2] cycles in fp64.
+                const double cyc = f * tau[tp];
+                const float frac = static_cast<float>(cyc - rint(cyc));
+                float sn, cs;
+                sincospif(2.0f * frac, &sn, &cs);
 #pragma unroll
-        for (uint32_t l = 0; l < 4u; ++l) {
-            y.x += hr[l] * x[l].x - hi[l] * x[l].y;
-            y.y += hr[l] * x[l].y + hi[l] * x[l].x;
-        }
-        v[m] = make_float2(y.x, -y.y);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    }
-    __syncthreads();  // the tables are done with: the transform takes their place
-    float *lre = mem, *lim = mem + N + N / 16;
-    const bool active = t < TPS;
-    if constexpr (LOGN < 12) {
+                for (uint32_t l = 0; l < 4; ++l) {
+                    if (l < a.nl) {
+                        const float2 gv = gs[l][tp];
+                        hr[l] += gv.x * cs + gv.y * sn;
+                        hi[l] += gv.y * cs - gv.x * sn;
+                    }
+                }
+            }
 #pragma unroll
-        for (uint32_t m = 0; m < B; ++m) {
-            const uint32_t k = t + 256u * m;
-            if (k < N) {
-                lre[Pad(k)] = v[m].x;
-                lim[Pad(k)] = v[m].y;
+            for (uint32_t l = 0; l < 4; ++l) {
+                if (l < a.nl) {
+                    const float2 x = gx[static_cast<size_t>(l) * gplane + u];
+                    y.x += hr[l] * x.x - hi[l] * x.y;
+                    y.y += hr[l] * x.y + hi[l] * x.x;
+                }
             }
         }
-        __syncthreads();
-        if (active)
-#pragma unroll
-            for (uint32_t r = 0; r < 16u; ++r) v[r] = make_float2(lre[Pad(t + r * TPS)], lim[Pad(t + r * TPS)]);
-        __syncthreads();
-    }
-    if (active) {
-        Dft<16>(v);
-#pragma unroll
-        for (uint32_t r = 0; r < 16u; ++r) {
-            lre[Pad(t * 16u + r)] = v[r].x;
-            lim[Pad(t * 16u + r)] = v[r].y;
-        }
+        buf[__brev(k) >> (32u - a.log2n)] = y;
     }
     __syncthreads();
-    const float sc = a.inv_sqrt_n;
-    if constexpr (LOGN >= 8) LdsPass<LOGN, 16, LOGN == 8>(lre, lim, t, 16, active, sc);
-    if constexpr (LOGN == 12) LdsPass<LOGN, 16, true>(lre, lim, t, 256, active, sc);
-    constexpr uint32_t kDone = LOGN >= 8 ? 256 : 16;  // points per transform so far
-    if constexpr (LOGN % 4 == 1) LdsPass<LOGN, 2, true>(lre, lim, t, kDone, active, sc);
-    if constexpr (LOGN % 4 == 2) LdsPass<LOGN, 4, true>(lre, lim, t, kDone, active, sc);
-    if constexpr (LOGN % 4 == 3) LdsPass<LOGN, 8, true>(lre, lim, t, kDone, active, sc);
-
+    // Radix-2 decimation-in-time inverse DFT: e^(+j 2 pi k n / N).
+    for (uint32_t h = 1; h < n; h <<= 1) {
+        const uint32_t stride = n / (2u * h);
+        for (uint32_t b = t; b < n / 2u; b += blockDim.x) {
+            const uint32_t grp = b / h, pos = b - grp * h;
+            const uint32_t i0 = grp * 2u * h + pos, i1 = i0 + h;
+            const float2 w = twiddle[pos * stride];
+            const float2 v = buf[i1], uu = buf[i0];
+            const float2 vw = make_float2(v.x * w.x - v.y * w.y, v.x * w.y + v.y * w.x);
+            buf[i0] = make_float2(uu.x + vw.x, uu.y + vw.y);
+            buf[i1] = make_float2(uu.x - vw.x, uu.y - vw.y);
+        }
+        __syncthreads();
+    }
     const uint32_t cp = a.cp[sym], first = a.start[sym] - cp;
     const size_t row = (static_cast<size_t>(slot) * a.nr + rx) * a.samples;
-    constexpr uint64_t kStep = 0x632be59bd9b4e019ull;
-    uint64_t key = (row + first + t) * kStep;
-    for (uint32_t p = t; p < cp + N; p += 256u, key += 256u * kStep) {
-        const uint32_t n = Pad(p < cp ? N - cp + p : p - cp);
-        const float2 z = Gauss2(a.seed ^ key);
-        const float re = lre[n] + a.sigma * z.x, im = a.sigma * z.y - lim[n];
-        const size_t pos = row + first + p;
+    for (uint32_t p = t; p < cp + n; p += blockDim.x) {
+        const float2 v = buf[p < cp ? n - cp + p : p - cp];
+        const uint64_t pos = row + first + p;
+        const float2 z = Gauss2(a.seed ^ (pos * 0x632be59bd9b4e019ull));
+        const float re = v.x * a.inv_sqrt_n + a.sigma * z.x, im = v.y * a.inv_sqrt_n + a.sigma * z.y;
         if (a.iq_float) {
             static_cast<float2 *>(iq)[pos] = make_float2(re, im);
         } else {
@@ -746,6 +674,7 @@ struct AiranPuschTxGpu {
     uint32_t max_tbs = 0, T = 1;
     uint32_t tb_chunks = 0, cb_chunks = 0, tb_parts = 0;
     uint32_t *tb_part = nullptr, *pow_tb = nullptr, *pow_cb = nullptr, *gold = nullptr;
+    float2 *twiddle = nullptr;
 };
 
 extern "C" {
@@ -806,16 +735,22 @@ int32_t airan_pusch_txgpu_Create(const PuschMimoConfig *config, const AiranTbPla
         p.G / 32u + 2u);
     const std::vector<uint32_t> ptb = ChunkPowers(t->tb_chunks, kTbChunkBits, tp.tb_poly, tp.tb_len);
     const std::vector<uint32_t> pcb = ChunkPowers(t->cb_chunks, kCbChunkBits, kPolyB, 24);
+    std::vector<float2> tw(g.fft / 2);
+    for (uint32_t k = 0; k < g.fft / 2; ++k) {
+        const double ph = 2.0 * M_PI * static_cast<double>(k) / static_cast<double>(g.fft);
+        tw[k] = make_float2(static_cast<float>(std::cos(ph)), static_cast<float>(std::sin(ph)));
+    }
     auto alloc = [](auto **ptr, size_t bytes) { return hipMalloc(reinterpret_cast<void **>(ptr), bytes) == hipSuccess; };
     if (!alloc(&t->tb_part, sizeof(uint32_t) * max_tbs * t->tb_parts) ||
         !alloc(&t->pow_tb, sizeof(uint32_t) * t->tb_chunks) || !alloc(&t->pow_cb, sizeof(uint32_t) * t->cb_chunks) ||
-        !alloc(&t->gold, sizeof(uint32_t) * gold.size()))
+        !alloc(&t->gold, sizeof(uint32_t) * gold.size()) || !alloc(&t->twiddle, sizeof(float2) * tw.size()))
         return fail(AIRAN_RESOURCE_TOO_SMALL);
     if (hipMemcpy(t->pow_tb, ptb.data(), sizeof(uint32_t) * ptb.size(), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(t->pow_cb, pcb.data(), sizeof(uint32_t) * pcb.size(), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(t->gold, gold.data(), sizeof(uint32_t) * gold.size(), hipMemcpyHostToDevice) != hipSuccess)
+        hipMemcpy(t->gold, gold.data(), sizeof(uint32_t) * gold.size(), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(t->twiddle, tw.data(), sizeof(float2) * tw.size(), hipMemcpyHostToDevice) != hipSuccess)
         return fail(AIRAN_LAUNCH_FAILED);
-    if ((st = airan::InitGoldTables()) != AIRAN_OK || (st = airan::InitOfdmTables()) != AIRAN_OK) return fail(st);
+    if ((st = airan::InitGoldTables()) != AIRAN_OK) return fail(st);
     *tx = t;
     return AIRAN_OK;
 }
@@ -827,6 +762,7 @@ void airan_pusch_txgpu_Destroy(AiranPuschTxGpu *t)
     FreeDev(t->pow_tb);
     FreeDev(t->pow_cb);
     FreeDev(t->gold);
+    FreeDev(t->twiddle);
     delete t;
 }
 
@@ -883,10 +819,14 @@ int32_t airan_pusch_txgpu_Channel(AiranPuschTxGpu *t, const float *grid, uint32_
         (iq_format != AIRAN_IQ_INT16_Q8_8 && iq_format != AIRAN_IQ_COMPLEX64))
         return AIRAN_INVALID_ARGUMENT;
     const Geom &g = t->g;
+    if (g.fft > kMaxFft) return AIRAN_UNSUPPORTED_PROFILE;
     ChanArgs a{};
     a.nr = g.nr;
     a.nl = g.nl;
     a.used = g.used;
+    a.fft = g.fft;
+    a.log2n = 0;
+    while ((1u << a.log2n) < g.fft) ++a.log2n;
     a.taps = taps;
     a.samples = g.samples;
     a.iq_float = iq_format == AIRAN_IQ_COMPLEX64;
@@ -898,19 +838,9 @@ int32_t airan_pusch_txgpu_Channel(AiranPuschTxGpu *t, const float *grid, uint32_
     a.sigma = std::sqrt(noise_var * 0.5f);
     a.inv_sqrt_n = 1.0f / std::sqrt(static_cast<float>(g.fft));
     a.seed = seed;
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(slots * g.nr * 14u), dim3(256), 0, static_cast<hipStream_t>(stream),
-                           reinterpret_cast<const float2 *>(grid), reinterpret_cast<const float2 *>(gains), delays, a, iq);
-    };
-    switch (g.fft) {
-    case 128: launch(ChannelOfdmKernel<7>); break;
-    case 256: launch(ChannelOfdmKernel<8>); break;
-    case 512: launch(ChannelOfdmKernel<9>); break;
-    case 1024: launch(ChannelOfdmKernel<10>); break;
-    case 2048: launch(ChannelOfdmKernel<11>); break;
-    case 4096: launch(ChannelOfdmKernel<12>); break;
-    default: return AIRAN_UNSUPPORTED_PROFILE;
-    }
+    hipLaunchKernelGGL(ChannelOfdmKernel, dim3(slots * g.nr * 14u), dim3(256), 0, static_cast<hipStream_t>(stream),
+                       reinterpret_cast<const float2 *>(grid), reinterpret_cast<const float2 *>(gains), delays,
+                       t->twiddle, a, iq);
     return airan::LaunchStatus();
 }
 
