@@ -7,10 +7,10 @@
 // (int16 value < 0) (:719-780), i.e. a REF-mode posterior in [-0.5, 0)
 // decodes to 0.
 //
-// Two kernels.  LdpcPairKernel (FP16 messages, at most 8 active rows): two
-// code blocks per workgroup, one in each fp16 half of every posterior word.
-// LdpcCheckPairKernel (the rest): one code block per workgroup, two checks
-// of it per lane.  In both the posterior lives in LDS, the message state in
+// Two kernels.  LdpcPairKernel (FP16 messages, at most 8 active rows, Z < 384
+// mainly; UsePair has the rule): two code blocks per workgroup, one in each
+// fp16 half of every posterior word.  LdpcCheckPairKernel (the rest): one code
+// block per workgroup, two checks of it per lane.  In both the posterior lives in LDS, the message state in
 // registers, a thread owns the same checks of every row (within a row the
 // threads touch a permutation of each column, so nothing conflicts) and a
 // barrier separates rows.
@@ -1069,20 +1069,17 @@ __device__ __forceinline__ uint32_t HalfIndex(uint32_t t, uint32_t z, uint32_t z
 // otherwise each position gathers its LLRs.  Ends before the barrier that
 // makes the posterior visible.
 __device__ inline void CheckLoadCodeword(uint32_t *lam, uint32_t z, uint32_t nl, const int16_t *__restrict__ cw,
-                                         const airan::RaggedCb &c, const airan::RaggedGrant &gr)
+                                         const airan::RateCb &rc, const airan::RateDev &r)
 {
     const uint32_t i = threadIdx.x, nt = blockDim.x, zh = z / 2;
     uint16_t *lam16 = reinterpret_cast<uint16_t *>(lam);
-    const airan::RateDev r{gr.g.qm, gr.g.cw_symbols, gr.g.cw_stride, z, c.kprime, c.filler, c.ncb, 1};
-    const airan::RateCb rc = airan::RateCbSetup({c.e, c.k0, c.ncb, c.cw_symbol_offset}, r);
-    const int16_t *src = cw + gr.cw_off;
     if (!airan::RateSingle(rc, r)) {
         for (uint32_t t = i; t < nl; t += nt)
-            lam16[HalfIndex(t, z, zh)] = static_cast<uint16_t>(InputH(airan::RateDematchValue(t, rc, r, src)));
+            lam16[HalfIndex(t, z, zh)] = static_cast<uint16_t>(InputH(airan::RateDematchValue(t, rc, r, cw)));
         return;
     }
     const uint32_t two_z = 2u * z, fstart = r.kprime - two_z, nf = r.ncb - r.filler;
-    const int16_t *slot = src + static_cast<size_t>(rc.slot0) * r.qm * r.cw_stride;
+    const int16_t *slot = cw + static_cast<size_t>(rc.slot0) * r.qm * r.cw_stride;
     for (uint32_t t = i; t < nl / 2u; t += nt) lam[t] = 0;
     __syncthreads();
     for (uint32_t t = two_z + fstart + i; t < min(nl, two_z + fstart + r.filler); t += nt)
@@ -1138,16 +1135,21 @@ __device__ inline void CheckLoadCodeword(uint32_t *lam, uint32_t z, uint32_t nl,
 
 constexpr uint32_t kCheckThreads = 192;
 
-// MAXROWS: kFewRows or kRows.  RAGGED: block b decodes code block list[b] of a
-// ragged batch, reading the grant's bit-plane codeword LLRs (src) itself (the
-// standalone rate-dematch arithmetic), with that block's Z, K and rows (no
-// lam_out); otherwise src holds the decoder LLRs [cb][68 Z].
-template <int MODE, int MAXROWS, uint32_t ZT, bool RAGGED>
+// Where a block's LLRs come from: decoder LLRs [cb][68 Z] in src; or bit-plane
+// codeword LLRs (the standalone rate-dematch arithmetic, no lam_out), of code
+// block list[b] of a ragged batch with that block's Z, K and rows, or of block
+// b of a chain's batch by its descriptor.
+constexpr int kSrcLlr = 0, kSrcRagged = 1, kSrcChain = 2;
+
+// MAXROWS: kFewRows or kRows.
+template <int MODE, int MAXROWS, uint32_t ZT, int SRC>
 __global__ void __launch_bounds__(kCheckThreads) __attribute__((amdgpu_waves_per_eu(MAXROWS <= kFewRows ? 3 : 2)))
     LdpcCheckPairKernel(const int16_t *__restrict__ src, int8_t *__restrict__ bits, int16_t *__restrict__ lam_out,
                         uint8_t *__restrict__ iters_out, LdpcDev d, const airan::RaggedCb *__restrict__ cbs,
-                        const airan::RaggedGrant *__restrict__ grants, const uint32_t *__restrict__ list)
+                        const airan::RaggedGrant *__restrict__ grants, const uint32_t *__restrict__ list,
+                        const RateMatchDescriptor *__restrict__ desc, airan::RateDev rate)
 {
+    constexpr bool RAGGED = SRC == kSrcRagged;
     constexpr bool kFull = MAXROWS <= kFewRows;  // every message of rows 4 .. 9 kept
     constexpr int kCoreEdges = AIRAN_BG1_ROW_START[4];
     constexpr int kExtEdges = AIRAN_BG1_ROW_START[kStaticRows] - kCoreEdges;
@@ -1177,7 +1179,12 @@ __global__ void __launch_bounds__(kCheckThreads) __attribute__((amdgpu_waves_per
     uint16_t *lam16 = reinterpret_cast<uint16_t *>(lam);
     if (i < 3) vote[i] = 0;
     if constexpr (RAGGED) {
-        CheckLoadCodeword(lam, Z, nl, src, cbs[cb], grants[cbs[cb].grant]);
+        const airan::RaggedCb &c = cbs[cb];
+        const airan::RaggedGrant &gr = grants[c.grant];
+        const airan::RateDev r{gr.g.qm, gr.g.cw_symbols, gr.g.cw_stride, Z, c.kprime, c.filler, c.ncb, 1};
+        CheckLoadCodeword(lam, Z, nl, src + gr.cw_off, airan::RateCbSetup({c.e, c.k0, c.ncb, c.cw_symbol_offset}, r), r);
+    } else if constexpr (SRC == kSrcChain) {
+        CheckLoadCodeword(lam, Z, nl, src, airan::RateCbSetup(desc[cb], rate), rate);
     } else {
         const int16_t *s = src + static_cast<size_t>(cb) * 68u * Z;
         if ((reinterpret_cast<uintptr_t>(src) & 7u) == 0) {
@@ -1280,7 +1287,7 @@ __global__ void __launch_bounds__(kCheckThreads) __attribute__((amdgpu_waves_per
         for (uint32_t t = i; t < d.k; t += kCheckThreads)
             bo[t] = static_cast<int8_t>(HardBits2<MODE>(lam16[HalfIndex(t, Z, zh)]) & 1u);
     }
-    if (!RAGGED && lam_out != nullptr) {
+    if (SRC == kSrcLlr && lam_out != nullptr) {
         const int16_t *s = src + static_cast<size_t>(cb) * 68u * Z;
         int16_t *lo = lam_out + static_cast<size_t>(cb) * 68u * Z;
         const float clip = MODE == AIRAN_LDPC_MODE_REF ? 5120.0f : 20.0f;
@@ -1317,11 +1324,11 @@ void LaunchPair(uint32_t rows, uint32_t threads, size_t lds, hipStream_t s, cons
 {
     using Kern = void (*)(const int16_t *, const RateMatchDescriptor *, int8_t *, int16_t *, uint8_t *, LdpcFastDev,
                           uint32_t *);
-    // Z = 384 (every PUSCH profile here): edges folded at compile time.
+    // Z = 384: edges folded at compile time (UsePair: 7 and 8 rows only).
     const bool z384 = d.z == 384;
-    Kern k = rows <= 4 ? (z384 ? LdpcPairKernel<FUSED, 4, 384> : LdpcPairKernel<FUSED, 4, 0>)
-           : rows == 5 ? (z384 ? LdpcPairKernel<FUSED, 5, 384> : LdpcPairKernel<FUSED, 5, 0>)
-           : rows == 6 ? (z384 ? LdpcPairKernel<FUSED, 6, 384> : LdpcPairKernel<FUSED, 6, 0>)
+    Kern k = rows <= 4 ? LdpcPairKernel<FUSED, 4, 0>
+           : rows == 5 ? LdpcPairKernel<FUSED, 5, 0>
+           : rows == 6 ? LdpcPairKernel<FUSED, 6, 0>
            : rows == 7 ? (z384 ? LdpcPairKernel<FUSED, 7, 384> : LdpcPairKernel<FUSED, 7, 0>)
                        : (z384 ? LdpcPairKernel<FUSED, 8, 384> : LdpcPairKernel<FUSED, 8, 0>);
     lds = z384 ? 0 : lds + kPairTailWords * sizeof(uint32_t);
@@ -1337,6 +1344,31 @@ bool FastEligible(uint32_t mode, uint32_t z, uint32_t rows)
     return mode == AIRAN_LDPC_MODE_FP16 && rows <= static_cast<uint32_t>(kFastRows) && z >= 24 && z <= 384;
 }
 
+// FP16 messages, at most kFastRows rows: two blocks a workgroup (the pair
+// decoder) or one block with two checks a lane (LdpcCheckPairKernel).
+// Z < 384: the pair; the check pair has 192 lanes for Z / 2 pairs of checks (2048 blocks of Z = 96, 6 rows: pair
+// 82 us, check pair 193).  Z = 384: the check pair, whose blocks take and
+// leave a compute unit one by one: us without early stop, pair / check pair,
+//   rows   128 blocks  600      4000      (8 iterations, launch included)
+//    4      61 / 52     90 / 81   -
+//    6      72 / 59    105 / 93   -
+//    8      81 / 70    156 / 110  635 / 435
+// and with early stop ahead at every count (8 rows, 300 blocks: 54 / 51).
+// The exception is between one and two blocks a compute unit with every
+// iteration run, where the pair's one workgroup a unit is the shorter of two
+// equal waits (7 rows, 300 blocks: 75 / 79; 8 rows 82 / 85; 6 rows 73 / 71).
+bool UsePair(uint32_t z, uint32_t rows, uint32_t num_cb, bool early_stop)
+{
+    if (z != 384) return true;
+    if (early_stop || rows < 7) return false;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return false;
+    const uint32_t n = static_cast<uint32_t>(std::max(cus, 0));
+    return num_cb > n && num_cb <= 2u * n;
+}
+
 uint32_t LiftIndex(uint32_t z)
 {
     uint32_t zi = 0;
@@ -1350,12 +1382,12 @@ void LaunchCheckPair(const LdpcDecodeOpArgsV1 *a, hipStream_t s)
     const LdpcDev d{a->z, LiftIndex(a->z), a->k, a->max_iterations, a->active_rows, a->early_stop ? 1u : 0u};
     const bool few = a->active_rows <= static_cast<uint32_t>(kFewRows), z384 = a->z == 384;
     using Kern = void (*)(const int16_t *, int8_t *, int16_t *, uint8_t *, LdpcDev, const airan::RaggedCb *,
-                          const airan::RaggedGrant *, const uint32_t *);
-    const Kern k = few ? (z384 ? LdpcCheckPairKernel<MODE, kFewRows, 384, false> : LdpcCheckPairKernel<MODE, kFewRows, 0, false>)
-                       : (z384 ? LdpcCheckPairKernel<MODE, kRows, 384, false> : LdpcCheckPairKernel<MODE, kRows, 0, false>);
+                          const airan::RaggedGrant *, const uint32_t *, const RateMatchDescriptor *, airan::RateDev);
+    const Kern k = few ? (z384 ? LdpcCheckPairKernel<MODE, kFewRows, 384, kSrcLlr> : LdpcCheckPairKernel<MODE, kFewRows, 0, kSrcLlr>)
+                       : (z384 ? LdpcCheckPairKernel<MODE, kRows, 384, kSrcLlr> : LdpcCheckPairKernel<MODE, kRows, 0, kSrcLlr>);
     hipLaunchKernelGGL(k, dim3(a->num_cb), dim3(kCheckThreads), 0, s, static_cast<const int16_t *>(a->lam_in),
                        static_cast<int8_t *>(a->bits), static_cast<int16_t *>(a->lam_out),
-                       static_cast<uint8_t *>(a->iterations_out), d, nullptr, nullptr, nullptr);
+                       static_cast<uint8_t *>(a->iterations_out), d, nullptr, nullptr, nullptr, nullptr, airan::RateDev{});
 }
 
 // The decoder operator (validated arguments).
@@ -1366,7 +1398,8 @@ int32_t LaunchDecode(const LdpcDecodeOpArgsV1 *a)
     const auto *in = static_cast<const int16_t *>(a->lam_in);
     auto *bits = static_cast<int8_t *>(a->bits);
     const bool aligned = (reinterpret_cast<uintptr_t>(in) & 7u) == 0 && (reinterpret_cast<uintptr_t>(bits) & 3u) == 0;
-    if (aligned && FastEligible(a->mode, a->z, a->active_rows)) {
+    if (aligned && FastEligible(a->mode, a->z, a->active_rows) &&
+        UsePair(a->z, a->active_rows, a->num_cb, a->early_stop != 0)) {
         if ((st = LoadLiftTable()) != AIRAN_OK) return st;
         const uint32_t rows = a->active_rows;  // validated >= 4
         LdpcFastDev fd{a->z, LiftIndex(a->z), a->k, a->max_iterations, rows, a->early_stop ? 1u : 0u, a->num_cb, {}};
@@ -1452,11 +1485,11 @@ int32_t LaunchLdpcRagged(const RaggedCb *cbs, const RaggedGrant *grants, const R
     auto launch = [&](auto kernel, const RaggedLdpcList &l) {
         if (l.count > 0)
             hipLaunchKernelGGL(kernel, dim3(l.count), dim3(kCheckThreads), 0, s, cw, bits, nullptr, iters_out, d, cbs,
-                               grants, l.list);
+                               grants, l.list, nullptr, RateDev{});
     };
-    launch(LdpcCheckPairKernel<kMode, kRows, 384, true>, many);
-    launch(LdpcCheckPairKernel<kMode, kFewRows, 384, true>, few);
-    launch(LdpcCheckPairKernel<kMode, kRows, 0, true>, other);
+    launch(LdpcCheckPairKernel<kMode, kRows, 384, kSrcRagged>, many);
+    launch(LdpcCheckPairKernel<kMode, kFewRows, 384, kSrcRagged>, few);
+    launch(LdpcCheckPairKernel<kMode, kRows, 0, kSrcRagged>, other);
     return LaunchStatus();
 }
 
@@ -1479,8 +1512,16 @@ int32_t LaunchLdpcFromCodeword(const Geom &g, const AiranTbPlanV1 &p, const Rate
         (p.Z % 24) != 0 || p.K == 0 || p.K > 22 * p.Z || p.Ncb <= p.filler || (reinterpret_cast<uintptr_t>(bits) & 3u) ||
         p.E_low >= (1u << 22) || p.E_high >= (1u << 22))
         return AIRAN_UNSUPPORTED_PROFILE;
-    int32_t st = LoadLiftTable();
-    if (st != AIRAN_OK) return st;
+    int32_t st;
+    if (!UsePair(p.Z, rows, num_cb, early_stop)) {
+        if ((st = LoadEdgeTable()) != AIRAN_OK) return st;
+        const LdpcDev d{p.Z, LiftIndex(p.Z), p.K, iters, rows, early_stop ? 1u : 0u};
+        const RateDev r{g.qm, g.cw_symbols, g.cw_stride, p.Z, p.Kprime, p.filler, p.Ncb, num_cb};
+        hipLaunchKernelGGL((LdpcCheckPairKernel<AIRAN_LDPC_MODE_FP16, kFewRows, 384, kSrcChain>), dim3(num_cb),
+                           dim3(kCheckThreads), 0, s, cw, bits, nullptr, iters_out, d, nullptr, nullptr, nullptr, desc, r);
+        return LaunchStatus();
+    }
+    if ((st = LoadLiftTable()) != AIRAN_OK) return st;
     LdpcFastDev fd{p.Z, LiftIndex(p.Z), p.K, iters, rows, early_stop ? 1u : 0u, num_cb,
                    {g.qm, g.cw_symbols, g.cw_stride, p.Z, p.Kprime, p.filler, p.Ncb, num_cb}};
     const size_t lds = static_cast<size_t>(22 + rows) * p.Z * sizeof(uint32_t);

@@ -1,5 +1,5 @@
-"""The decoder kernel of one code block per workgroup (REF mode, more than 8
-active rows, unaligned buffers) bit for bit against the oracle where it can go
+"""The decoder kernel of one code block per workgroup (Z = 384, REF mode, more
+than 8 active rows, unaligned buffers) bit for bit against the oracle where it can go
 wrong: every lifting size (the halves of 12 .. 192 words), the row counts at
 which its unrolled rows, its two register arrays and its kernels end, buffers
 of any alignment, a K that is no multiple of 4, and int16 inputs large enough
@@ -66,3 +66,56 @@ def test_full_range_inputs(gpu_stream, mode, rows):
     lam = rng.integers(-32768, 32768, (4, 68 * 96)).astype(np.int16)
     lam[3] = np.where(rng.integers(0, 2, 68 * 96), 32767, -32768)
     _check(lam.reshape(-1), 4, 96, 22 * 96, 20, rows, mode, True, want_lam=False)
+
+
+@pytest.mark.parametrize("rows", [4, 5, 6, 7, 8])
+@pytest.mark.parametrize("n,early", [(3, True), (300, False), (300, True), (520, False)])
+def test_few_rows_at_every_dispatch(gpu_stream, rows, n, early):
+    """Z = 384 and at most 8 rows: one block per workgroup, or two between one
+    and two blocks a compute unit without early stop.  Three distinct blocks,
+    repeated: every repetition decodes alike."""
+    z, k = 384, 22 * 384
+    lam = _llrs(z, 3, rows, 4.0, rows)
+    oracle = load_oracle()
+    ref = lam.copy()
+    bits, it = np.zeros(3 * k, np.int8), np.zeros(3, np.uint8)
+    oracle.or_ldpc_decode(z, 3, ptr(ref), abi.LDPC_MODE_FP16, 4, rows, k, 1 if early else 0, ptr(bits), ptr(it))
+    reps = -(-n // 3)
+    dev = torch.from_numpy(np.tile(lam.reshape(3, -1), (reps, 1))[:n].copy()).cuda().reshape(-1)
+    got, lam_out, git = ops.ldpc_decode(dev, n, z, k, 4, rows, abi.LDPC_MODE_FP16, early, want_lam=True)
+    torch.cuda.synchronize()
+    tile = lambda a: np.tile(a.reshape(3, -1), (reps, 1))[:n]  # noqa: E731
+    assert np.array_equal(git.cpu().numpy(), tile(it).reshape(-1))
+    assert np.array_equal(got.cpu().numpy().reshape(n, -1), tile(bits))
+    assert np.array_equal(lam_out.cpu().numpy().reshape(n, -1), tile(ref))
+
+
+@pytest.mark.parametrize("rank,qm,rate", [(4, 8, 0.85), (3, 6, 0.91), (2, 4, 0.93), (1, 8, 0.8)])
+def test_chain_blocks_match_operators(gpu_stream, rank, qm, rate):
+    """The decoder reading a chain's codeword LLRs itself against rate dematch
+    + decoder as operators."""
+    from puschrx import profiles as P
+    from puschrx.chain import ChainOptions, NativeChain
+    prof = P.Profile(name="t", rx=4, rank=rank, num_rb=51, fft=1024, qm=qm, code_rate=rate)
+    cfg = prof.config()
+    g = ops.Geometry(cfg)
+    tbs = ops.tbs(51, 12 * g.ndata, qm, rank, rate)
+    plan = ops.tb_plan(tbs, g.cw_symbols * qm, qm, rank)
+    assert plan.Z == 384 and ops.ldpc_active_rows(plan) <= 8  # the fused decoder's shape
+    n = 3
+    rng = np.random.default_rng(rank)
+    iq = torch.from_numpy(rng.normal(0, 1, (n, g.nr, g.samples, 2)).astype(np.float32)).cuda()
+    for early in (1, 0):
+        opts = ChainOptions(tau_s=100e-9, fd_hz=10.0, iq_format=abi.IQ_COMPLEX64, early_stop=early)
+        chain = NativeChain(cfg, plan, max_slots=n, opts=opts, use_graph=False)
+        chain.enqueue(iq, n)
+        cw = chain.fetch("cw_llr", torch.int16, n * qm * g.cw_stride).reshape(n, -1)
+        bits = chain.fetch("bits", torch.int8, 3 * plan.C * plan.K).cpu().numpy().reshape(3, -1)
+        torch.cuda.synchronize()
+        for t in range(3):
+            lam = ops.rate_dematch(cfg, cw[t].contiguous(), 1, plan)
+            want, _, _ = ops.ldpc_decode(lam, plan.C, plan.Z, plan.K, opts.ldpc_iterations, ops.ldpc_active_rows(plan),
+                                         abi.LDPC_MODE_FP16, bool(early))
+            torch.cuda.synchronize()
+            assert np.array_equal(bits[t], want.cpu().numpy()), t
+        chain.close()
