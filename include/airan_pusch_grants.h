@@ -16,9 +16,10 @@
  *                           and the CE prior); one launch per CE step over
  *                           every shape, each shape's grants together
  *   detect + demap + descramble   one launch over (grant, symbol, tile) items
- *   rate dematch            one launch over all code blocks
- *   LDPC (FP16 messages)    one launch over the code blocks with <= 8 active
- *                           rows, one over the rest
+ *   LDPC (FP16 messages)    de-rate-matches while loading each code block;
+ *                           one launch over the blocks of Z = 384 with more
+ *                           than 10 active rows, one over those with fewer,
+ *                           one over the other lifting sizes
  *   CRC                     one launch over all code blocks + one per TB
  *
  * replayed from one HIP graph per batch.  Every stage computes what the
