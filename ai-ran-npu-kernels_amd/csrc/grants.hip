@@ -197,9 +197,9 @@ struct AiranGrantBatch {
     uint32_t n_tiles = 0, tile = 256;
     std::vector<RaggedTile> host_tiles_src;  // (grant, ds, used) per row, for rebuilding tiles
     RaggedCb *cbs = nullptr;
-    uint32_t *many_list = nullptr, *few_list = nullptr, *other_list = nullptr;  // decoder launches
+    uint32_t *many_list = nullptr, *few_list = nullptr, *other_list = nullptr, *any_list = nullptr;  // decoder launches
     uint32_t *tb_first = nullptr, *tb_count = nullptr;
-    uint32_t n_many = 0, n_few = 0, n_other = 0;
+    uint32_t n_many = 0, n_few = 0, n_other = 0, n_any = 0;
     // CE groups: grants of one shape, adjacent in the channel buffers.
     struct CeGroup {
         ShapeKey key;
@@ -273,8 +273,8 @@ int32_t EnqueueStages(AiranGrantBatch *b, const void *iq, hipStream_t s)
     if ((st = airan::LaunchStatus()) != AIRAN_OK) return st;
     const uint32_t ncb = static_cast<uint32_t>(b->num_cb);
     if ((st = airan::LaunchLdpcRagged(b->cbs, b->grants, {b->many_list, b->n_many}, {b->few_list, b->n_few},
-                                      {b->other_list, b->n_other}, b->opts.ldpc_iterations, b->opts.early_stop != 0,
-                                      b->cw, b->bits, b->iters, s)) != AIRAN_OK)
+                                      {b->other_list, b->n_other}, {b->any_list, b->n_any}, b->opts.ldpc_iterations,
+                                      b->opts.early_stop != 0, b->cw, b->bits, b->iters, s)) != AIRAN_OK)
         return st;
     return airan::LaunchCrcRagged(b->cbs, ncb, b->bits, b->cb_ok, b->tb_part, b->tb_first, b->tb_count, b->tb_ok,
                                   b->n, s);
@@ -423,7 +423,7 @@ int32_t airan_pusch_grants_Create(const PuschMimoConfig *configs, const AiranTbP
     std::map<uint32_t, std::vector<RaggedStream>> streams;
     std::vector<RaggedItem> gen, ls, nz;
     std::vector<RaggedCb> cbs;
-    std::vector<uint32_t> many, few, other, tb_first(n), tb_count(n);
+    std::vector<uint32_t> many, few, other, any, tb_first(n), tb_count(n);
     for (uint32_t i = 0; i < n; ++i) {
         const Geom &g = geom[i];
         const AiranTbPlanV1 &p = plans[i];
@@ -459,7 +459,8 @@ int32_t airan_pusch_grants_Create(const PuschMimoConfig *configs, const AiranTbP
             c.len_tb = p.crc_tb;
             c.poly_tb = airan::CrcTbPoly(p.crc_tb);
             c.xpow = airan::CrcXpowHost(p, r);
-            (p.Z != 384 ? other : rows > airan::LdpcFewRows() ? many : few).push_back(static_cast<uint32_t>(cbs.size()));
+            (!airan::LdpcLiftSize(p.Z) ? any : p.Z != 384 ? other : rows > airan::LdpcFewRows() ? many : few)
+                .push_back(static_cast<uint32_t>(cbs.size()));
             cbs.push_back(c);
         }
     }
@@ -479,14 +480,16 @@ int32_t airan_pusch_grants_Create(const PuschMimoConfig *configs, const AiranTbP
     b->n_noise = static_cast<uint32_t>(nz.size());
     // The decoder's longest blocks (most rows) first, so that the launch ends
     // with short ones.
-    for (std::vector<uint32_t> *l : {&many, &few, &other})
+    for (std::vector<uint32_t> *l : {&many, &few, &other, &any})
         std::stable_sort(l->begin(), l->end(), [&](uint32_t x, uint32_t y) { return cbs[x].rows > cbs[y].rows; });
     b->n_many = static_cast<uint32_t>(many.size());
     b->n_few = static_cast<uint32_t>(few.size());
     b->n_other = static_cast<uint32_t>(other.size());
+    b->n_any = static_cast<uint32_t>(any.size());
     if (!Upload(&b->grants, rec, &by) || !Upload(&b->gen_items, gen, &by) || !Upload(&b->ls_items, ls, &by) ||
         !Upload(&b->noise_items, nz, &by) || !Upload(&b->cbs, cbs, &by) || !Upload(&b->many_list, many, &by) ||
-        !Upload(&b->few_list, few, &by) || !Upload(&b->other_list, other, &by) || !Upload(&b->tb_first, tb_first, &by) ||
+        !Upload(&b->few_list, few, &by) || !Upload(&b->other_list, other, &by) ||
+        !Upload(&b->any_list, any, &by) || !Upload(&b->tb_first, tb_first, &by) ||
         !Upload(&b->tb_count, tb_count, &by) || !DevAlloc(&b->rx_re, rx, &by) || !DevAlloc(&b->rx_im, rx, &by) ||
         !DevAlloc(&b->ref_re, ref, &by) || !DevAlloc(&b->ref_im, ref, &by) || !DevAlloc(&b->hls_re, hls, &by) ||
         !DevAlloc(&b->hls_im, hls, &by) || !DevAlloc(&b->noise_ls, noise, &by) ||
@@ -557,8 +560,8 @@ void airan_pusch_grants_Destroy(AiranGrantBatch *b)
         if (f.streams) (void)hipFree(f.streams);
     airan::DestroyCeGrouped(b->ce_grouped);
     if (b->ce_ws_all) (void)hipFree(b->ce_ws_all);
-    void *bufs[] = {b->grants, b->gen_items, b->ls_items, b->noise_items, b->tiles, b->cbs, b->many_list, b->few_list, b->other_list,
-                    b->tb_first, b->tb_count, b->rx_re, b->rx_im, b->ref_re, b->ref_im, b->hls_re, b->hls_im,
+    void *bufs[] = {b->grants, b->gen_items, b->ls_items, b->noise_items, b->tiles, b->cbs, b->many_list, b->few_list,
+                    b->other_list, b->any_list, b->tb_first, b->tb_count, b->rx_re, b->rx_im, b->ref_re, b->ref_im, b->hls_re, b->hls_im,
                     b->noise_ls, b->noise_ce, b->h_re, b->h_im, b->gold, b->cw,
                     b->bits, b->iters, b->cb_ok, b->tb_ok, b->tb_part};
     for (void *p : bufs)

@@ -130,15 +130,18 @@ int32_t LaunchDmrsRagged(const RaggedGrant *grants, const RaggedItem *gen_items,
 uint32_t HostDmrsCinit(const PuschMimoConfig &cfg, uint32_t symbol);
 // LDPC (FP16 messages) of the listed code blocks, from the grants' codeword
 // LLRs (rate dematch in the decoder's load): Z = 384 with more than
-// LdpcFewRows() rows, with at most as many, and blocks of other Z.
+// LdpcFewRows() rows, with at most as many, blocks of the smaller sizes 24 <<
+// zi (LdpcLiftSize), and of any other Z.
 struct RaggedLdpcList {
     const uint32_t *list = nullptr;
     uint32_t count = 0;
 };
 uint32_t LdpcFewRows();
+bool LdpcLiftSize(uint32_t z);
 int32_t LaunchLdpcRagged(const RaggedCb *cbs, const RaggedGrant *grants, const RaggedLdpcList &many,
-                         const RaggedLdpcList &few, const RaggedLdpcList &other, uint32_t iters, bool early_stop,
-                         const int16_t *cw, int8_t *bits, uint8_t *iters_out, hipStream_t s);
+                         const RaggedLdpcList &few, const RaggedLdpcList &other, const RaggedLdpcList &any,
+                         uint32_t iters, bool early_stop, const int16_t *cw, int8_t *bits, uint8_t *iters_out,
+                         hipStream_t s);
 // CRC24B of every code block and the CRC of every TB (tb_first / tb_count
 // index the blocks of each TB).
 int32_t LaunchCrcRagged(const RaggedCb *cbs, uint32_t num_cb, const int8_t *bits, uint8_t *cb_ok, uint32_t *tb_part,

@@ -761,6 +761,21 @@ int32_t LoadEdgeTable()
     return AIRAN_OK;
 }
 
+// Lifting sizes other than 24 << zi (plans made by hand may have any of 24 ..
+// 384): one check per lane, word j of a column holds position j in its low
+// half and zero in the high one, so that odd sizes work and no rotation is
+// needed.  Their edge words (word index col Z + shift mod Z in bits 0 .. 15,
+// Z - shift mod Z above) are made by each workgroup, in LDS.
+constexpr uint32_t kAnyZ = 1;  // as ZT
+constexpr uint32_t kMaxZ = 384;
+
+constexpr bool IsLiftSize(uint32_t z)
+{
+    for (int zi = 0; zi < kNumLift; ++zi)
+        if (z == 24u << zi) return true;
+    return false;
+}
+
 // LDS byte of an edge's word for the lane (4 i = i4) and the rotation that
 // puts check i's position into the low half.
 struct EdgeAt {
@@ -779,11 +794,21 @@ __device__ __forceinline__ EdgeAt StaticEdge(int e, uint32_t i4)
     return {(wrap ? i4 - 4u * zh : i4) + 4u * (AIRAN_BG1_COL[e] * zh + sh), wrap != hi ? 16u : 0u};
 }
 
-// The edge of table word w; zh4 = 2 Z.
+// The edge of table word w; zh4 = 2 Z (4 Z with one check per lane).
+template <uint32_t ZT>
 __device__ __forceinline__ EdgeAt TableEdge(uint32_t w, uint32_t i4, uint32_t zh4)
 {
+    if constexpr (ZT == kAnyZ) return {i4 + 4u * (w & 0xffffu) - (i4 >= 4u * (w >> 16) ? zh4 : 0u), 0u};
     const bool hi = (w >> 31) != 0, wrap = i4 >= ((w >> 16) & 0x3ffu);
     return {i4 + (w & 0xffffu) - (wrap ? zh4 : 0u), wrap != hi ? 16u : 0u};
+}
+
+// Word e of a table: scalar, also from LDS.
+template <uint32_t ZT>
+__device__ __forceinline__ uint32_t TableWord(const uint32_t *tab, uint32_t e)
+{
+    if constexpr (ZT == kAnyZ) return __builtin_amdgcn_readfirstlane(tab[e]);
+    return tab[e];
 }
 
 __device__ __forceinline__ uint32_t Rot16(uint32_t v, uint32_t rot) { return __builtin_amdgcn_alignbit(v, v, rot); }
@@ -863,10 +888,10 @@ __device__ __forceinline__ void FullRow(uint32_t *lam, const uint32_t *tab, uint
     constexpr int E0 = AIRAN_BG1_ROW_START[R], DEG = StaticDeg(R);
     uint32_t s1p, d12;
     auto edge = [&](int k, uint32_t i4) {
-        if constexpr (ZT != 0)
+        if constexpr (ZT == kMaxZ)
             return StaticEdge<ZT>(E0 + k, i4);
         else
-            return TableEdge(tab[E0 + k], i4, zh4);
+            return TableEdge<ZT>(TableWord<ZT>(tab, E0 + k), i4, zh4);
     };
     CheckRow<MODE, DEG>(
         lam, i4, inf_flag, s1p, d12, edge, [&](int k) { return msg[k]; },
@@ -884,10 +909,10 @@ __device__ __forceinline__ void PackedRow(uint32_t *lam, const uint32_t *tab, ui
     const uint32_t o1 = st[0], od = st[1], oe = st[2], os = st[3];
     uint32_t ne = 0, ns = 0;
     auto edge = [&](int k, uint32_t i4) {
-        if constexpr (ZT != 0)
+        if constexpr (ZT == kMaxZ)
             return StaticEdge<ZT>(E0 + k, i4);
         else
-            return TableEdge(tab[E0 + k], i4, zh4);
+            return TableEdge<ZT>(TableWord<ZT>(tab, E0 + k), i4, zh4);
     };
     CheckRow<MODE, DEG>(
         lam, i4, inf_flag, st[0], st[1], edge,
@@ -902,14 +927,14 @@ __device__ __forceinline__ void PackedRow(uint32_t *lam, const uint32_t *tab, ui
 
 // A row of the loop: state s1p, d12 and meta (edge k: sign bit k, minimum
 // flag bit 8 + k, and 16 above for the other check).  w: its edge words.
-template <int MODE, int DEG>
+template <int MODE, uint32_t ZT, int DEG>
 __device__ __forceinline__ void LoopRow(uint32_t *lam, const uint32_t *w, uint32_t i4, uint32_t zh4, uint32_t &s1p,
                                         uint32_t &d12, uint32_t &meta, uint32_t *inf_flag)
 {
     const uint32_t o1 = s1p, od = d12, om = meta;
     uint32_t nm = 0;
     CheckRow<MODE, DEG>(
-        lam, i4, inf_flag, s1p, d12, [&](int k, uint32_t i4) { return TableEdge(w[k], i4, zh4); },
+        lam, i4, inf_flag, s1p, d12, [&](int k, uint32_t i4) { return TableEdge<ZT>(w[k], i4, zh4); },
         [&](int k) { return PkMadU16((om >> (8 + k)) & 0x00010001u, od, o1) ^ ((om << (15 - k)) & 0x80008000u); },
         [&](int k, uint32_t x, uint32_t e, uint32_t) {
             nm |= e << (8 + k);
@@ -951,7 +976,7 @@ struct RowState {
 };
 
 // Rows r0 .. r0 + count - 1 of the loop.
-template <int MODE, int N>
+template <int MODE, uint32_t ZT, int N>
 __device__ __forceinline__ void LoopRows(uint32_t *lam, const uint32_t *tab, int r0, int count, bool mine, uint32_t i4,
                                          uint32_t zh4, RowState<N> &st, uint32_t *inf_flag)
 {
@@ -959,7 +984,7 @@ __device__ __forceinline__ void LoopRows(uint32_t *lam, const uint32_t *tab, int
     uint32_t info = kEdges.row[r0];
     uint32_t w[kMaxLoopDeg];
 #pragma unroll
-    for (int k = 0; k < kMaxLoopDeg; ++k) w[k] = tab[(info & 0xffffu) + k];
+    for (int k = 0; k < kMaxLoopDeg; ++k) w[k] = TableWord<ZT>(tab, (info & 0xffffu) + k);
 #pragma nounroll
     for (int j = 0; j < count; ++j) {
         // The next row's words, on their way while this row is worked on.
@@ -967,15 +992,15 @@ __device__ __forceinline__ void LoopRows(uint32_t *lam, const uint32_t *tab, int
         uint32_t nw[kMaxLoopDeg];
         const uint32_t ne0 = (info & 0xffffu) + (info >> 16);
 #pragma unroll
-        for (int k = 0; k < kMaxLoopDeg; ++k) nw[k] = tab[ne0 + k];
+        for (int k = 0; k < kMaxLoopDeg; ++k) nw[k] = TableWord<ZT>(tab, ne0 + k);
         if (mine) {
             uint32_t a = st.s1p[j], b = st.d12[j], c = st.meta[j];
             switch (info >> 16) {
-            case 4: LoopRow<MODE, 4>(lam, w, i4, zh4, a, b, c, inf_flag); break;
-            case 5: LoopRow<MODE, 5>(lam, w, i4, zh4, a, b, c, inf_flag); break;
-            case 6: LoopRow<MODE, 6>(lam, w, i4, zh4, a, b, c, inf_flag); break;
-            case 7: LoopRow<MODE, 7>(lam, w, i4, zh4, a, b, c, inf_flag); break;
-            default: LoopRow<MODE, 8>(lam, w, i4, zh4, a, b, c, inf_flag); break;
+            case 4: LoopRow<MODE, ZT, 4>(lam, w, i4, zh4, a, b, c, inf_flag); break;
+            case 5: LoopRow<MODE, ZT, 5>(lam, w, i4, zh4, a, b, c, inf_flag); break;
+            case 6: LoopRow<MODE, ZT, 6>(lam, w, i4, zh4, a, b, c, inf_flag); break;
+            case 7: LoopRow<MODE, ZT, 7>(lam, w, i4, zh4, a, b, c, inf_flag); break;
+            default: LoopRow<MODE, ZT, 8>(lam, w, i4, zh4, a, b, c, inf_flag); break;
             }
             st.s1p[j] = a;
             st.d12[j] = b;
@@ -1002,7 +1027,7 @@ __device__ __forceinline__ uint32_t HardBits2(uint32_t v)
 // Bit 0 / 16 set where check i / i + Z/2 of one of the rows [r0, r1) fails.
 // FP16 without EXACT: the sign-bit XOR (no posterior is -0, and without an
 // infinite or NaN extrinsic none is a NaN; see PairSyndrome).
-template <int MODE, bool EXACT>
+template <int MODE, uint32_t ZT, bool EXACT>
 __device__ __forceinline__ uint32_t TableSyndrome(uint32_t *lam, const uint32_t *tab, int r0, int r1, uint32_t i4,
                                                   uint32_t zh4)
 {
@@ -1014,7 +1039,7 @@ __device__ __forceinline__ uint32_t TableSyndrome(uint32_t *lam, const uint32_t 
         uint32_t p = 0;
 #pragma unroll 4
         for (int k = 0; k < deg; ++k) {
-            const EdgeAt a = TableEdge(tab[(info & 0xffffu) + k], i4, zh4);
+            const EdgeAt a = TableEdge<ZT>(TableWord<ZT>(tab, (info & 0xffffu) + k), i4, zh4);
             const uint32_t v = Rot16(LdsWord(lam, a.byte), a.rot);
             p ^= EXACT || MODE == AIRAN_LDPC_MODE_REF ? HardBits2<MODE>(v) : (v >> 15);
         }
@@ -1067,12 +1092,17 @@ __device__ __forceinline__ uint32_t HalfIndex(uint32_t t, uint32_t z, uint32_t z
 // transmitted bit lands on its own position (RateSingle), the planes are read
 // in aligned 16-byte chunks of 8 symbols and scattered (see PairLoad);
 // otherwise each position gathers its LLRs.  Ends before the barrier that
-// makes the posterior visible.
+// makes the posterior visible.  ONE: word t holds position t alone, gathered.
+template <bool ONE>
 __device__ inline void CheckLoadCodeword(uint32_t *lam, uint32_t z, uint32_t nl, const int16_t *__restrict__ cw,
                                          const airan::RateCb &rc, const airan::RateDev &r)
 {
     const uint32_t i = threadIdx.x, nt = blockDim.x, zh = z / 2;
     uint16_t *lam16 = reinterpret_cast<uint16_t *>(lam);
+    if constexpr (ONE) {
+        for (uint32_t t = i; t < nl; t += nt) lam[t] = InputH(airan::RateDematchValue(t, rc, r, cw));
+        return;
+    }
     if (!airan::RateSingle(rc, r)) {
         for (uint32_t t = i; t < nl; t += nt)
             lam16[HalfIndex(t, z, zh)] = static_cast<uint16_t>(InputH(airan::RateDematchValue(t, rc, r, cw)));
@@ -1133,7 +1163,7 @@ __device__ inline void CheckLoadCodeword(uint32_t *lam, uint32_t z, uint32_t nl,
     }
 }
 
-constexpr uint32_t kCheckThreads = 192;
+constexpr uint32_t CheckThreads(uint32_t zt) { return zt == kAnyZ ? kMaxZ : kMaxZ / 2; }
 
 // Where a block's LLRs come from: decoder LLRs [cb][68 Z] in src; or bit-plane
 // codeword LLRs (the standalone rate-dematch arithmetic, no lam_out), of code
@@ -1143,21 +1173,24 @@ constexpr int kSrcLlr = 0, kSrcRagged = 1, kSrcChain = 2;
 
 // MAXROWS: kFewRows or kRows.
 template <int MODE, int MAXROWS, uint32_t ZT, int SRC>
-__global__ void __launch_bounds__(kCheckThreads) __attribute__((amdgpu_waves_per_eu(MAXROWS <= kFewRows ? 3 : 2)))
+__global__ void __launch_bounds__(CheckThreads(ZT)) __attribute__((amdgpu_waves_per_eu(MAXROWS <= kFewRows ? 3 : 2)))
     LdpcCheckPairKernel(const int16_t *__restrict__ src, int8_t *__restrict__ bits, int16_t *__restrict__ lam_out,
                         uint8_t *__restrict__ iters_out, LdpcDev d, const airan::RaggedCb *__restrict__ cbs,
                         const airan::RaggedGrant *__restrict__ grants, const uint32_t *__restrict__ list,
                         const RateMatchDescriptor *__restrict__ desc, airan::RateDev rate)
 {
-    constexpr bool RAGGED = SRC == kSrcRagged;
+    constexpr bool RAGGED = SRC == kSrcRagged, kOne = ZT == kAnyZ;
+    static_assert(!kOne || SRC != kSrcLlr, "no operator call reaches it");
+    constexpr uint32_t kCheckThreads = CheckThreads(ZT);
     constexpr bool kFull = MAXROWS <= kFewRows;  // every message of rows 4 .. 9 kept
     constexpr int kCoreEdges = AIRAN_BG1_ROW_START[4];
     constexpr int kExtEdges = AIRAN_BG1_ROW_START[kStaticRows] - kCoreEdges;
     // The posterior, then the waves' syndrome votes (two words) and the flag
     // of an infinite or NaN extrinsic (sticky: it only selects the exact
     // syndrome).  One array, so that the posterior is at LDS address 0.
-    __shared__ __align__(16) uint32_t lam[(22 + MAXROWS) * 192 + 4];
-    uint32_t *vote = lam + (22 + MAXROWS) * 192, *inf_flag = vote + 2;
+    constexpr uint32_t kTabWords = kOne ? AIRAN_BG1_EDGES + kMaxLoopDeg : 0;
+    __shared__ __align__(16) uint32_t lam[(22 + MAXROWS) * kCheckThreads + 4 + kTabWords];
+    uint32_t *vote = lam + (22 + MAXROWS) * kCheckThreads, *inf_flag = vote + 2;
     const uint32_t i = threadIdx.x;
     uint32_t cb = blockIdx.x;
     size_t bits_off;
@@ -1167,24 +1200,32 @@ __global__ void __launch_bounds__(kCheckThreads) __attribute__((amdgpu_waves_per
         d.z = c.z;
         d.k = c.k;
         d.rows = c.rows;
-        d.zi = 0;
-        while ((24u << d.zi) < d.z) ++d.zi;
+        if constexpr (!kOne) {
+            d.zi = 0;
+            while ((24u << d.zi) < d.z) ++d.zi;
+        }
         bits_off = c.bits_off;
     } else {
         bits_off = static_cast<size_t>(cb) * d.k;
     }
-    const uint32_t Z = ZT != 0 ? ZT : d.z, zh = Z / 2, zh4 = 2u * Z;
+    const uint32_t Z = ZT == kMaxZ ? ZT : d.z, zh = kOne ? Z : Z / 2, zh4 = 4u * zh;
     const int rows = static_cast<int>(d.rows);
     const uint32_t nl = (22u + d.rows) * Z;  // positions the active rows touch
     uint16_t *lam16 = reinterpret_cast<uint16_t *>(lam);
     if (i < 3) vote[i] = 0;
+    if constexpr (kOne)
+        for (uint32_t e = i; e < kTabWords; e += kCheckThreads) {
+            const uint32_t s = e < AIRAN_BG1_EDGES ? AIRAN_BG1_SHIFT[e] % Z : 0u;
+            vote[4 + e] = (e < AIRAN_BG1_EDGES ? AIRAN_BG1_COL[e] * Z + s : 0u) | (Z - s) << 16;
+        }
     if constexpr (RAGGED) {
         const airan::RaggedCb &c = cbs[cb];
         const airan::RaggedGrant &gr = grants[c.grant];
         const airan::RateDev r{gr.g.qm, gr.g.cw_symbols, gr.g.cw_stride, Z, c.kprime, c.filler, c.ncb, 1};
-        CheckLoadCodeword(lam, Z, nl, src + gr.cw_off, airan::RateCbSetup({c.e, c.k0, c.ncb, c.cw_symbol_offset}, r), r);
+        const airan::RateCb rc = airan::RateCbSetup({c.e, c.k0, c.ncb, c.cw_symbol_offset}, r);
+        CheckLoadCodeword<kOne>(lam, Z, nl, src + gr.cw_off, rc, r);
     } else if constexpr (SRC == kSrcChain) {
-        CheckLoadCodeword(lam, Z, nl, src, airan::RateCbSetup(desc[cb], rate), rate);
+        CheckLoadCodeword<kOne>(lam, Z, nl, src, airan::RateCbSetup(desc[cb], rate), rate);
     } else {
         const int16_t *s = src + static_cast<size_t>(cb) * 68u * Z;
         if ((reinterpret_cast<uintptr_t>(src) & 7u) == 0) {
@@ -1206,7 +1247,7 @@ __global__ void __launch_bounds__(kCheckThreads) __attribute__((amdgpu_waves_per
                 lam16[HalfIndex(t, Z, zh)] = static_cast<uint16_t>(StartH<MODE>(s[t]));
         }
     }
-    const uint32_t *tab = kEdges.w[d.zi];
+    const uint32_t *tab = kOne ? vote + 4 : kEdges.w[d.zi];
     uint32_t core[kCoreEdges];
 #pragma unroll
     for (int e = 0; e < kCoreEdges; ++e) core[e] = 0;
@@ -1225,8 +1266,8 @@ __global__ void __launch_bounds__(kCheckThreads) __attribute__((amdgpu_waves_per
         uint32_t i4 = 4u * i;
         StaticRows<MODE, ZT, kFull, 0>(lam, tab, i4, zh4, mine, rows, core, ext, inf_flag);
         if constexpr (MAXROWS > kStaticRows) {
-            LoopRows<MODE, 32>(lam, tab, kStaticRows, min(rows - kStaticRows, 32), mine, i4, zh4, sa, inf_flag);
-            LoopRows<MODE, 4>(lam, tab, kStaticRows + 32, rows - kStaticRows - 32, mine, i4, zh4, sb, inf_flag);
+            LoopRows<MODE, ZT, 32>(lam, tab, kStaticRows, min(rows - kStaticRows, 32), mine, i4, zh4, sa, inf_flag);
+            LoopRows<MODE, ZT, 4>(lam, tab, kStaticRows + 32, rows - kStaticRows - 32, mine, i4, zh4, sb, inf_flag);
         }
         ++it;
         if (d.early_stop) {
@@ -1236,12 +1277,12 @@ __global__ void __launch_bounds__(kCheckThreads) __attribute__((amdgpu_waves_per
             const bool exact = MODE == AIRAN_LDPC_MODE_FP16 && *inf_flag != 0;
             uint32_t bad = 0;
             if (mine && !exact) {
-                if constexpr (ZT != 0)
+                if constexpr (ZT == kMaxZ)
                     bad = StaticSyndrome<MODE, ZT, 0, 4>(lam, i4);
                 else
-                    bad = TableSyndrome<MODE, false>(lam, tab, 0, 4, i4, zh4);
+                    bad = TableSyndrome<MODE, ZT, false>(lam, tab, 0, 4, i4, zh4);
             } else if (mine) {
-                bad = TableSyndrome<MODE, true>(lam, tab, 0, 4, i4, zh4);
+                bad = TableSyndrome<MODE, ZT, true>(lam, tab, 0, 4, i4, zh4);
             }
             if (__ballot(bad != 0) != 0 && (i & 63u) == 0) vote[0] = 1u;
             __syncthreads();
@@ -1249,7 +1290,7 @@ __global__ void __launch_bounds__(kCheckThreads) __attribute__((amdgpu_waves_per
             if (ok) {
                 bad = 0;
                 if (mine && !exact) {
-                    if constexpr (ZT != 0 && MAXROWS <= kFewRows) {
+                    if constexpr (ZT == kMaxZ && MAXROWS <= kFewRows) {
                         // Unrolled up to the few rows; a row beyond the
                         // block's is not read (its column is not loaded).
                         if (rows > 4) bad |= StaticSyndrome<MODE, ZT, 4, 5>(lam, i4);
@@ -1259,10 +1300,10 @@ __global__ void __launch_bounds__(kCheckThreads) __attribute__((amdgpu_waves_per
                         if (rows > 8) bad |= StaticSyndrome<MODE, ZT, 8, 9>(lam, i4);
                         if (rows > 9) bad |= StaticSyndrome<MODE, ZT, 9, 10>(lam, i4);
                     } else {
-                        bad = TableSyndrome<MODE, false>(lam, tab, 4, rows, i4, zh4);
+                        bad = TableSyndrome<MODE, ZT, false>(lam, tab, 4, rows, i4, zh4);
                     }
                 } else if (mine) {
-                    bad = TableSyndrome<MODE, true>(lam, tab, 4, rows, i4, zh4);
+                    bad = TableSyndrome<MODE, ZT, true>(lam, tab, 4, rows, i4, zh4);
                 }
                 if (__ballot(bad != 0) != 0 && (i & 63u) == 0) vote[1] = 1u;
                 __syncthreads();
@@ -1276,7 +1317,9 @@ __global__ void __launch_bounds__(kCheckThreads) __attribute__((amdgpu_waves_per
     // (every posterior is final: the last row and the votes ended in barriers)
     if (iters_out != nullptr && i == 0) iters_out[cb] = static_cast<uint8_t>(it);
     int8_t *bo = bits + bits_off;
-    if ((d.k & 3u) == 0 && (reinterpret_cast<uintptr_t>(bo) & 3u) == 0) {
+    if (kOne) {
+        for (uint32_t t = i; t < d.k; t += kCheckThreads) bo[t] = static_cast<int8_t>(HardBits2<MODE>(lam[t]) & 1u);
+    } else if ((d.k & 3u) == 0 && (reinterpret_cast<uintptr_t>(bo) & 3u) == 0) {
         for (uint32_t t = 4u * i; t < d.k; t += 4u * kCheckThreads) {
             const uint32_t h = HalfIndex(t, Z, zh), sh = h & 1u;
             const uint4 v = *reinterpret_cast<const uint4 *>(lam + h / 2u);
@@ -1385,7 +1428,7 @@ void LaunchCheckPair(const LdpcDecodeOpArgsV1 *a, hipStream_t s)
                           const airan::RaggedGrant *, const uint32_t *, const RateMatchDescriptor *, airan::RateDev);
     const Kern k = few ? (z384 ? LdpcCheckPairKernel<MODE, kFewRows, 384, kSrcLlr> : LdpcCheckPairKernel<MODE, kFewRows, 0, kSrcLlr>)
                        : (z384 ? LdpcCheckPairKernel<MODE, kRows, 384, kSrcLlr> : LdpcCheckPairKernel<MODE, kRows, 0, kSrcLlr>);
-    hipLaunchKernelGGL(k, dim3(a->num_cb), dim3(kCheckThreads), 0, s, static_cast<const int16_t *>(a->lam_in),
+    hipLaunchKernelGGL(k, dim3(a->num_cb), dim3(CheckThreads(kMaxZ)), 0, s, static_cast<const int16_t *>(a->lam_in),
                        static_cast<int8_t *>(a->bits), static_cast<int16_t *>(a->lam_out),
                        static_cast<uint8_t *>(a->iterations_out), d, nullptr, nullptr, nullptr, nullptr, airan::RateDev{});
 }
@@ -1475,25 +1518,29 @@ int32_t airan_ldpc_decode_Enqueue(const LdpcDecodeOpArgsV1 *a, void *workspace, 
 namespace airan {
 
 int32_t LaunchLdpcRagged(const RaggedCb *cbs, const RaggedGrant *grants, const RaggedLdpcList &many,
-                         const RaggedLdpcList &few, const RaggedLdpcList &other, uint32_t iters, bool early_stop,
-                         const int16_t *cw, int8_t *bits, uint8_t *iters_out, hipStream_t s)
+                         const RaggedLdpcList &few, const RaggedLdpcList &other, const RaggedLdpcList &any,
+                         uint32_t iters, bool early_stop, const int16_t *cw, int8_t *bits, uint8_t *iters_out,
+                         hipStream_t s)
 {
     const int32_t st = LoadEdgeTable();
     if (st != AIRAN_OK) return st;
     const LdpcDev d{0, LiftIndex(384), 0, iters, 0, early_stop ? 1u : 0u};
     constexpr int kMode = AIRAN_LDPC_MODE_FP16;
-    auto launch = [&](auto kernel, const RaggedLdpcList &l) {
+    auto launch = [&](auto kernel, const RaggedLdpcList &l, uint32_t threads = CheckThreads(kMaxZ)) {
         if (l.count > 0)
-            hipLaunchKernelGGL(kernel, dim3(l.count), dim3(kCheckThreads), 0, s, cw, bits, nullptr, iters_out, d, cbs,
+            hipLaunchKernelGGL(kernel, dim3(l.count), dim3(threads), 0, s, cw, bits, nullptr, iters_out, d, cbs,
                                grants, l.list, nullptr, RateDev{});
     };
     launch(LdpcCheckPairKernel<kMode, kRows, 384, kSrcRagged>, many);
     launch(LdpcCheckPairKernel<kMode, kFewRows, 384, kSrcRagged>, few);
     launch(LdpcCheckPairKernel<kMode, kRows, 0, kSrcRagged>, other);
+    launch(LdpcCheckPairKernel<kMode, kRows, kAnyZ, kSrcRagged>, any, CheckThreads(kAnyZ));
     return LaunchStatus();
 }
 
 uint32_t LdpcFewRows() { return kFewRows; }
+
+bool LdpcLiftSize(uint32_t z) { return IsLiftSize(z); }
 
 int32_t InitLdpcTables()
 {
@@ -1518,7 +1565,7 @@ int32_t LaunchLdpcFromCodeword(const Geom &g, const AiranTbPlanV1 &p, const Rate
         const LdpcDev d{p.Z, LiftIndex(p.Z), p.K, iters, rows, early_stop ? 1u : 0u};
         const RateDev r{g.qm, g.cw_symbols, g.cw_stride, p.Z, p.Kprime, p.filler, p.Ncb, num_cb};
         hipLaunchKernelGGL((LdpcCheckPairKernel<AIRAN_LDPC_MODE_FP16, kFewRows, 384, kSrcChain>), dim3(num_cb),
-                           dim3(kCheckThreads), 0, s, cw, bits, nullptr, iters_out, d, nullptr, nullptr, nullptr, desc, r);
+                           dim3(CheckThreads(kMaxZ)), 0, s, cw, bits, nullptr, iters_out, d, nullptr, nullptr, nullptr, desc, r);
         return LaunchStatus();
     }
     if ((st = LoadLiftTable()) != AIRAN_OK) return st;
