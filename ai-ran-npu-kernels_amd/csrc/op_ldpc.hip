@@ -1560,12 +1560,16 @@ int32_t LaunchLdpcFromCodeword(const Geom &g, const AiranTbPlanV1 &p, const Rate
         p.E_low >= (1u << 22) || p.E_high >= (1u << 22))
         return AIRAN_UNSUPPORTED_PROFILE;
     int32_t st;
-    if (!UsePair(p.Z, rows, num_cb, early_stop)) {
+    const bool any = !IsLiftSize(p.Z);
+    if (any || !UsePair(p.Z, rows, num_cb, early_stop)) {
         if ((st = LoadEdgeTable()) != AIRAN_OK) return st;
         const LdpcDev d{p.Z, LiftIndex(p.Z), p.K, iters, rows, early_stop ? 1u : 0u};
         const RateDev r{g.qm, g.cw_symbols, g.cw_stride, p.Z, p.Kprime, p.filler, p.Ncb, num_cb};
-        hipLaunchKernelGGL((LdpcCheckPairKernel<AIRAN_LDPC_MODE_FP16, kFewRows, 384, kSrcChain>), dim3(num_cb),
-                           dim3(CheckThreads(kMaxZ)), 0, s, cw, bits, nullptr, iters_out, d, nullptr, nullptr, nullptr, desc, r);
+        constexpr int kMode = AIRAN_LDPC_MODE_FP16;
+        const auto k = any ? LdpcCheckPairKernel<kMode, kRows, kAnyZ, kSrcChain>
+                           : LdpcCheckPairKernel<kMode, kFewRows, 384, kSrcChain>;
+        hipLaunchKernelGGL(k, dim3(num_cb), dim3(CheckThreads(any ? kAnyZ : kMaxZ)), 0, s, cw, bits, nullptr, iters_out,
+                           d, nullptr, nullptr, nullptr, desc, r);
         return LaunchStatus();
     }
     if ((st = LoadLiftTable()) != AIRAN_OK) return st;

@@ -95,3 +95,35 @@ def test_ragged_batch(gpu_stream, early):
         assert (tb_ok[i] == 1) == np.array_equal(got, payloads[i][0]), i
     assert tb_ok[3] == 0 and tb_ok.sum() >= 7
     batch.close()
+
+
+@pytest.mark.parametrize("early", [1, 0])
+@pytest.mark.parametrize("prb,qm,z", [(6, 2, 72), (11, 2, 120), (6, 4, 144), (10, 6, 360)])
+def test_chain(gpu_stream, prb, qm, z, early):
+    """Sizes that are a multiple of 24 and few rows: the decoder reads the
+    chain's codeword LLRs itself."""
+    from puschrx import profiles as P
+    from puschrx.chain import ChainOptions, NativeChain
+    cfg = P.Profile(name="t", rx=4, rank=1, num_rb=prb, fft=256, qm=qm, code_rate=0.5).config()
+    g = ops.Geometry(cfg)
+    plan = any_size_plan(g, z, 1)
+    rows = ops.ldpc_active_rows(plan)
+    print(f"Z {z}, {rows} rows", flush=True)
+    assert rows <= 8
+    n = 3
+    payload = np.random.default_rng(z).integers(0, 2, (n, plan.tbs), dtype=np.uint8)
+    iq = transmit(cfg, plan, payload, z, 45.0)
+    opts = ChainOptions(tau_s=100e-9, fd_hz=10.0, iq_format=abi.IQ_COMPLEX64, early_stop=early)
+    chain = NativeChain(cfg, plan, max_slots=n, opts=opts, use_graph=False)
+    chain.enqueue(iq, n)
+    cw = chain.fetch("cw_llr", torch.int16, n * qm * g.cw_stride).reshape(n, -1)
+    bits = chain.fetch("bits", torch.int8, n * plan.K).reshape(n, -1)
+    iters = chain.fetch("iterations", torch.uint8, n)
+    tb_ok = chain.fetch("tb_ok", torch.uint8, n)
+    torch.cuda.synchronize()
+    cw, bits, iters, tb_ok = (x.cpu().numpy() for x in (cw, bits, iters, tb_ok))
+    for t in range(n):
+        want, it = oracle_decode(cfg, plan, cw[t], opts.ldpc_iterations, bool(early))
+        assert np.array_equal(bits[t], want) and iters[t] == it[0], t
+        assert (tb_ok[t] == 1) == np.array_equal(bits[t][: plan.tbs], payload[t]), t
+    chain.close()
