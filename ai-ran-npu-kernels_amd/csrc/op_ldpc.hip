@@ -29,10 +29,6 @@ extern __shared__ uint16_t airan_ldpc_lam[];
 
 namespace {
 
-// Per-device "constant tables loaded" flags of kLift and kEdges, guarded by
-// one mutex (callers on several host threads may load them at once).
-std::mutex g_table_mutex;
-
 // ------------------------------------------------------------------ fast path
 // FP16 messages and at most kFastRows active rows (every code rate above
 // about 0.75), with:
@@ -66,14 +62,9 @@ struct Bg1LiftDev {
 
 __constant__ Bg1LiftDev kLift;
 
-bool g_lift_loaded[64] = {};
-
-int32_t LoadLiftTable()
+// To the current device.
+int32_t CopyLiftTable()
 {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return AIRAN_LAUNCH_FAILED;
-    std::lock_guard<std::mutex> lock(g_table_mutex);
-    if (g_lift_loaded[dev]) return AIRAN_OK;
     for (int r = 0; r < kFastRows; ++r)
         if (AIRAN_BG1_ROW_START[r] != FastRowStart(r) ||
             AIRAN_BG1_ROW_START[r + 1] - AIRAN_BG1_ROW_START[r] != kFastDeg[r])
@@ -85,9 +76,7 @@ int32_t LoadLiftTable()
             t.w[zi][e] = static_cast<uint32_t>(AIRAN_BG1_COL[e]) * z |
                          (static_cast<uint32_t>(AIRAN_BG1_SHIFT[e]) % z) << 16;
     }
-    if (hipMemcpyToSymbol(HIP_SYMBOL(kLift), &t, sizeof(t)) != hipSuccess) return AIRAN_LAUNCH_FAILED;
-    g_lift_loaded[dev] = true;
-    return AIRAN_OK;
+    return hipMemcpyToSymbol(HIP_SYMBOL(kLift), &t, sizeof(t)) == hipSuccess ? AIRAN_OK : AIRAN_LAUNCH_FAILED;
 }
 
 using h16 = _Float16;
@@ -734,15 +723,10 @@ struct Bg1EdgeDev {
 
 __constant__ Bg1EdgeDev kEdges;
 
-bool g_edges_loaded[64] = {};
-
-int32_t LoadEdgeTable()
+// To the current device, under g_table_mutex.
+int32_t CopyEdgeTable()
 {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return AIRAN_LAUNCH_FAILED;
-    std::lock_guard<std::mutex> lock(g_table_mutex);
-    if (g_edges_loaded[dev]) return AIRAN_OK;
-    static Bg1EdgeDev t;  // under the lock
+    static Bg1EdgeDev t;
     t = Bg1EdgeDev{};
     for (int r = 0; r < kRows; ++r) {
         const uint32_t e0 = AIRAN_BG1_ROW_START[r], deg = AIRAN_BG1_ROW_START[r + 1] - e0;
@@ -756,9 +740,27 @@ int32_t LoadEdgeTable()
             t.w[zi][e] = 4u * (AIRAN_BG1_COL[e] * zh + sh) | 4u * (zh - sh) << 16 | (s >= zh ? 1u << 31 : 0u);
         }
     }
-    if (hipMemcpyToSymbol(HIP_SYMBOL(kEdges), &t, sizeof(t)) != hipSuccess) return AIRAN_LAUNCH_FAILED;
-    g_edges_loaded[dev] = true;
-    return AIRAN_OK;
+    return hipMemcpyToSymbol(HIP_SYMBOL(kEdges), &t, sizeof(t)) == hipSuccess ? AIRAN_OK : AIRAN_LAUNCH_FAILED;
+}
+
+// Per-device "constant tables loaded" flags, guarded by a mutex (callers on
+// several host threads may load them at once).
+std::mutex g_table_mutex;
+bool g_tables_loaded[64] = {};
+
+// Both tables on the current device, whichever kernel the call takes: that
+// depends on the number of blocks and their alignment, and a caller who has
+// decoded once may capture the next call, where nothing can be copied.
+int32_t LoadTables()
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return AIRAN_LAUNCH_FAILED;
+    std::lock_guard<std::mutex> lock(g_table_mutex);
+    if (g_tables_loaded[dev]) return AIRAN_OK;
+    int32_t st = CopyLiftTable();
+    if (st == AIRAN_OK) st = CopyEdgeTable();
+    g_tables_loaded[dev] = st == AIRAN_OK;
+    return st;
 }
 
 // Lifting sizes other than 24 << zi (plans made by hand may have any of 24 ..
@@ -1436,14 +1438,14 @@ void LaunchCheckPair(const LdpcDecodeOpArgsV1 *a, hipStream_t s)
 // The decoder operator (validated arguments).
 int32_t LaunchDecode(const LdpcDecodeOpArgsV1 *a)
 {
-    int32_t st;
+    const int32_t st = LoadTables();
+    if (st != AIRAN_OK) return st;
     hipStream_t s = static_cast<hipStream_t>(a->stream);
     const auto *in = static_cast<const int16_t *>(a->lam_in);
     auto *bits = static_cast<int8_t *>(a->bits);
     const bool aligned = (reinterpret_cast<uintptr_t>(in) & 7u) == 0 && (reinterpret_cast<uintptr_t>(bits) & 3u) == 0;
     if (aligned && FastEligible(a->mode, a->z, a->active_rows) &&
         UsePair(a->z, a->active_rows, a->num_cb, a->early_stop != 0)) {
-        if ((st = LoadLiftTable()) != AIRAN_OK) return st;
         const uint32_t rows = a->active_rows;  // validated >= 4
         LdpcFastDev fd{a->z, LiftIndex(a->z), a->k, a->max_iterations, rows, a->early_stop ? 1u : 0u, a->num_cb, {}};
         const size_t fast_lds = static_cast<size_t>(22 + rows) * a->z * sizeof(uint32_t);
@@ -1451,7 +1453,6 @@ int32_t LaunchDecode(const LdpcDecodeOpArgsV1 *a)
                           static_cast<int16_t *>(a->lam_out), static_cast<uint8_t *>(a->iterations_out), fd, nullptr);
         return airan::LaunchStatus();
     }
-    if ((st = LoadEdgeTable()) != AIRAN_OK) return st;
     if (a->mode == AIRAN_LDPC_MODE_FP16)
         LaunchCheckPair<AIRAN_LDPC_MODE_FP16>(a, s);
     else
@@ -1522,7 +1523,7 @@ int32_t LaunchLdpcRagged(const RaggedCb *cbs, const RaggedGrant *grants, const R
                          uint32_t iters, bool early_stop, const int16_t *cw, int8_t *bits, uint8_t *iters_out,
                          hipStream_t s)
 {
-    const int32_t st = LoadEdgeTable();
+    const int32_t st = LoadTables();
     if (st != AIRAN_OK) return st;
     const LdpcDev d{0, LiftIndex(384), 0, iters, 0, early_stop ? 1u : 0u};
     constexpr int kMode = AIRAN_LDPC_MODE_FP16;
@@ -1546,8 +1547,7 @@ int32_t InitLdpcTables()
 {
     // So that a caller who ran airan_InitDevice launches nothing but the
     // decoder afterwards.
-    const int32_t st = LoadLiftTable();
-    return st == AIRAN_OK ? LoadEdgeTable() : st;
+    return LoadTables();
 }
 
 int32_t LaunchLdpcFromCodeword(const Geom &g, const AiranTbPlanV1 &p, const RateMatchDescriptor *desc,
@@ -1559,10 +1559,10 @@ int32_t LaunchLdpcFromCodeword(const Geom &g, const AiranTbPlanV1 &p, const Rate
         (p.Z % 24) != 0 || p.K == 0 || p.K > 22 * p.Z || p.Ncb <= p.filler || (reinterpret_cast<uintptr_t>(bits) & 3u) ||
         p.E_low >= (1u << 22) || p.E_high >= (1u << 22))
         return AIRAN_UNSUPPORTED_PROFILE;
-    int32_t st;
+    const int32_t st = LoadTables();
+    if (st != AIRAN_OK) return st;
     const bool any = !IsLiftSize(p.Z);
     if (any || !UsePair(p.Z, rows, num_cb, early_stop)) {
-        if ((st = LoadEdgeTable()) != AIRAN_OK) return st;
         const LdpcDev d{p.Z, LiftIndex(p.Z), p.K, iters, rows, early_stop ? 1u : 0u};
         const RateDev r{g.qm, g.cw_symbols, g.cw_stride, p.Z, p.Kprime, p.filler, p.Ncb, num_cb};
         constexpr int kMode = AIRAN_LDPC_MODE_FP16;
@@ -1572,7 +1572,6 @@ int32_t LaunchLdpcFromCodeword(const Geom &g, const AiranTbPlanV1 &p, const Rate
                            d, nullptr, nullptr, nullptr, desc, r);
         return LaunchStatus();
     }
-    if ((st = LoadLiftTable()) != AIRAN_OK) return st;
     LdpcFastDev fd{p.Z, LiftIndex(p.Z), p.K, iters, rows, early_stop ? 1u : 0u, num_cb,
                    {g.qm, g.cw_symbols, g.cw_stride, p.Z, p.Kprime, p.filler, p.Ncb, num_cb}};
     const size_t lds = static_cast<size_t>(22 + rows) * p.Z * sizeof(uint32_t);
