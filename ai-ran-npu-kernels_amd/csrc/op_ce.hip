@@ -934,19 +934,21 @@ constexpr uint32_t kPostRx = 8;
 
 // Rescale (per model), pair combination h = (g_a + sign g_b) / 2 with
 // relative error (err_a + err_b) / 2, and time interpolation over the D DMRS
-// symbols.  One thread per subcarrier of one (slot, layer, kPostRx receive
-// antennas) = blockIdx.y.  Writes H[slot][rx][l][sym][sc] fp16 for sc < pad
-// (zero beyond used).  Bound by the writes: 64 slots, 4 Rx, 273 PRB 312 MB in 60
-// us; 23 slots, 64 Rx, 133 PRB 185 us, where one thread for all antennas
-// left 2.5 workgroups per CU and took 307.
+// symbols.  One thread per subcarrier of one (slot, layer) = blockIdx.y and
+// kPostRx receive antennas; x holds the subcarriers of each chunk of antennas
+// in turn, so that y stays within the device's 65536 for every chain (4096
+// slots).  Writes H[slot][rx][l][sym][sc] fp16 for sc < pad (zero beyond used).
+// Bound by the writes: 64 slots, 4 Rx, 273 PRB 312 MB in 60 us; 23 slots, 64
+// Rx, 133 PRB 185 us, where one thread for all antennas left 2.5 workgroups per
+// CU and took 307.
 template <int D>
 __device__ __forceinline__ void CePostKernelBody(const CeWs &w, __half *__restrict__ out_r, __half *__restrict__ out_i,
                                                     uint32_t out_layers, const CeApply &c, uint32_t bx, uint32_t by)
 {
-    const uint32_t sc = bx * blockDim.x + threadIdx.x;
-    const uint32_t chunks = (c.nr + kPostRx - 1u) / kPostRx, sl = by / chunks;
-    const uint32_t rx0 = (by - sl * chunks) * kPostRx, rx1 = min(c.nr, rx0 + kPostRx);
-    const uint32_t slot = sl / c.nl, l = sl - slot * c.nl;
+    const uint32_t sc_blocks = (c.pad + blockDim.x - 1u) / blockDim.x, chunk = bx / sc_blocks;
+    const uint32_t sc = (bx - chunk * sc_blocks) * blockDim.x + threadIdx.x;
+    const uint32_t rx0 = chunk * kPostRx, rx1 = min(c.nr, rx0 + kPostRx);
+    const uint32_t slot = by / c.nl, l = by - slot * c.nl;
     if (sc >= c.pad) return;
     const size_t plane = static_cast<size_t>(c.nsym) * c.pad;
     out_r += static_cast<size_t>(slot) * c.nr * out_layers * plane;
@@ -1360,9 +1362,9 @@ void StepGrids(const LmmseFilter &f, uint32_t slots, CeJobDev *j)
     j->interp_per_xcd = airan::CeilDiv(large, 8);
     j->small_per_xcd = airan::CeilDiv(small, 8);
     const uint32_t gx[kCeSteps] = {z, 8 * std::max(j->proj_per_xcd, j->proj_small_per_xcd), slots * f.nm * ncol, hv,
-                                   8 * j->interp_per_xcd, 8 * j->small_per_xcd, airan::CeilDiv(g.pad, 256),
-                                   slots * kScaleParts};
-    const uint32_t gy[kCeSteps] = {f.nb, f.nb, 1, f.nb, f.nb, f.nb, slots * g.nl * airan::CeilDiv(g.nr, kPostRx), 1};
+                                   8 * j->interp_per_xcd, 8 * j->small_per_xcd,
+                                   airan::CeilDiv(g.pad, 256) * airan::CeilDiv(g.nr, kPostRx), slots * kScaleParts};
+    const uint32_t gy[kCeSteps] = {f.nb, f.nb, 1, f.nb, f.nb, f.nb, slots * g.nl, 1};
     for (int k = 0; k < kCeSteps; ++k) {
         j->gx[k] = gx[k];
         j->gy[k] = gy[k];
