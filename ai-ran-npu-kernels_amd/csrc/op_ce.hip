@@ -417,6 +417,8 @@ __device__ __forceinline__ void CeProjectMfmaKernelBody(const CeWs &w, uint32_t 
                                                               uint32_t per_xcd, uint32_t bx, uint32_t by)
 {
     constexpr uint32_t KB = RB;  // 32-eigenvector blocks per wave
+    // A grouped launch has the grid of the form that needs more workgroups.
+    if ((bx >> 3) >= per_xcd) return;
     const uint32_t tile = (bx & 7u) * per_xcd + (bx >> 3);
     const CeBaseDev &bd = c.b[by];
     const uint32_t ncol = c.nr * c.ndmrs, N = BaseRows(bd.nq, slots, ncol);

@@ -40,3 +40,32 @@ def test_batch_equals_slots(gpu_stream, rx, rank, prb, slots):
             assert torch.equal(a[s * k:(s + 1) * k].view(torch.int16), b.view(torch.int16)), s
     batch.close()
     one.close()
+
+
+def test_grouped_forms(gpu_stream):
+    """A ragged batch of 20 grants of one rank-3 shape: its pair's base (320
+    rows) takes the 128-row form and the single layer's (160) the 32-row form
+    within one grouped launch."""
+    from puschrx import grants as G
+    from puschrx.chain import ChainOptions, NativeChain
+    grants = [G.Grant(name=f"g{i}", rank=3, qm=4, num_rb=11, fft_size=256, code_rate=0.4, rnti=i + 1,
+                      padded_subcarriers=256) for i in range(20)]
+    compiled = G.compile_grants(G.Radio(), grants)
+    batch = G.GrantBatch(compiled, dict(iq_format=abi.IQ_COMPLEX64, tau_s=200e-9, fd_hz=30.0), use_graph=False)
+    assert batch.num_shapes == 1
+    rng = np.random.default_rng(3)
+    g = ops.Geometry(compiled[0][1])
+    iqs = [rng.normal(0, 1, (g.nr, g.samples, 2)).astype(np.float32) for _ in compiled]
+    batch.enqueue(batch.pack_iq(iqs))
+    opts = ChainOptions(tau_s=200e-9, fd_hz=30.0, iq_format=abi.IQ_COMPLEX64)
+    for i in (0, 7, 19):
+        _, cfg, plan = compiled[i]
+        n = cfg.qm * g.cw_stride
+        got = batch.fetch("cw_llr", torch.int16, n, batch.layout[i].cw_offset)
+        one = NativeChain(cfg, plan, max_slots=1, opts=opts, use_graph=False)
+        one.enqueue(torch.from_numpy(iqs[i][None]).cuda(), 1)
+        want = one.fetch("cw_llr", torch.int16, n)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), i
+        one.close()
+    batch.close()
