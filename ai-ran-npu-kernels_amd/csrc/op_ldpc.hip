@@ -770,6 +770,9 @@ int32_t LoadTables()
 // Z - shift mod Z above) are made by each workgroup, in LDS.
 constexpr uint32_t kAnyZ = 1;  // as ZT
 constexpr uint32_t kMaxZ = 384;
+// As ZT: a size below 384 read from the arguments; one of at most 96, with the
+// lanes and the LDS of 96.
+constexpr uint32_t kLowZ = 0, kZ96 = 2;
 
 constexpr bool IsLiftSize(uint32_t z)
 {
@@ -1165,7 +1168,9 @@ __device__ inline void CheckLoadCodeword(uint32_t *lam, uint32_t z, uint32_t nl,
     }
 }
 
-constexpr uint32_t CheckThreads(uint32_t zt) { return zt == kAnyZ ? kMaxZ : kMaxZ / 2; }
+constexpr uint32_t CheckThreads(uint32_t zt) { return zt == kAnyZ ? kMaxZ : zt == kZ96 ? 64 : kMaxZ / 2; }
+// Words of a column's posterior.
+constexpr uint32_t ColWords(uint32_t zt) { return zt == kZ96 ? 48 : CheckThreads(zt); }
 
 // Where a block's LLRs come from: decoder LLRs [cb][68 Z] in src; or bit-plane
 // codeword LLRs (the standalone rate-dematch arithmetic, no lam_out), of code
@@ -1191,8 +1196,8 @@ __global__ void __launch_bounds__(CheckThreads(ZT)) __attribute__((amdgpu_waves_
     // of an infinite or NaN extrinsic (sticky: it only selects the exact
     // syndrome).  One array, so that the posterior is at LDS address 0.
     constexpr uint32_t kTabWords = kOne ? AIRAN_BG1_EDGES + kMaxLoopDeg : 0;
-    __shared__ __align__(16) uint32_t lam[(22 + MAXROWS) * kCheckThreads + 4 + kTabWords];
-    uint32_t *vote = lam + (22 + MAXROWS) * kCheckThreads, *inf_flag = vote + 2;
+    __shared__ __align__(16) uint32_t lam[(22 + MAXROWS) * ColWords(ZT) + 4 + kTabWords];
+    uint32_t *vote = lam + (22 + MAXROWS) * ColWords(ZT), *inf_flag = vote + 2;
     const uint32_t i = threadIdx.x;
     uint32_t cb = blockIdx.x;
     size_t bits_off;
@@ -1391,8 +1396,9 @@ bool FastEligible(uint32_t mode, uint32_t z, uint32_t rows)
 
 // FP16 messages, at most kFastRows rows: two blocks a workgroup (the pair
 // decoder) or one block with two checks a lane (LdpcCheckPairKernel).
-// Z < 384: the pair; the check pair has 192 lanes for Z / 2 pairs of checks (2048 blocks of Z = 96, 6 rows: pair
-// 82 us, check pair 193).  Z = 384: the check pair, whose blocks take and
+// Z < 384: the pair, whose lanes are all at work where a check pair's Z / 2 are
+// few (8 iterations, pair / check pair: 2048 blocks of Z = 96, 6 rows 81 / 88 us,
+// 4000 of Z = 24, 8 rows 81 / 178).  Z = 384: the check pair, whose blocks take and
 // leave a compute unit one by one: us without early stop, pair / check pair,
 //   rows   128 blocks  600      4000      (8 iterations, launch included)
 //    4      61 / 52     90 / 81   -
@@ -1421,16 +1427,38 @@ uint32_t LiftIndex(uint32_t z)
     return zi;
 }
 
+// Check pair decoder, Z <= 96: one wave and the LDS of Z = 96 per block, where
+// the blocks outnumber what is resident with 192 lanes each (registers allow 2
+// workgroups of 3 waves a compute unit, 4 up to kFewRows rows; below that the
+// idle lanes only help to load).  4000 blocks, 8 iterations at most, Z = 24 /
+// 48 / 96: 46 rows, FP16 484 / 483 / 500 us against 1599 / 1436 / 1491 with 192
+// lanes and the LDS of 384, REF 746 / 647 / 668 against 2069 / 1849 / 1909; 9
+// rows, FP16 207 / 187 / 199 against 359 / 333 / 357.  1200 blocks of Z = 48: 46
+// rows 261 / 537, 9 rows 120 / 154.
+bool SmallBlocks(uint32_t z, uint32_t num_cb, bool few)
+{
+    int dev = 0, cus = 0;
+    if (z > 96 || hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return false;
+    return num_cb > static_cast<uint32_t>(std::max(cus, 0)) * (few ? 4u : 2u);
+}
+
 template <int MODE>
 void LaunchCheckPair(const LdpcDecodeOpArgsV1 *a, hipStream_t s)
 {
     const LdpcDev d{a->z, LiftIndex(a->z), a->k, a->max_iterations, a->active_rows, a->early_stop ? 1u : 0u};
-    const bool few = a->active_rows <= static_cast<uint32_t>(kFewRows), z384 = a->z == 384;
     using Kern = void (*)(const int16_t *, int8_t *, int16_t *, uint8_t *, LdpcDev, const airan::RaggedCb *,
                           const airan::RaggedGrant *, const uint32_t *, const RateMatchDescriptor *, airan::RateDev);
-    const Kern k = few ? (z384 ? LdpcCheckPairKernel<MODE, kFewRows, 384, kSrcLlr> : LdpcCheckPairKernel<MODE, kFewRows, 0, kSrcLlr>)
-                       : (z384 ? LdpcCheckPairKernel<MODE, kRows, 384, kSrcLlr> : LdpcCheckPairKernel<MODE, kRows, 0, kSrcLlr>);
-    hipLaunchKernelGGL(k, dim3(a->num_cb), dim3(CheckThreads(kMaxZ)), 0, s, static_cast<const int16_t *>(a->lam_in),
+    const bool few = a->active_rows <= static_cast<uint32_t>(kFewRows);
+    const uint32_t zt = a->z == kMaxZ ? kMaxZ : SmallBlocks(a->z, a->num_cb, few) ? kZ96 : kLowZ;
+    const Kern k = few ? (zt == kMaxZ   ? LdpcCheckPairKernel<MODE, kFewRows, kMaxZ, kSrcLlr>
+                          : zt == kZ96  ? LdpcCheckPairKernel<MODE, kFewRows, kZ96, kSrcLlr>
+                                        : LdpcCheckPairKernel<MODE, kFewRows, kLowZ, kSrcLlr>)
+                       : (zt == kMaxZ   ? LdpcCheckPairKernel<MODE, kRows, kMaxZ, kSrcLlr>
+                          : zt == kZ96  ? LdpcCheckPairKernel<MODE, kRows, kZ96, kSrcLlr>
+                                        : LdpcCheckPairKernel<MODE, kRows, kLowZ, kSrcLlr>);
+    hipLaunchKernelGGL(k, dim3(a->num_cb), dim3(CheckThreads(zt)), 0, s, static_cast<const int16_t *>(a->lam_in),
                        static_cast<int8_t *>(a->bits), static_cast<int16_t *>(a->lam_out),
                        static_cast<uint8_t *>(a->iterations_out), d, nullptr, nullptr, nullptr, nullptr, airan::RateDev{});
 }
@@ -1534,7 +1562,7 @@ int32_t LaunchLdpcRagged(const RaggedCb *cbs, const RaggedGrant *grants, const R
     };
     launch(LdpcCheckPairKernel<kMode, kRows, 384, kSrcRagged>, many);
     launch(LdpcCheckPairKernel<kMode, kFewRows, 384, kSrcRagged>, few);
-    launch(LdpcCheckPairKernel<kMode, kRows, 0, kSrcRagged>, other);
+    launch(LdpcCheckPairKernel<kMode, kRows, kLowZ, kSrcRagged>, other);
     launch(LdpcCheckPairKernel<kMode, kRows, kAnyZ, kSrcRagged>, any, CheckThreads(kAnyZ));
     return LaunchStatus();
 }

@@ -90,6 +90,28 @@ def test_few_rows_at_every_dispatch(gpu_stream, rows, n, early):
     assert np.array_equal(lam_out.cpu().numpy().reshape(n, -1), tile(ref))
 
 
+@pytest.mark.parametrize("mode", [abi.LDPC_MODE_REF, abi.LDPC_MODE_FP16])
+@pytest.mark.parametrize("z,rows,n", [(24, 46, 520), (48, 11, 520), (96, 43, 520), (24, 10, 1040), (96, 9, 1040)])
+def test_many_small_blocks(gpu_stream, mode, z, rows, n):
+    """Z <= 96 and more blocks than are resident at once with 192 lanes each:
+    one wave per block, whose lanes are fewer than the columns' runs."""
+    k = 22 * z - 2
+    lam = _llrs(z, 3, rows, 3.0, z + rows)
+    oracle = load_oracle()
+    ref = lam.copy()
+    bits, it = np.zeros(3 * k, np.int8), np.zeros(3, np.uint8)
+    oracle.or_ldpc_decode(z, 3, ptr(ref), mode, 6, rows, k, 1, ptr(bits), ptr(it))
+    tile = lambda a: np.tile(a.reshape(3, -1), (-(-n // 3), 1))[:n]  # noqa: E731
+    for offset in (0, 1):
+        dev = torch.zeros(n * 68 * z + offset, dtype=torch.int16, device="cuda")
+        dev[offset:] = torch.from_numpy(tile(lam).reshape(-1).copy()).cuda()
+        got, lam_out, git = ops.ldpc_decode(dev[offset:], n, z, k, 6, rows, mode, True, want_lam=True)
+        torch.cuda.synchronize()
+        assert np.array_equal(git.cpu().numpy(), tile(it).reshape(-1))
+        assert np.array_equal(got.cpu().numpy().reshape(n, -1), tile(bits))
+        assert np.array_equal(lam_out.cpu().numpy().reshape(n, -1), tile(ref))
+
+
 @pytest.mark.parametrize("rank,qm,rate", [(4, 8, 0.85), (3, 6, 0.91), (2, 4, 0.93), (1, 8, 0.8)])
 def test_chain_blocks_match_operators(gpu_stream, rank, qm, rate):
     """The decoder reading a chain's codeword LLRs itself against rate dematch
