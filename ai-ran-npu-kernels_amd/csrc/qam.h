@@ -38,7 +38,7 @@ __device__ inline void QamUT(uint32_t qm, __half y, __half n, int *u, int *t)
     *u = uu > 1000 ? 1000 : (uu < -1000 ? -1000 : uu);
 }
 
-__device__ inline int Clip2560(int v) { return v > 2560 ? 2560 : (v < -2560 ? -2560 : v); }
+__host__ __device__ inline int Clip2560(int v) { return v > 2560 ? 2560 : (v < -2560 ? -2560 : v); }
 
 // 256QAM closed form (gen_data.py:28-40), returned already negated (positive
 // => bit 0).
@@ -68,7 +68,7 @@ __device__ inline void Axis256(int u, int t, int *out)
 
 // PAM level under the reference mapper polarity (bit i of code = c_i, c_0 the
 // sign bit): level = d0 e1, e_m = 1, e_i = 2^(m-i) - d_i e_{i+1}, d = 2c - 1.
-__device__ inline int PamLevel(int m, int code)
+__host__ __device__ inline int PamLevel(int m, int code)
 {
     int e = 1;
     for (int i = m - 1; i >= 1; --i) e = (1 << (m - i)) - (2 * ((code >> i) & 1) - 1) * e;
@@ -78,7 +78,7 @@ __device__ inline int PamLevel(int m, int code)
 // Max-log by exhaustion over the 2^m levels: LLR_i = min_{c_i=1} cost -
 // min_{c_i=0} cost with cost = t s^2 - 2 u s; equal to the 256QAM closed form
 // for every integer (u, t).
-__device__ inline void AxisExhaustive(int m, int u, int t, int *out)
+__host__ __device__ inline void AxisExhaustive(int m, int u, int t, int *out)
 {
     int b0[4], b1[4];
     for (int i = 0; i < m; ++i) b0[i] = b1[i] = 0x7fffffff;
@@ -125,7 +125,7 @@ typedef _Float16 h16x2_t __attribute__((ext_vector_type(2)));
 // constant in t (2 i t >= |u|, and the t terms exceed the clip), so t is
 // limited there and all sums fit 16 bits.
 template <int QM>
-__device__ inline void AxisPair(s16x2_t u, s16x2_t t, s16x2_t (&w)[QM / 2])
+__host__ __device__ inline void AxisPair(s16x2_t u, s16x2_t t, s16x2_t (&w)[QM / 2])
 {
     constexpr int M = QM / 2;
     const s16x2_t a = __builtin_elementwise_max(u, -u), t2 = t + t;
@@ -155,7 +155,9 @@ __device__ inline void AxisPair(s16x2_t u, s16x2_t t, s16x2_t (&w)[QM / 2])
 
 // QamUT and AxisPair of one symbol (x = (I, Q) in fp16).  The fp16 quotients
 // D / n by the hardware reciprocal: rounded to fp16 they equal the division's
-// for every fp16 n and each of the eight constants (checked by exhaustion).
+// for every fp16 n and each of the eight constants: none lies as close to a
+// boundary of fp16 rounding as 1 ulp of the reciprocal and the product's
+// rounding reach, but for thresholds below 1/4, where t is 0 either way.
 // The limits of u apply before its rounding (integers, so the same), the
 // order of max and min giving a NaN u = -1000 as QamUT does.
 template <int QM>
