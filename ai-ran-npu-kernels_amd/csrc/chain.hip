@@ -61,8 +61,9 @@ __global__ void __launch_bounds__(256) GoldBitsKernel(uint32_t *__restrict__ bit
 // Newton step, the demapper packed by axis in 16 bits); with 1700 (separate
 // multiplies and adds, IEEE divisions, 32-bit demapper per axis) it was bound
 // by their issue at 111 us.  9 slots of 106 PRB, rank 2, 64QAM: 5.6 us against
-// 37 of an exhaustive search over the levels.  ZF (one Rx, one layer): single-tap zero forcing with n0 = the slot's noise (the
-// equalize_zf_siso arithmetic) in place of the LMMSE solve.
+// 37 of an exhaustive search over the levels.  ZF (one Rx, one layer):
+// single-tap zero forcing with n0 = the slot's noise (the equalize_zf_siso
+// arithmetic) in place of the LMMSE solve.
 typedef _Float16 h16x4_t __attribute__((ext_vector_type(4)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));

@@ -97,7 +97,8 @@ __global__ void __launch_bounds__(256) RaggedDetectKernel(const __half *__restri
     if (sc >= gr.g.used) return;
     // Uniform over the workgroup.
     auto run = [&](auto nl, auto qm) {
-        RaggedDetectRe<decltype(nl)::value, decltype(qm)::value>(gr, t.ds, sc, rx_re, rx_im, h_re, h_im, noise, gold, cw);
+        RaggedDetectRe<decltype(nl)::value, decltype(qm)::value>(gr, t.ds, sc, rx_re, rx_im, h_re, h_im, noise, gold,
+                                                                 cw);
     };
     auto layers = [&](auto qm) {
         switch (gr.g.nl) {
@@ -561,7 +562,8 @@ void airan_pusch_grants_Destroy(AiranGrantBatch *b)
     airan::DestroyCeGrouped(b->ce_grouped);
     if (b->ce_ws_all) (void)hipFree(b->ce_ws_all);
     void *bufs[] = {b->grants, b->gen_items, b->ls_items, b->noise_items, b->tiles, b->cbs, b->many_list, b->few_list,
-                    b->other_list, b->any_list, b->tb_first, b->tb_count, b->rx_re, b->rx_im, b->ref_re, b->ref_im, b->hls_re, b->hls_im,
+                    b->other_list, b->any_list, b->tb_first, b->tb_count, b->rx_re, b->rx_im, b->ref_re, b->ref_im,
+                    b->hls_re, b->hls_im,
                     b->noise_ls, b->noise_ce, b->h_re, b->h_im, b->gold, b->cw,
                     b->bits, b->iters, b->cb_ok, b->tb_ok, b->tb_part};
     for (void *p : bufs)

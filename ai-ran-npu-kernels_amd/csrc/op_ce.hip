@@ -413,8 +413,8 @@ __global__ void __launch_bounds__(256) CeZSplitKernel(const __half *__restrict__
 // base; each XCD takes a contiguous range of tiles ordered split major, so
 // the operands of one split are read through one L2.
 template <uint32_t RB>
-__device__ __forceinline__ void CeProjectMfmaKernelBody(const CeWs &w, uint32_t slots, const CeApply &c, uint32_t k_tiles,
-                                                              uint32_t per_xcd, uint32_t bx, uint32_t by)
+__device__ __forceinline__ void CeProjectMfmaKernelBody(const CeWs &w, uint32_t slots, const CeApply &c,
+                                                              uint32_t k_tiles, uint32_t per_xcd, uint32_t bx, uint32_t by)
 {
     constexpr uint32_t KB = RB;  // 32-eigenvector blocks per wave
     // A grouped launch has the grid of the form that needs more workgroups.
@@ -655,7 +655,8 @@ __device__ __forceinline__ void CeScaleKernelBody(const __half *__restrict__ noi
                              bd.rank / 16u, v);
     }
 }
-__global__ void __launch_bounds__(256) CeScaleKernel(const __half *__restrict__ noise_in, __half *__restrict__ noise_out,
+__global__ void __launch_bounds__(256) CeScaleKernel(const __half *__restrict__ noise_in,
+                                                     __half *__restrict__ noise_out,
                                                      CeWs w, CeApply c, uint32_t slots)
 {
     CeScaleKernelBody(noise_in, noise_out, w, c, slots, blockIdx.x);
@@ -671,7 +672,8 @@ __global__ void __launch_bounds__(256) CeScaleKernel(const __half *__restrict__ 
 // its rows r = sc + shift the columns; rows and columns past the last read
 // clamped (valid) addresses and are not stored.  Grid: row tiles fastest (they
 // share the |A|^2 tile), then column tiles; y: bases.
-__device__ __forceinline__ void CeHvMfmaKernelBody(const CeWs &w, uint32_t slots, const CeApply &c, uint32_t bx, uint32_t by)
+__device__ __forceinline__ void CeHvMfmaKernelBody(const CeWs &w, uint32_t slots, const CeApply &c, uint32_t bx,
+                                                   uint32_t by)
 {
     __shared__ float part[3][16][64];
     const CeBaseDev &bd = c.b[by];
@@ -821,8 +823,8 @@ __global__ void __launch_bounds__(256, 2) CeInterpMfmaKernel(CeWs w, uint32_t sl
 // One 273-PRB slot (32 rows) 15 us against 38 of 128-row tiles, 96
 // ragged grants 162 against 548 (a 128-row tile per 8 columns and model,
 // and four copies of the filter).
-__device__ __forceinline__ void CeInterpSmallKernelBody(const CeWs &w, uint32_t slots, const CeApply &c, uint32_t per_xcd,
-                                                           uint32_t bx, uint32_t by)
+__device__ __forceinline__ void CeInterpSmallKernelBody(const CeWs &w, uint32_t slots, const CeApply &c,
+                                                           uint32_t per_xcd, uint32_t bx, uint32_t by)
 {
     const CeBaseDev &bd = c.b[by];
     const uint32_t ncol = c.nr * c.ndmrs, N = BaseRows(bd.nq, slots, ncol);
@@ -1402,8 +1404,8 @@ int32_t LaunchCeApply(const LmmseFilter *f, const __half *hr, const __half *hi, 
     auto grid = [&](int step) { return dim3(j.gx[step], j.gy[step]); };
     hipLaunchKernelGGL(CeZSplitKernel, grid(0), dim3(256), 0, s, hr, hi, w, slots, c);
     if (j.proj_per_xcd)
-        hipLaunchKernelGGL(CeProjectMfmaKernel, dim3(8 * j.proj_per_xcd, f->nb), dim3(256), 0, s, w, slots, c, j.k_tiles,
-                           j.proj_per_xcd);
+        hipLaunchKernelGGL(CeProjectMfmaKernel, dim3(8 * j.proj_per_xcd, f->nb), dim3(256), 0, s, w, slots, c,
+                           j.k_tiles, j.proj_per_xcd);
     if (j.proj_small_per_xcd)
         hipLaunchKernelGGL(CeProjectSmallKernel, dim3(8 * j.proj_small_per_xcd, f->nb), dim3(256), 0, s, w, slots, c,
                            j.k_tiles, j.proj_small_per_xcd);
@@ -1412,7 +1414,8 @@ int32_t LaunchCeApply(const LmmseFilter *f, const __half *hr, const __half *hi, 
     hipLaunchKernelGGL(CeHvMfmaKernel, grid(3), dim3(256), 0, s, w, slots, c);
     if (j.interp_per_xcd)
         hipLaunchKernelGGL(CeInterpMfmaKernel, grid(4), dim3(256), 0, s, w, slots, c, j.interp_per_xcd);
-    if (j.small_per_xcd) hipLaunchKernelGGL(CeInterpSmallKernel, grid(5), dim3(256), 0, s, w, slots, c, j.small_per_xcd);
+    if (j.small_per_xcd)
+        hipLaunchKernelGGL(CeInterpSmallKernel, grid(5), dim3(256), 0, s, w, slots, c, j.small_per_xcd);
     const dim3 pgrid = grid(6);
     switch (g.ndmrs) {
     case 1: hipLaunchKernelGGL(CePostKernel<1>, pgrid, dim3(256), 0, s, w, out_re, out_im, out_layers, c); break;

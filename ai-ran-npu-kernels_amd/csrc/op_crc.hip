@@ -2,15 +2,13 @@
 // (TS 38.212 5.1) on decoded bits, plus payload packing.
 //
 // The CRC remainder is linear in the message bits: for an n-bit message
-// (data followed by its parity) the remainder is XOR over set bits j of
-// x^(L + n - 1 - j) mod g, a GF(2) matrix times the bit vector.  Thread t
-// of the checking kernel owns the 24 positions [24 t, 24 t + 24) of every
-// code block and holds that slice of the matrix as masks m[k] (bit 23 - jj of
-// m[k] = bit k of position 24 t + jj's term): its share of remainder bit k is
-// the parity of (its 24 bits & m[k]); the shares are XOR-reduced over the
-// workgroup.  The TB remainder of code block r is its local remainder times
-// x^(bits after r) mod g, accumulated with atomicXor (order independent) per
-// TB.
+// (data followed by its parity) it is the XOR over set bits j of
+// x^(L + n - 1 - j) mod g, a GF(2) matrix times the bit vector.  Two kernels:
+// CbCrcKernel, a workgroup per code block, whose threads multiply the 32 bits of
+// a chunk, as a polynomial, by the tabulated power of the chunk's end; and from
+// kCrcMfmaMin blocks on CrcMfmaKernel, the product on the matrix cores, 32 blocks
+// to a workgroup.  Each block's share of its TB's remainder is its local one times
+// x^(bits after it) mod g, written per block and XORed by a wave per TB.
 #include <algorithm>
 #include <mutex>
 #include <vector>
@@ -384,8 +382,8 @@ int32_t LaunchCrcRagged(const RaggedCb *cbs, uint32_t num_cb, const int8_t *bits
     const int32_t st = EnsureTables(&t);
     if (st != AIRAN_OK) return st;
     if (num_cb == 0 || num_tbs == 0) return AIRAN_INVALID_ARGUMENT;
-    hipLaunchKernelGGL(RaggedCrcKernel, dim3(num_cb), dim3(kChunkThreads), 0, s, bits, cbs, t->pow_b, t->pow_a, t->pow_16,
-                       cb_ok, tb_part);
+    hipLaunchKernelGGL(RaggedCrcKernel, dim3(num_cb), dim3(kChunkThreads), 0, s, bits, cbs, t->pow_b, t->pow_a,
+                       t->pow_16, cb_ok, tb_part);
     hipLaunchKernelGGL(RaggedCrcFinishKernel, dim3(num_tbs), dim3(64), 0, s, tb_part, tb_first, tb_count, tb_ok);
     return LaunchStatus();
 }

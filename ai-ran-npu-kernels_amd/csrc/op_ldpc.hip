@@ -841,9 +841,10 @@ __device__ __forceinline__ uint32_t Int8Magnitude2(uint32_t v)
 // One row: edge(k, i4) places edge k, old(k) is its message (both checks),
 // put(k, x, e, m) takes the new one (e: 1 per half where the edge is at the
 // minimum); s1p and d12 return the kept messages' two magnitudes with the
-// row's parity in the sign bits, as s1p and s2p - s1p (mod 2^16 per half).  The addresses are computed anew for the second pass (three
-// instructions an edge, against two registers and a mask), and a long row is
-// taken kChunk edges at a time, both to stay within the registers.
+// row's parity in the sign bits, as s1p and s2p - s1p (mod 2^16 per half).  The
+// addresses are computed anew for the second pass (three instructions an edge,
+// against two registers and a mask), and a long row is taken kChunk edges at a
+// time, both to stay within the registers.
 template <int MODE, int DEG, typename Edge, typename Old, typename Put>
 __device__ __forceinline__ void CheckRow(uint32_t *lam, uint32_t i4, uint32_t *inf_flag, uint32_t &s1p, uint32_t &d12,
                                          Edge edge, Old old, Put put)
@@ -1244,7 +1245,8 @@ __global__ void __launch_bounds__(CheckThreads(ZT)) __attribute__((amdgpu_waves_
                 const uint2 a = *reinterpret_cast<const uint2 *>(s + col * Z + j);
                 const uint2 b = *reinterpret_cast<const uint2 *>(s + col * Z + zh + j);
                 auto word = [&](uint32_t x, uint32_t y, uint32_t sh) {
-                    return StartH<MODE>(static_cast<int16_t>(x >> sh)) | StartH<MODE>(static_cast<int16_t>(y >> sh)) << 16;
+                    return StartH<MODE>(static_cast<int16_t>(x >> sh)) |
+                           StartH<MODE>(static_cast<int16_t>(y >> sh)) << 16;
                 };
                 *reinterpret_cast<uint4 *>(lam + col * zh + j) =
                     make_uint4(word(a.x, b.x, 0), word(a.x, b.x, 16), word(a.y, b.y, 0), word(a.y, b.y, 16));
@@ -1460,7 +1462,8 @@ void LaunchCheckPair(const LdpcDecodeOpArgsV1 *a, hipStream_t s)
                                         : LdpcCheckPairKernel<MODE, kRows, kLowZ, kSrcLlr>);
     hipLaunchKernelGGL(k, dim3(a->num_cb), dim3(CheckThreads(zt)), 0, s, static_cast<const int16_t *>(a->lam_in),
                        static_cast<int8_t *>(a->bits), static_cast<int16_t *>(a->lam_out),
-                       static_cast<uint8_t *>(a->iterations_out), d, nullptr, nullptr, nullptr, nullptr, airan::RateDev{});
+                       static_cast<uint8_t *>(a->iterations_out), d, nullptr, nullptr, nullptr, nullptr,
+                       airan::RateDev{});
 }
 
 // The decoder operator (validated arguments).

@@ -144,7 +144,8 @@ __host__ __device__ inline void AxisPair(s16x2_t u, s16x2_t t, s16x2_t (&w)[QM /
         w[2] = (t2 + a) - (cl[2] + cl[2]);
     }
     if constexpr (M == 4) {
-        w[1] = (a * static_cast<short>(4) + (cl[1] + cl[2] + cl[3])) - (t2 * static_cast<short>(10) + (cl[5] + cl[6] + cl[7]));
+        w[1] = (a * static_cast<short>(4) + (cl[1] + cl[2] + cl[3])) -
+               (t2 * static_cast<short>(10) + (cl[5] + cl[6] + cl[7]));
         w[2] = (t2 * static_cast<short>(3) + (a + a) + cl[3] + cl[5]) - (cl[4] * static_cast<short>(4) + cl[1] + cl[7]);
         w[3] = (t2 + a) + (cl[4] - cl[2] - cl[6]) * static_cast<short>(2);
     }

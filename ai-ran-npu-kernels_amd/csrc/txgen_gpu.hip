@@ -185,7 +185,8 @@ __device__ inline uint32_t CrcTimes(uint32_t a, uint32_t b, uint32_t poly)
     uint32_t r = 0;
     b <<= 8;
 #pragma unroll 4
-    for (int i = 0; i < 24; ++i, b <<= 1) r = CrcTimesX(r, poly) ^ (a & static_cast<uint32_t>(static_cast<int32_t>(b) >> 31));
+    for (int i = 0; i < 24; ++i, b <<= 1)
+        r = CrcTimesX(r, poly) ^ (a & static_cast<uint32_t>(static_cast<int32_t>(b) >> 31));
     return r;
 }
 
@@ -383,13 +384,15 @@ __global__ void __launch_bounds__(kEncodeThreads) EncodeKernel(const uint8_t *__
             for (uint32_t j = 0; j < kCbChunkBits; j += 32u) {
                 const int32_t b = static_cast<int32_t>(p.per_cb + j) - static_cast<int32_t>(kCbChunkBits * (t + 1u));
                 uint32_t v = 0;
-                if (b > -32) v = b < 0 ? lin[0] << static_cast<uint32_t>(-b) : airan::BitsAt(lin, static_cast<uint32_t>(b));
+                if (b > -32)
+                    v = b < 0 ? lin[0] << static_cast<uint32_t>(-b) : airan::BitsAt(lin, static_cast<uint32_t>(b));
                 res = CrcWord(res, v, table);
             }
             const uint32_t pk = kCbChunkBits * t < p.per_cb ? a.pow_cb[t] : 0u;
             const uint32_t crc = WaveXor(CrcTimes(res, pk, kPolyB << 8));
             if (t == 0) {
-                const uint64_t v = static_cast<uint64_t>(__brev(crc)) << (p.per_cb & 31u);  // first bit the highest power
+                // The first bit is the highest power.
+                const uint64_t v = static_cast<uint64_t>(__brev(crc)) << (p.per_cb & 31u);
                 lin[p.per_cb >> 5] |= static_cast<uint32_t>(v);
                 lin[(p.per_cb >> 5) + 1] |= static_cast<uint32_t>(v >> 32);
             }
@@ -794,7 +797,10 @@ int32_t airan_pusch_txgpu_EncodeTbs(AiranPuschTxGpu *t, const uint8_t *payload, 
     ea.tb_part = t->tb_part;
     ea.pow_cb = t->pow_cb;
     ea.gold = t->gold;
-    const auto encode = g.qm == 2 ? EncodeKernel<2> : (g.qm == 4 ? EncodeKernel<4> : (g.qm == 6 ? EncodeKernel<6> : EncodeKernel<8>));
+    const auto encode = g.qm == 2   ? EncodeKernel<2>
+                        : g.qm == 4 ? EncodeKernel<4>
+                        : g.qm == 6 ? EncodeKernel<6>
+                                    : EncodeKernel<8>;
     hipLaunchKernelGGL(encode, dim3(ncb), dim3(kEncodeThreads), 0, s, payload, tp, ea, reinterpret_cast<float2 *>(grid),
                        coded_bits);
     DmrsArgs da{};
