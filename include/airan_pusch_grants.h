@@ -19,7 +19,8 @@
  *   LDPC (FP16 messages)    de-rate-matches while loading each code block;
  *                           one launch over the blocks of Z = 384 with more
  *                           than 10 active rows, one over those with fewer,
- *                           one over the other lifting sizes
+ *                           one over Z = 24, 48, 96 and 192, one over any
+ *                           other Z of 24 .. 384 (plans made by hand)
  *   CRC                     one launch over all code blocks + one per TB
  *
  * replayed from one HIP graph per batch.  Every stage computes what the
