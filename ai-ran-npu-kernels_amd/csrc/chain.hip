@@ -325,8 +325,6 @@ struct AiranPuschChain {
     int16_t *cw = nullptr;
     RateMatchDescriptor *desc = nullptr;
     int16_t *lam = nullptr;
-    uint8_t *ldpc_ws = nullptr;
-    size_t ldpc_ws_bytes = 0;
     int8_t *bits = nullptr;
     uint8_t *iters = nullptr, *cb_ok = nullptr, *tb_ok = nullptr;
     uint8_t *crc_ws = nullptr;
@@ -475,7 +473,7 @@ int32_t EnqueueStages(AiranPuschChain *c, const void *iq, const uint16_t *slot_n
     la.mode = c->opts.ldpc_mode;
     la.early_stop = c->opts.early_stop ? 1u : 0u;
     la.stream = s;
-    st = airan_ldpc_decode_Enqueue(&la, c->ldpc_ws, c->ldpc_ws_bytes);
+    st = airan::LaunchLdpc(la);
     if (st != AIRAN_OK) return st;
     mark();
     if ((st = EnqueueCrc(c, tbs, s)) != AIRAN_OK) return st;
@@ -554,8 +552,6 @@ int32_t airan_pusch_chain_Create(const PuschMimoConfig *config, const AiranTbPla
     const size_t gold_words = (static_cast<size_t>(T) * g.cw_symbols * g.qm + 31) / 32 + 2;
     const size_t dmrs_elems = S * g.nl * g.ndmrs * g.ref_pad;  // one DMRS reference per slot
     c->ce_ws_bytes = c->ls_zf ? 0 : airan::CeWorkspaceBytes(g, static_cast<uint32_t>(S));
-    c->ldpc_ws_bytes =
-        c->fused_ldpc ? 0 : airan_ldpc_decode_WorkspaceBytes(static_cast<uint32_t>(ncb), p.Z, c->active_rows);
     c->crc_ws_bytes = c->crc ? airan_crc_check_WorkspaceBytes(static_cast<uint32_t>(NT)) : 0;
     const size_t iq_elem = options->iq_format == AIRAN_IQ_COMPLEX64 ? 8 : 4;
     size_t &b = c->bytes;
@@ -568,7 +564,7 @@ int32_t airan_pusch_chain_Create(const PuschMimoConfig *config, const AiranTbPla
         !Alloc(&c->ce_ws, c->ce_ws_bytes, &b) || !Alloc(&c->h_re, S * g.nr * g.nl * plane, &b) ||
         !Alloc(&c->h_im, S * g.nr * g.nl * plane, &b) || !Alloc(&c->gold, gold_words, &b) ||
         !Alloc(&c->cw, S * g.qm * g.cw_stride, &b) || !Alloc(&c->desc, ncb, &b) ||
-        !Alloc(&c->lam, c->fused_ldpc ? 0 : ncb * 68 * p.Z, &b) || !Alloc(&c->ldpc_ws, c->ldpc_ws_bytes, &b) ||
+        !Alloc(&c->lam, c->fused_ldpc ? 0 : ncb * 68 * p.Z, &b) ||
         !Alloc(&c->bits, ncb * p.K, &b) || !Alloc(&c->iters, ncb, &b) || !Alloc(&c->cb_ok, ncb, &b) ||
         !Alloc(&c->tb_ok, NT, &b) || !Alloc(&c->refiner_keep, S, &b) || !Alloc(&c->crc_xpow, p.C, &b) ||
         !Alloc(&c->crc_ws, c->crc_ws_bytes, &b) ||
@@ -638,7 +634,7 @@ void airan_pusch_chain_Destroy(AiranPuschChain *c)
         if (e != nullptr) (void)hipEventDestroy(e);
     airan_channel_est_lmmse_DestroyFilter(c->filter);
     void *bufs[] = {c->dmrs_re, c->dmrs_im, c->slot_default, c->rx_re, c->rx_im, c->hls_re, c->hls_im, c->noise_ls, c->noise_ce,
-                    c->ce_ws, c->h_re, c->h_im, c->gold, c->cw, c->desc, c->lam, c->ldpc_ws, c->bits,
+                    c->ce_ws, c->h_re, c->h_im, c->gold, c->cw, c->desc, c->lam, c->bits,
                     c->iters, c->cb_ok, c->tb_ok, c->crc_ws, c->zero_iq, c->refiner_keep, c->crc_xpow,
                     c->ldpc_queue};
     for (void *p : bufs) Free(p);

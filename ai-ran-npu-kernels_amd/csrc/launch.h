@@ -128,6 +128,8 @@ int32_t LaunchDmrsRagged(const RaggedGrant *grants, const RaggedItem *gen_items,
                          __half *noise, hipStream_t s);
 // c_init of DMRS symbol `symbol` of cfg (mimo_dmrs_gen.cpp:38-45).
 uint32_t HostDmrsCinit(const PuschMimoConfig &cfg, uint32_t symbol);
+// airan_ldpc_decode_Enqueue without a workspace (the decoder reads none).
+int32_t LaunchLdpc(const LdpcDecodeOpArgsV1 &a);
 // LDPC (FP16 messages) of the listed code blocks, from the grants' codeword
 // LLRs (rate dematch in the decoder's load): Z = 384 with more than
 // LdpcFewRows() rows, with at most as many, blocks of the smaller sizes 24 <<

@@ -1570,6 +1570,12 @@ int32_t LaunchLdpcRagged(const RaggedCb *cbs, const RaggedGrant *grants, const R
     return LaunchStatus();
 }
 
+int32_t LaunchLdpc(const LdpcDecodeOpArgsV1 &a)
+{
+    const int32_t st = airan_ldpc_decode_ValidateOpArgs(&a);
+    return st == AIRAN_OK ? LaunchDecode(&a) : st;
+}
+
 uint32_t LdpcFewRows() { return kFewRows; }
 
 bool LdpcLiftSize(uint32_t z) { return IsLiftSize(z); }
