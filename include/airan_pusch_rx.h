@@ -35,8 +35,7 @@ extern "C" {
 
 /* ============================================================ device init */
 /* Loads the per-device constant tables (Gold jump-ahead matrices, FFT
- * twiddles, LDPC base graph) and takes the device address of the decoder's
- * no-alloc message array for the current device.  Called implicitly by the
+ * twiddles, LDPC base graph) of the current device.  Called implicitly by the
  * first Enqueue on a device; call it explicitly before capturing a stream
  * into a HIP graph. */
 int32_t airan_InitDevice(void);
@@ -723,6 +722,8 @@ typedef struct LdpcDecodeOpArgsV1 {
     void *stream;
 } LdpcDecodeOpArgsV1;
 int32_t airan_ldpc_decode_ValidateOpArgs(const LdpcDecodeOpArgsV1 *args);
+/* The workspace that Enqueue asks for (0 up to 8 active rows).  The decoder
+ * does not touch it: its message state is in registers. */
 size_t airan_ldpc_decode_WorkspaceBytes(uint32_t num_cb, uint32_t z, uint32_t active_rows);
 int32_t airan_ldpc_decode_Enqueue(const LdpcDecodeOpArgsV1 *args, void *workspace,
                                   size_t workspace_bytes);

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from oracle_lib import load_oracle, ptr
-from puschrx import ops
+from puschrx import abi, ops
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -53,4 +53,23 @@ def test_crc_of_every_block(gpu_stream, tbs, ntb, offset):
     cb_ok, tb_ok, _ = ops.crc_check(plan, ntb, buf[offset:])
     torch.cuda.synchronize()
     assert np.array_equal(cb_ok.cpu().numpy().reshape(ntb, plan.C), cb_want)
+    assert np.array_equal(tb_ok.cpu().numpy(), tb_want)
+
+
+@pytest.mark.parametrize("z,c,ntb", [(25, 1, 5), (45, 2, 4), (383, 3, 3), (52, 1, 3001)])
+def test_crc_of_odd_block_sizes(gpu_stream, z, c, ntb):
+    """K = 22 z that is no multiple of 16 (plans made by hand), also at a count
+    where blocks of another size would take the matrix product."""
+    kprime, crc_cb = 22 * z - 7, 24 if c > 1 else 0
+    plan = abi.AiranTbPlanV1(tbs=c * (kprime - crc_cb) - 16, crc_tb=16, crc_cb=crc_cb, C=c, K=22 * z, Kprime=kprime, Z=z)
+    rng = np.random.default_rng(z)
+    bits = np.repeat(_blocks(plan, rng)[None], ntb, axis=0)
+    cb_want, tb_want = np.ones((ntb, c), np.uint8), np.ones(ntb, np.uint8)
+    for t in range(0, ntb, 2):  # one checked payload bit of every other TB
+        r = int(rng.integers(c))
+        bits[t, r, int(rng.integers(kprime - crc_cb))] ^= 1
+        cb_want[t, r], tb_want[t] = 1 if c == 1 else 0, 0
+    cb_ok, tb_ok, _ = ops.crc_check(plan, ntb, torch.from_numpy(bits.reshape(-1)).cuda())
+    torch.cuda.synchronize()
+    assert np.array_equal(cb_ok.cpu().numpy().reshape(ntb, c), cb_want)
     assert np.array_equal(tb_ok.cpu().numpy(), tb_want)

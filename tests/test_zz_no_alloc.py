@@ -1,9 +1,8 @@
-"""airan_ldpc_decode_EnqueueNoAlloc (the decoder with its message state in
-the library's fixed device array, for callers that cannot allocate) against
+"""airan_ldpc_decode_EnqueueNoAlloc (for callers that cannot allocate) against
 airan_ldpc_decode_Enqueue with a caller workspace: identical bits, clamped
 posteriors and iteration counts on two calls in a row, the second with fewer
-code blocks (the array keeps the first call's state, which the decoder must
-not read); requests beyond the array are rejected before anything runs."""
+code blocks (nothing of the first call may show); requests whose workspace
+would exceed the stated limit are rejected before anything runs."""
 import ctypes as C
 
 import numpy as np
