@@ -769,10 +769,10 @@ int32_t LoadTables()
 // needed.  Their edge words (word index col Z + shift mod Z in bits 0 .. 15,
 // Z - shift mod Z above) are made by each workgroup, in LDS.
 // Half of every packed operation is idle and each edge word is an LDS read and a
-// readfirstlane: one
-// kernel for all of them, and not the fastest for any.  Ragged batches of one size, against the kernel with a compressed
-// state in memory that decoded them before: 600 blocks of Z = 383, 25 rows 1795
-// -> 1090 us, 2000 of Z = 36, 45 rows 4211 -> 3539, 200 of Z = 340 898 -> 438.
+// readfirstlane: one kernel for all of them, not the fastest for any.  Ragged
+// batches of one size, against the kernel with a compressed state in memory that
+// decoded them before: 600 blocks of Z = 383, 25 rows 1795 -> 1090 us, 2000 of
+// Z = 36, 45 rows 4211 -> 3539, 200 of Z = 340 898 -> 438.
 constexpr uint32_t kAnyZ = 1;  // as ZT
 constexpr uint32_t kMaxZ = 384;
 // As ZT: a size below 384 read from the arguments; one of at most 96, with the
